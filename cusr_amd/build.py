@@ -127,12 +127,13 @@ def build(jobs: int | None = None, verbose: bool = False, defines=(), out: Path 
     jobs = jobs or min(8, os.cpu_count() or 4)
     compiles = []
     for rtype, ad, name in FIT_VARIANTS:
-        obj = bdir / f"fit_launch_fit_{name}.o"
-        compiles.append([HIPCC, *flags, *extra, REMARKS, "-x", "hip",
-                         f"-DCUSR_FIT_R={rtype}",
-                         f"-DCUSR_FIT_AD={ad}", f"-DCUSR_FIT_LAUNCH=launch_fit_{name}",
-                         f"-DCUSR_PASS_LAUNCH=launch_pass_{name}", "-c",
-                         str(csrc / "fit_kernels.hip"), "-o", str(obj)])
+        for kind, part in [(k, p) for p in (2, 1, 0) for k in ("fit", "pass")]:
+            obj = bdir / f"fit_{kind}_{name}_{part}.o"
+            compiles.append([HIPCC, *flags, *extra, REMARKS, "-x", "hip",
+                             f"-DCUSR_FIT_R={rtype}", f"-DCUSR_FIT_AD={ad}",
+                             f"-DCUSR_PART={part}",
+                             f"-DCUSR_{kind.upper()}_LAUNCH=launch_{kind}_{name}_{part}", "-c",
+                             str(csrc / "fit_kernels.hip"), "-o", str(obj)])
     compiles.append([HIPCC, *flags, *extra, REMARKS, "-x", "hip", "-c",
                      str(csrc / "co_lib.hip"), "-o", str(bdir / "co_lib.o")])
     compiles.append([HIPCC, *flags, "-x", "hip", "-c", str(csrc / "program.cpp"),

@@ -139,6 +139,11 @@ struct Ctx {
     DevBuf prog, desc, X, Y, C0, C, status, li, lf, iters, stage;
     DevBuf data_X, data_Y;   // co_data_upload: X [D][N] column-major, y [N]
     DevBuf state;            // scratch of tail and split fits (run_fit)
+    // workspace of the V values (program.h) per launch range, and its columns
+    // in use: null where the range has none or they would not fit
+    DevBuf vwork[kMaxRanges];
+    void *v_ptr[kMaxRanges] = {};
+    size_t v_max = 0;        // bytes such a workspace may take: an eighth of the device's memory
     void *static_scratch = nullptr;   // this device's address of `scratch`
     HostBuf<uint64_t> h_prog;
     HostBuf<ExprDesc> h_desc;
@@ -180,6 +185,57 @@ int grow(DevBuf &b, size_t bytes) {
         if (r_ != CO_OK) return r_;           \
     } while (0)
 
+// The V workspaces given back (a fit then runs V in every pass); true if there
+// were any. hipFree waits for the device.
+bool drop_vwork(Ctx *ctx) {
+    bool any = false;
+    for (int r = 0; r < kMaxRanges; ++r) {
+        if (ctx->vwork[r].p) {
+            (void)hipFree(ctx->vwork[r].p);
+            any = true;
+        }
+        ctx->vwork[r] = DevBuf();
+        ctx->v_ptr[r] = nullptr;
+    }
+    return any;
+}
+
+// grow for what a fit needs: out of memory, it takes the place of the V
+// workspaces, which a fit can do without.
+int grow_needed(Ctx *ctx, DevBuf &b, size_t bytes) {
+    int rc = grow(b, bytes);
+    if (rc == CO_ERR_OOM && drop_vwork(ctx)) rc = grow(b, bytes);
+    return rc;
+}
+
+#define CO_GROW_NEEDED(ctx, buf, bytes)                \
+    do {                                               \
+        int r_ = grow_needed((ctx), (buf), (bytes));   \
+        if (r_ != CO_OK) return r_;                    \
+    } while (0)
+
+// The workspace of range r for `cols` columns of N values (fp64; fp32 fits use
+// half of it), grown with a quarter of headroom and kept. ctx->v_ptr[r] stays
+// null, and no error is returned, where it would pass v_max or does not fit.
+void set_vwork(Ctx *ctx, int r, int64_t cols, int N) {
+    DevBuf &b = ctx->vwork[r];
+    const size_t bytes = sizeof(double) * (size_t)cols * (size_t)N;
+    ctx->v_ptr[r] = nullptr;
+    if (bytes == 0 || bytes > ctx->v_max) return;
+    if (bytes > b.cap) {
+        if (b.p) (void)hipFree(b.p);
+        b = DevBuf();
+        const size_t want = bytes + bytes / 4;
+        if (hipMalloc(&b.p, want) != hipSuccess) {
+            (void)hipGetLastError();
+            b = DevBuf();
+            return;
+        }
+        b.cap = want;
+    }
+    ctx->v_ptr[r] = b.p;
+}
+
 template <typename T>
 int grow_host(HostBuf<T> &b, size_t n) {
     if (n == 0) n = 1;
@@ -211,23 +267,23 @@ T *ptr(DevBuf &b) { return (T *)b.p; }
 
 unsigned blocks_for(size_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
 
-// dynamic LDS a workgroup of a fit kernel family may use: the device's LDS
-// per workgroup less the family's static arrays (constants and pass sums)
-size_t max_dyn_lds(const Ctx *ctx, bool gen) {
-    const size_t st = fit_static_lds(gen);
+// dynamic LDS a workgroup of a bin's fit kernel may use: the device's LDS per
+// workgroup less the kernel's static arrays (constants and pass sums)
+size_t max_dyn_lds(const Ctx *ctx, int bin) {
+    const size_t st = fit_static_lds(bin);
     return ctx->lds_per_block > st ? ctx->lds_per_block - st : 0;
 }
 
 // the launcher's choice of instance (fit_kernels.hip): the large-N one from
 // kLargeN points where its tables differ
 template <typename R, int AD>
-size_t lds_for_k(int K, int N, int D, int slots, int tape) {
+size_t lds_for_k(int K, int N, int rows, int tape) {
     switch (K) {
 #define CUSR_LDS_CASE(k)                                                        \
     case k:                                                                     \
         return (large_n_variant<R, k, AD>() && N >= kLargeN)                    \
-                   ? fit_lds_bytes_t<R, k, AD, 1>(D, slots, tape)               \
-                   : fit_lds_bytes_t<R, k, AD, 0>(D, slots, tape);
+                   ? fit_lds_bytes_t<R, k, AD, 1>(rows, tape)                   \
+                   : fit_lds_bytes_t<R, k, AD, 0>(rows, tape);
     CUSR_LDS_CASE(0) CUSR_LDS_CASE(1) CUSR_LDS_CASE(2) CUSR_LDS_CASE(3) CUSR_LDS_CASE(4)
     CUSR_LDS_CASE(5) CUSR_LDS_CASE(6) CUSR_LDS_CASE(7) CUSR_LDS_CASE(8) CUSR_LDS_CASE(9)
     CUSR_LDS_CASE(10) CUSR_LDS_CASE(11) CUSR_LDS_CASE(12) CUSR_LDS_CASE(13)
@@ -237,15 +293,15 @@ size_t lds_for_k(int K, int N, int D, int slots, int tape) {
     }
 }
 
-size_t fit_lds_bytes(bool mixed, bool rev, int K, int N, int D, int slots, int tape) {
+size_t fit_lds_bytes(bool mixed, bool rev, int K, int N, int rows, int tape) {
     if (K == CO_GENERAL_BIN)
-        return mixed ? fit_lds_bytes_gen<float>(D, slots, tape)
-                     : fit_lds_bytes_gen<double>(D, slots, tape);
+        return mixed ? fit_lds_bytes_gen<float>(rows, tape)
+                     : fit_lds_bytes_gen<double>(rows, tape);
     if (mixed)
-        return rev ? lds_for_k<float, CO_AD_REVERSE>(K, N, D, slots, tape)
-                   : lds_for_k<float, CO_AD_FORWARD>(K, N, D, slots, tape);
-    return rev ? lds_for_k<double, CO_AD_REVERSE>(K, N, D, slots, tape)
-               : lds_for_k<double, CO_AD_FORWARD>(K, N, D, slots, tape);
+        return rev ? lds_for_k<float, CO_AD_REVERSE>(K, N, rows, tape)
+                   : lds_for_k<float, CO_AD_FORWARD>(K, N, rows, tape);
+    return rev ? lds_for_k<double, CO_AD_REVERSE>(K, N, rows, tape)
+               : lds_for_k<double, CO_AD_FORWARD>(K, N, rows, tape);
 }
 
 // Device buffers of a population of M expressions with `words` program words.
@@ -260,21 +316,21 @@ int grow_buffers(Ctx *ctx, const PopHeader *h, size_t words, bool in32, bool on_
     // round's) does not free and allocate again (about 1 ms of a C5 round
     // when it did)
     if (sizeof(uint64_t) * words > ctx->prog.cap)
-        CO_GROW(ctx->prog, sizeof(uint64_t) * (words + words / 4));
-    CO_GROW(ctx->desc, sizeof(ExprDesc) * M);
-    CO_GROW(ctx->X, sizeof(double) * nX);
-    CO_GROW(ctx->Y, sizeof(double) * nY);
+        CO_GROW_NEEDED(ctx, ctx->prog, sizeof(uint64_t) * (words + words / 4));
+    CO_GROW_NEEDED(ctx, ctx->desc, sizeof(ExprDesc) * M);
+    CO_GROW_NEEDED(ctx, ctx->X, sizeof(double) * nX);
+    CO_GROW_NEEDED(ctx, ctx->Y, sizeof(double) * nY);
     const size_t Ch = (size_t)C + (size_t)C / 4;
-    if (sizeof(double) * C > ctx->C0.cap) CO_GROW(ctx->C0, sizeof(double) * Ch);
-    if (sizeof(double) * C > ctx->C.cap) CO_GROW(ctx->C, sizeof(double) * Ch);
-    CO_GROW(ctx->status, sizeof(int32_t) * M);
-    CO_GROW(ctx->li, sizeof(double) * M);
-    CO_GROW(ctx->lf, sizeof(double) * M);
-    CO_GROW(ctx->iters, sizeof(int32_t) * M);
+    if (sizeof(double) * C > ctx->C0.cap) CO_GROW_NEEDED(ctx, ctx->C0, sizeof(double) * Ch);
+    if (sizeof(double) * C > ctx->C.cap) CO_GROW_NEEDED(ctx, ctx->C, sizeof(double) * Ch);
+    CO_GROW_NEEDED(ctx, ctx->status, sizeof(int32_t) * M);
+    CO_GROW_NEEDED(ctx, ctx->li, sizeof(double) * M);
+    CO_GROW_NEEDED(ctx, ctx->lf, sizeof(double) * M);
+    CO_GROW_NEEDED(ctx, ctx->iters, sizeof(int32_t) * M);
     size_t stage = esz * nX;
     if (in32 && esz * nY > stage) stage = esz * nY;
     if (in32 && esz * C > stage) stage = esz * C;
-    if (stage > ctx->stage.cap) CO_GROW(ctx->stage, stage + stage / 4);
+    if (stage > ctx->stage.cap) CO_GROW_NEEDED(ctx, ctx->stage, stage + stage / 4);
     return CO_OK;
 }
 
@@ -349,11 +405,12 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
     CO_HIP(hipSetDevice(ctx->device));
     ctx->resident = false;
     const int M = h->M_prob;
-    CO_GROW_HOST(ctx->h_prog, h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1);
+    CO_GROW_HOST(ctx->h_prog, staged_words_max(h->total_nodes, h->n_vars));
     CO_GROW_HOST(ctx->h_desc, M > 0 ? (size_t)M : 1);
-    int rc = decode_population(h, nt, nv, ci, metas, ctx->h_prog.data(), nullptr, nullptr,
-                               ctx->h_desc.data(), nullptr, nullptr, nullptr, nullptr,
-                               &ctx->plan);
+    int rc = check_header(h, nt, nv, ci, metas);
+    if (rc == CO_OK)
+        rc = decode_range(h, nt, nv, ci, metas, 0, M, 0, ctx->h_prog.data(), ctx->h_desc.data(),
+                          &ctx->plan);
     if (rc != CO_OK) return rc;
     if (on_data && (ctx->data_N < 0 || h->N != ctx->data_N || h->n_vars != ctx->data_D))
         return CO_ERR_DATA;
@@ -367,6 +424,7 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
     const size_t words = (size_t)ctx->plan.words;
     rc = grow_buffers(ctx, h, words, in32, on_data, shared_y);
     if (rc != CO_OK) return rc;
+    set_vwork(ctx, 0, ctx->plan.vcols, h->N);
     hipStream_t s = ctx->stream;
     if (words)
         CO_HIP(hipMemcpyAsync(ctx->prog.p, ctx->h_prog.data(), sizeof(uint64_t) * words,
@@ -384,13 +442,14 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
 // One launch of a fit: its bin, workgroups, LDS and stream (planned before
 // anything is launched, so a launch that cannot fit is refused up front).
 struct LaunchPlan {
-    int bin, pos, cnt, slots, tape, kmax, stream;
+    int bin, pos, cnt, rows, tape, uni, kmax, stream;   // uni: doubles of the scalar area
     size_t wave_bytes;
     int pwaves[2];
     size_t lds[2];
 };
 
-typedef hipError_t (*Launcher)(int, unsigned, size_t, hipStream_t, const FitArgs &);
+// Bytes of a launch's per-wavefront scalar area.
+int uni_bytes(const LaunchPlan &b) { return (b.uni * (int)sizeof(double) + 15) & ~15; }
 
 // The launches of one fit, planned and issued range by range. The
 // descriptors of a range are in launch order (decode_population /
@@ -439,7 +498,7 @@ struct FitRun {
     Segment seg[2] = {};
     bool lane_used[kExtraStreams] = {};
     int range = 0;   // ranges issued so far
-    Launcher launch = nullptr, launch_pass = nullptr;
+    const Launcher *launch = nullptr, *launch_pass = nullptr;   // by part_of_bin
 
     // Option checks and the fit's arguments (ctx->plan holds N, D, M, C).
     int begin(Ctx *c, const CoOptions &o) {
@@ -477,7 +536,6 @@ struct FitRun {
         fa.loss_final = ptr<double>(ctx->lf);
         fa.iters = ptr<int32_t>(ctx->iters);
         fa.N = plan.N;
-        fa.D = plan.D;
         fa.max_iter = opt.max_iter;
         fa.guard = opt.fp64_guard ? 1 : 0;
         fa.shared_y = ctx->shared_y ? 1 : 0;
@@ -536,7 +594,10 @@ struct FitRun {
             while (pos < p1 && (gen ? ctx->h_desc[pos].gen != 0
                                     : (!ctx->h_desc[pos].gen && ctx->h_desc[pos].K == bin))) {
                 const ExprDesc &d = ctx->h_desc[pos];
-                if (d.slots > b.slots) b.slots = d.slots;
+                const int rows = rev ? d.rows_rev : d.rows;
+                const int uni = d.n_c ? uni_doubles(d.K, d.cslots, rev ? d.ctape : 0) : 0;
+                if (rows > b.rows) b.rows = rows;
+                if (uni > b.uni) b.uni = uni;
                 if (d.tape > b.tape) b.tape = d.tape;
                 if (d.K > b.kmax) b.kmax = d.K;
                 ++b.cnt;
@@ -551,10 +612,9 @@ struct FitRun {
             // workgroup (each summing several partitions) when LDS is short. The
             // split path's pass workgroups are one wavefront with no partition
             // sums in LDS.
-            b.wave_bytes =
-                (fit_lds_bytes(mixed, rev, bin, plan.N, plan.D, b.slots, b.tape) + 15) &
-                ~(size_t)15;
-            const size_t cap = max_dyn_lds(ctx, gen);
+            b.wave_bytes = uni_bytes(b) + ((fit_lds_bytes(mixed, rev, bin, plan.N, b.rows, b.tape) +
+                                            15) & ~(size_t)15);
+            const size_t cap = max_dyn_lds(ctx, bin);
             const int ks = gen ? b.kmax : bin;
             for (int g = 0; g < (b.kmax == 0 || split ? 1 : nseg); ++g) {
                 const int sp = split ? 1 : seg[g].parts;
@@ -588,7 +648,8 @@ struct FitRun {
         const size_t psum_bytes = split ? sizeof(double) * (size_t)parts * pwidth * M : 0;
         Scratch own;
         if (!sc) {
-            if (state_bytes + psum_bytes) CO_GROW(ctx->state, state_bytes + psum_bytes);
+            if (state_bytes + psum_bytes)
+                CO_GROW_NEEDED(ctx, ctx->state, state_bytes + psum_bytes);
             own.p = ctx->state.p;
             own.cap = ctx->state.cap;
             sc = &own;
@@ -656,15 +717,17 @@ struct FitRun {
                 FitArgs fk = fa;
                 fk.desc = fa.desc + b.pos;
                 fk.psum = fa.psum + (size_t)b.pos * parts * pwidth;
-                fk.slots = b.slots;
+                fk.rows = b.rows;
                 fk.tape = b.tape;
+                fk.uni_bytes = uni_bytes(b);
+                fk.V = ctx->v_ptr[range];
                 fk.parts = parts;
                 fk.pwaves = 1;
                 fk.wave_bytes = (int)b.wave_bytes;
                 fk.it_end = opt.max_iter;
                 fk.resume = 0;
                 for (int r = 0; r < rounds; ++r) {
-                    CO_LAUNCH_HIP(launch_pass(b.bin, (unsigned)b.cnt * parts, b.lds[0], ks, fk));
+                    CO_LAUNCH_HIP(launch_pass[part_of_bin(b.bin)](b.bin, (unsigned)b.cnt * parts, b.lds[0], ks, fk));
                     launch_step(b.bin, (unsigned)b.cnt, ks, fk, mixed ? 1 : 0);
                     CO_LAUNCH_HIP(hipGetLastError());
                 }
@@ -673,14 +736,16 @@ struct FitRun {
                 for (int g = 0; g < (b.kmax == 0 ? 1 : nseg); ++g) {
                     FitArgs fk = fa;
                     fk.desc = fa.desc + b.pos;
-                    fk.slots = b.slots;
+                    fk.rows = b.rows;
                     fk.tape = b.tape;
+                    fk.uni_bytes = uni_bytes(b);
+                    fk.V = ctx->v_ptr[range];
                     fk.parts = seg[g].parts;
                     fk.pwaves = b.pwaves[g];
                     fk.wave_bytes = (int)b.wave_bytes;
                     fk.it_end = seg[g].it_end;
                     fk.resume = seg[g].resume;
-                    CO_LAUNCH_HIP(launch(b.bin, (unsigned)b.cnt, b.lds[g], ks, fk));
+                    CO_LAUNCH_HIP(launch[part_of_bin(b.bin)](b.bin, (unsigned)b.cnt, b.lds[g], ks, fk));
                 }
             }
             CO_LAUNCH_HIP(hipEventRecord(ctx->ev_b1[range][b.bin], ks));
@@ -838,9 +903,9 @@ int fit_pipelined(Ctx *ctx, const CoOptions &opt, const PopHeader *h, const int3
         return CO_ERR_DATA;
     const int M = h->M_prob;
     const bool shared_y = on_data || (pop_flags(h) & POP_FLAG_SHARED_Y) != 0;
-    CO_GROW_HOST(ctx->h_prog, h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1);
+    CO_GROW_HOST(ctx->h_prog, staged_words_max(h->total_nodes, h->n_vars));
     CO_GROW_HOST(ctx->h_desc, (size_t)M);
-    rc = grow_buffers(ctx, h, h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1, in32, on_data,
+    rc = grow_buffers(ctx, h, staged_words_max(h->total_nodes, h->n_vars), in32, on_data,
                       shared_y);
     if (rc != CO_OK) return rc;
     ctx->on_data = on_data;
@@ -881,6 +946,7 @@ int fit_pipelined(Ctx *ctx, const CoOptions &opt, const PopHeader *h, const int3
 #endif
         rc = decode_range(h, nt, nv, ci, metas, m0, m1, wb, ctx->h_prog.data(),
                           ctx->h_desc.data(), &rp);
+        if (rc == CO_OK) set_vwork(ctx, j, rp.vcols, h->N);
 #ifdef CUSR_EXP_TIMING
         const double q1 = now_ms();
 #endif
@@ -923,9 +989,7 @@ int fit_pipelined(Ctx *ctx, const CoOptions &opt, const PopHeader *h, const int3
         if (j == 0) *setup_ms = now_ms() - t0;
         wb += rp.words;
         pl.n_gen += rp.n_gen;
-        if (rp.max_tape > pl.max_tape) pl.max_tape = rp.max_tape;
-        if (rp.max_n > pl.max_n) pl.max_n = rp.max_n;
-        if (rp.max_slots > pl.max_slots) pl.max_slots = rp.max_slots;
+        pl.vcols += rp.vcols;
         ctx->ranges.push_back(m1);
     }
     pl.words = wb;
@@ -1015,6 +1079,9 @@ extern "C" int co_init(int device_id, void **handle_out) {
                                          device_id);
     if (e == hipSuccess)
         ctx->lds_per_block = lds_per_block > 0 ? (size_t)lds_per_block : 0;
+    size_t mem_free = 0, mem_total = 0;
+    if (e == hipSuccess) e = hipMemGetInfo(&mem_free, &mem_total);
+    ctx->v_max = mem_total / 8;
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     for (int i = 0; i < kExtraStreams && e == hipSuccess; ++i)
         e = hipStreamCreateWithFlags(&ctx->lanes[i], hipStreamNonBlocking);
@@ -1264,16 +1331,19 @@ extern "C" int co_eval_ex(void *handle, const PopHeader *h, const int32_t *nt, c
     CO_HIP(hipSetDevice(ctx->device));
     ctx->resident = false;  // the evaluation reuses the population buffers
     const int M = h->M_prob;
-    CO_GROW_HOST(ctx->h_prog, h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1);
+    CO_GROW_HOST(ctx->h_prog, staged_words_max(h->total_nodes, h->n_vars));
     CO_GROW_HOST(ctx->h_desc, M > 0 ? (size_t)M : 1);
     Plan plan = {};
-    int rc = decode_population(h, nt, nv, ci, metas, ctx->h_prog.data(), nullptr, nullptr,
-                               ctx->h_desc.data(), nullptr, nullptr, nullptr, nullptr, &plan);
+    int rc = check_header(h, nt, nv, ci, metas);
+    if (rc == CO_OK)
+        rc = decode_range(h, nt, nv, ci, metas, 0, M, 0, ctx->h_prog.data(), ctx->h_desc.data(),
+                          &plan);
     if (rc != CO_OK || M == 0) return rc;
     const int N = h->N, D = h->n_vars, C = h->total_c;
     const size_t nX = (size_t)N * D, nY = (size_t)M * N, words = (size_t)plan.words;
-    // one workgroup per expression: inputs and spill slots of 64 points in LDS
-    const size_t lds = (size_t)(D + plan.max_slots) * kLanes * (precision == CO_PREC_FP64 ? 8 : 4);
+    // one workgroup per expression: C's scalars, then the rows of 64 points in LDS
+    const int uni = (uni_doubles(h->K_max > 0 ? CO_MAX_K : 0, plan.max_cslots, 0) * (int)sizeof(double) + 15) & ~15;
+    const size_t lds = uni + (size_t)plan.max_rows * kLanes * (precision == CO_PREC_FP64 ? 8 : 4);
     if (lds + sizeof(double) * CO_MAX_K > ctx->lds_per_block) return CO_ERR_BOUNDS;
     CO_GROW(ctx->prog, sizeof(uint64_t) * words);
     CO_GROW(ctx->desc, sizeof(ExprDesc) * M);
@@ -1300,7 +1370,7 @@ extern "C" int co_eval_ex(void *handle, const PopHeader *h, const int32_t *nt, c
     ea.C = ptr<double>(ctx->C0);
     ea.Yout = ptr<double>(ctx->Y);
     ea.N = N;
-    ea.D = D;
+    ea.uni_bytes = uni;
     // descriptors in launch order: the wide programs first, then the fast ones
     const int ng = plan.n_gen, nf = M - plan.n_gen;
     ea.desc = ptr<ExprDesc>(ctx->desc);
@@ -1335,8 +1405,8 @@ extern "C" int co_decode(const PopHeader *h, const int32_t *nt, const float *nv,
         tmp.resize(h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1);
         prog = tmp.data();
     }
-    return decode_population(h, nt, nv, ci, metas, prog, order_out, bin_start_out, nullptr,
-                             stack_out, nullptr, program_off_out, route_out, nullptr);
+    return decode_population(h, nt, nv, ci, metas, prog, order_out, bin_start_out, stack_out,
+                             program_off_out, route_out);
 }
 
 extern "C" int co_upload_ex(void *handle, const PopHeader *h, const int32_t *nt,
@@ -1404,6 +1474,7 @@ extern "C" void co_teardown(void *handle) {
                       &ctx->data_X, &ctx->data_Y, &ctx->state};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
+    drop_vwork(ctx);
     if (ctx->h_prog.p) (void)hipHostFree(ctx->h_prog.p);
     if (ctx->h_desc.p) (void)hipHostFree(ctx->h_desc.p);
     if (ctx->h_stage.p) (void)hipHostFree(ctx->h_stage.p);

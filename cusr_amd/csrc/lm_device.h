@@ -136,6 +136,12 @@ struct FastFmt {
     static __device__ __forceinline__ int scale_b(W w) { return (int)((w.h >> 17) & 1u); }
     static __device__ __forceinline__ int tape_a(W w) { return (int)((w.h >> 18) & 1u); }
     static __device__ __forceinline__ int tape_b(W w) { return (int)((w.h >> 19) & 1u); }
+    static __device__ __forceinline__ int root(W w) { return (int)((w.h >> 20) & 1u); }
+    static __device__ __forceinline__ int cidx(W w) { return (int)((w.h >> 21) & 255u); }
+    // variable of variable row r
+    static __device__ __forceinline__ int var(ProgPtr, uint64_t map, int r) {
+        return (int)((map >> (4 * r)) & 15u);
+    }
 };
 struct WideFmt {
     typedef Wide W;
@@ -146,23 +152,28 @@ struct WideFmt {
         w.b = p[2 * pc + 1];
         return w;
     }
-    static __device__ __forceinline__ int fid(W w) { return wins_fid(w.a); }
-    static __device__ __forceinline__ int binary(W w) { return wins_binary(w.a); }
-    static __device__ __forceinline__ int akind(W w) { return wins_akind(w.a); }
-    static __device__ __forceinline__ int aidx(W w) { return wins_aidx(w.a); }
-    static __device__ __forceinline__ int bkind(W w) { return wins_bkind(w.a); }
-    static __device__ __forceinline__ int bidx(W w) { return wins_bidx(w.a); }
-    static __device__ __forceinline__ int toslot(W w) { return wins_toslot(w.a); }
-    static __device__ __forceinline__ int didx(W w) { return wins_didx(w.a); }
-    static __device__ __forceinline__ int lo(W w) { return wins_lo(w.b); }
-    static __device__ __forceinline__ int mid(W w) { return wins_mid(w.b); }
-    static __device__ __forceinline__ int hi(W w) { return wins_hi(w.b); }
-    static __device__ __forceinline__ int tape(W w) { return wins_tape(w.b); }
-    static __device__ __forceinline__ int sel(W w) { return wins_sel(w.a); }
-    static __device__ __forceinline__ int scale_a(W w) { return wins_scale_a(w.a); }
-    static __device__ __forceinline__ int scale_b(W w) { return wins_scale_b(w.a); }
-    static __device__ __forceinline__ int tape_a(W w) { return wins_tape_a(w.a); }
-    static __device__ __forceinline__ int tape_b(W w) { return wins_tape_b(w.a); }
+    static __device__ __forceinline__ int fid(W w) { return wst_fid(w.a); }
+    static __device__ __forceinline__ int binary(W w) { return wst_bit(w.a, 6); }
+    static __device__ __forceinline__ int akind(W w) { return wst_akind(w.a); }
+    static __device__ __forceinline__ int aidx(W w) { return wst_aidx(w.a); }
+    static __device__ __forceinline__ int bkind(W w) { return wst_bkind(w.a); }
+    static __device__ __forceinline__ int bidx(W w) { return wst_bidx(w.a); }
+    static __device__ __forceinline__ int toslot(W w) { return wst_bit(w.a, 26); }
+    static __device__ __forceinline__ int didx(W w) { return wst_didx(w.b); }
+    static __device__ __forceinline__ int lo(W w) { return wst_lo(w.b); }
+    static __device__ __forceinline__ int mid(W w) { return wst_mid(w.b); }
+    static __device__ __forceinline__ int hi(W w) { return wst_hi(w.b); }
+    static __device__ __forceinline__ int tape(W w) { return wst_tape(w.b); }
+    static __device__ __forceinline__ int sel(W w) { return wst_bit(w.a, 21); }
+    static __device__ __forceinline__ int scale_a(W w) { return wst_bit(w.a, 22); }
+    static __device__ __forceinline__ int scale_b(W w) { return wst_bit(w.a, 23); }
+    static __device__ __forceinline__ int tape_a(W w) { return wst_bit(w.a, 24); }
+    static __device__ __forceinline__ int tape_b(W w) { return wst_bit(w.a, 25); }
+    static __device__ __forceinline__ int root(W w) { return wst_bit(w.a, 27); }
+    static __device__ __forceinline__ int cidx(W w) { return wst_cidx(w.a); }
+    static __device__ __forceinline__ int var(ProgPtr rows, uint64_t, int r) {
+        return (int)rows[r];
+    }
 };
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -171,6 +182,19 @@ __device__ __forceinline__ double uni(double v) {
     p.x = __builtin_amdgcn_readfirstlane(p.x);
     p.y = __builtin_amdgcn_readfirstlane(p.y);
     return *reinterpret_cast<double *>(&p);
+}
+
+// LDS order within one wavefront: its LDS accesses are performed in the order
+// they are issued, so only the compiler has to keep it; no wait.
+__device__ __forceinline__ void wave_order_lds() {
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
 // ------------------------------------------------------------------ math
@@ -447,8 +471,8 @@ __device__ __forceinline__ R safe_mul(R a, R b) {
 // Per-wavefront LDS areas; every array is [index][p][lane].
 template <typename R, int P>
 struct WaveLds {
-    R *x;      // [D][P][64] the batch's inputs
-    R *slot;   // [slots][P][64] spilled right operands (adjoints in the reverse sweep)
+    R *x;      // [rows][P][64] the batch's inputs, V values and slots (adjoints in
+               // the reverse sweep)
     R *tape;   // [tape][P][64] reverse-AD partials
 };
 
@@ -708,25 +732,24 @@ __device__ __forceinline__ void add_tangent(R *T, int k, const R *v) {
 template <typename R, int P>
 __device__ __forceinline__ void fetch(int kind, int idx, const R *acc, const WaveLds<R, P> &w,
                                       const double *cs, int lane, R *out) {
-    // the running value first (one test), then bit 0 of the kind: a variable
-    // or a spilled value, one per-lane LDS read from the row's base chosen
-    // by bit 1 without a branch; else a constant. Bit tests, unlike equality
-    // tests, are not merged into a balanced compare tree.
+    // the running value first (one test), then bit 0 of the kind: a row of the
+    // wavefront (variable, V value or slot), one per-lane LDS read; else a
+    // constant. Bit tests, unlike equality tests, are not merged into a
+    // balanced compare tree.
     if (kind == OPD_ACC) {
         CUSR_FOR_P out[p] = acc[p];
     } else if (kind & 1) {
-        R *base = (kind & 2) ? w.slot : w.x;
-        CUSR_FOR_P out[p] = lds_at<R, P>(base, idx, p, lane);
+        CUSR_FOR_P out[p] = lds_at<R, P>(w.x, idx, p, lane);
     } else {
         const R c = (R)cs[idx];
         CUSR_FOR_P out[p] = c;
     }
 }
 
-// Forward sweep of one program over P points whose inputs are in w.x.
-// JAC: 0 value only, 1 forward AD into T[p*K + j] (which must hold 1.0 on
-// entry: the tangent of constant k with respect to itself), 2 partials to the
-// tape.
+// Forward sweep of one program over P points whose inputs are in w.x. cs: the
+// constants, C values in place. JAC: 0 value only, 1 forward AD into T[p*K + j]
+// (which must hold the tangent of M's operand with respect to constant j on
+// entry: 1.0, or what C left), 2 partials to the tape.
 template <int K, typename R, int P, int JAC, typename F = FastFmt>
 __device__ __forceinline__ void forward_pass(ProgPtr prog, int n, const WaveLds<R, P> &w,
                                              const double *cs, int lane, R *acc, R *T) {
@@ -784,17 +807,149 @@ __device__ __forceinline__ void forward_pass(ProgPtr prog, int n, const WaveLds<
         const bool spill = F::toslot(ins);
         if (spill) {
             const int di = F::didx(ins);
-            CUSR_FOR_P lds_at<R, P>(w.slot, di, p, lane) = o[p];
+            CUSR_FOR_P lds_at<R, P>(w.x, di, p, lane) = o[p];
         }
         CUSR_FOR_P acc[p] = o[p];
     }
 }
 
+// LDS of one wavefront for the scalar program C (program.h, uni_doubles).
+struct UniLds {
+    double *cm;      // [K] the constants, then C's values in place
+    double *t0;      // [K] forward AD: the tangents M starts from
+    double *slot;    // C's spill slots
+    double *tape;    // reverse AD: C's partials
+};
+__device__ __forceinline__ UniLds uni_lds(double *base, int K, int cslots) {
+    UniLds u;
+    u.cm = base;
+    u.t0 = base + K;
+    u.slot = base + 2 * K;
+    u.tape = u.slot + cslots;
+    return u;
+}
+
+// The scalar program C at constants cs: every lane computes the same single
+// value per operator (one point per lane whatever P the passes take). The
+// interpreter's steps, with C's own LDS in place of rows. Bound by the step's
+// dependent chain (1,300 cycles on the benchmark operators at K = 8); it replaces
+// the operators' steps in every batch of the pass.
+template <int K, typename R, int JAC, typename F>
+__device__ __forceinline__ void const_phase(ProgPtr prog, int n, const UniLds &u, const double *cs,
+                                            int lane, int Kr) {
+    R T[K > 0 ? K : 1];
+#pragma unroll
+    for (int j = 0; j < K; ++j) T[j] = R(1);
+    if (lane < Kr) u.cm[lane] = cs[lane];
+    wave_order_lds();
+    R acc[1];
+    const ProgPtr end = prog + F::kWords * n;
+    for (ProgPtr q = prog; q != end; q += F::kWords) {
+        const typename F::W ins = F::load(q, 0);
+        const int fid = F::fid(ins);
+        R a[1], b[1], o[1], d1[1], d2[1];
+        uint64_t z1[1], z2[1];
+        const auto get = [&](int kind, int idx, R *out) {
+            if (kind == OPD_ACC) {
+                out[0] = acc[0];
+            } else {
+                const double *base = (kind & 1) ? u.slot : cs;
+                out[0] = (R)base[idx];
+            }
+        };
+        if (F::binary(ins)) {
+            get(F::bkind(ins), F::bidx(ins), b);
+            get(F::akind(ins), F::aidx(ins), a);
+            binary_p<R, 1, JAC != 1>(fid, a, b, JAC == 2 || (JAC == 1 && F::scale_b(ins)), o, d1,
+                                     d2, z1, z2);
+            if constexpr (JAC == 2) {
+                const int t = F::tape(ins), ta = F::tape_a(ins);
+                if (ta && lane == 0) u.tape[t] = (double)d1[0];
+                if (F::tape_b(ins) && lane == 0) u.tape[t + ta] = (double)d2[0];
+            }
+        } else {
+            get(F::akind(ins), F::aidx(ins), a);
+            unary_p<R, 1, 1>(fid, a, o, d1, z1);
+            if constexpr (JAC == 2) {
+                if (F::tape_a(ins) && lane == 0) u.tape[F::tape(ins)] = (double)d1[0];
+            }
+        }
+        if constexpr (JAC == 1) {
+            if (F::scale_a(ins))
+                scale_range<K, R, 1>(T, F::lo(ins), F::mid(ins), d1, z1, F::sel(ins));
+            if (F::scale_b(ins))
+                scale_range<K, R, 1>(T, F::mid(ins), F::hi(ins), d2, z2, F::sel(ins));
+        }
+        // a subtree's last value takes the place of its first constant; cs
+        // itself keeps the constants (the other subtrees' operands)
+        const bool spill = F::toslot(ins), root = F::root(ins);
+        if (spill || root) {
+            double *dst = root ? u.cm + F::lo(ins) : u.slot + F::didx(ins);
+            if (lane == 0) *dst = (double)o[0];
+            wave_order_lds();
+        }
+        acc[0] = o[0];
+    }
+    if constexpr (JAC == 1) {
+        // all lanes hold the same row: entry j from lane j, in one store
+        double t = 0.0;
+#pragma unroll
+        for (int j = 0; j < K; ++j) t = lane == j ? (double)T[j] : t;
+        if (lane < K) u.t0[lane] = t;
+    }
+    wave_order_lds();
+}
+
+// Reverse sweep of the C subtree whose root is instruction `at` of C, the
+// adjoints of its root in accadj: C's partials are one value per wavefront, the
+// adjoints one per point. Adjoint slots: rows crow, crow + 1, ...
+template <int K, typename R, int P, typename F>
+__device__ __forceinline__ void reverse_const(ProgPtr progc, int at, const WaveLds<R, P> &w,
+                                              const double *tape, int crow, int lane, R *accadj,
+                                              R *T) {
+    const int first = at - F::cidx(F::load(progc, at)) + 1;
+    for (int pc = at; pc >= first; --pc) {
+        const typename F::W ins = F::load(progc, pc);
+        R adj[P];
+        if (F::toslot(ins)) {
+            const int di = crow + F::didx(ins);
+            CUSR_FOR_P adj[p] = lds_at<R, P>(w.x, di, p, lane);
+        } else {
+            CUSR_FOR_P adj[p] = accadj[p];
+        }
+        const int t = F::tape(ins), ta = F::tape_a(ins);
+        const int nop = F::binary(ins) ? 2 : 1;
+        for (int side = 0; side < nop; ++side) {
+            const int kind = side ? F::bkind(ins) : F::akind(ins);
+            const int idx = side ? F::bidx(ins) : F::aidx(ins);
+            R g[P];
+            if (side ? F::tape_b(ins) : ta) {
+                const R d = (R)tape[t + (side ? ta : 0)];
+                CUSR_FOR_P g[p] = safe_mul<R>(adj[p], d);
+            } else if (side && F::fid(ins) == OP_SUB) {
+                CUSR_FOR_P g[p] = (adj[p] == R(0)) ? R(0) : -adj[p];
+            } else {
+                CUSR_FOR_P g[p] = (adj[p] == R(0)) ? R(0) : adj[p];
+            }
+            if (kind == OPD_ACC) {
+                CUSR_FOR_P accadj[p] = g[p];
+            } else if (kind == OPD_SLOT) {
+                CUSR_FOR_P lds_at<R, P>(w.x, crow + idx, p, lane) = g[p];
+            } else {
+                add_tangent<K, R, P>(T, idx, g);
+            }
+        }
+    }
+}
+
 // Reverse sweep over the tape written by forward_pass<..., 2>:
 // T[p*K + k] = d f / d c_k, T zero on entry (cusr/kernel/revad_interp.cuh:131-156). The
-// adjoints of spilled values live in the slot area (their values are dead).
+// adjoints of spilled values live in the slots' rows (their values are dead).
+// V subtrees hold no constant, so the sweep ends at their rows; a C subtree
+// is swept where its root's adjoint arises.
 template <int K, typename R, int P, typename F = FastFmt>
-__device__ __forceinline__ void reverse_pass(ProgPtr prog, int n, const WaveLds<R, P> &w,
+__device__ __forceinline__ void reverse_pass(ProgPtr prog, int n, ProgPtr progc,
+                                             const WaveLds<R, P> &w, const double *ctape, int crow,
                                              int lane, R *T) {
     R accadj[P];
     CUSR_FOR_P accadj[p] = R(1);
@@ -803,12 +958,16 @@ __device__ __forceinline__ void reverse_pass(ProgPtr prog, int n, const WaveLds<
         R adj[P];
         if (F::toslot(ins)) {
             const int di = F::didx(ins);
-            CUSR_FOR_P adj[p] = lds_at<R, P>(w.slot, di, p, lane);
+            CUSR_FOR_P adj[p] = lds_at<R, P>(w.x, di, p, lane);
         } else {
             CUSR_FOR_P adj[p] = accadj[p];
         }
         const int t = F::tape(ins), ta = F::tape_a(ins);
         const int nop = F::binary(ins) ? 2 : 1;
+        // an operand that is a C subtree is swept after the operands: its
+        // adjoint waits in gc, accadj may hold the other operand's
+        int at = -1;
+        R gc[P];
         for (int side = 0; side < nop; ++side) {
             const int kind = side ? F::bkind(ins) : F::akind(ins);
             const int idx = side ? F::bidx(ins) : F::aidx(ins);
@@ -827,22 +986,36 @@ __device__ __forceinline__ void reverse_pass(ProgPtr prog, int n, const WaveLds<
             if (kind == OPD_ACC) {
                 CUSR_FOR_P accadj[p] = g[p];
             } else if (kind == OPD_SLOT) {
-                CUSR_FOR_P lds_at<R, P>(w.slot, idx, p, lane) = g[p];
+                CUSR_FOR_P lds_at<R, P>(w.x, idx, p, lane) = g[p];
+            } else if (F::root(ins)) {
+                at = F::cidx(ins);
+                CUSR_FOR_P gc[p] = g[p];
             } else {
                 add_tangent<K, R, P>(T, idx, g);   // T starts at 0: 0 + adjoint
             }
         }
+        if (at >= 0) reverse_const<K, R, P, F>(progc, at, w, ctape, crow, lane, gc, T);
     }
 }
 
 // ------------------------------------------------------- one data pass
 
+// What a pass does with an expression's V program (program.h): run it in
+// every batch, run it and keep its values in the workspace, or load them.
+enum { V_RUN = 0, V_KEEP = 1, V_LOAD = 2 };
+
 struct PassArgs {
-    ProgPtr prog;       // this expression's program
-    int n;
+    ProgPtr prog;       // this expression's staged program: C, V, M
+    int n_c, n_v, n_m;
+    int mvars, vrows, ovars, crow;   // ExprDesc
+    int Kr;             // constants
+    uint64_t map;
+    int vmode;          // V_*
+    void *V;            // [vrows][N] workspace columns, of the fit's type (null: none)
+    UniLds u;           // C's scalars (n_c > 0)
     const double *X;    // [D][N] column-major
     const double *y;    // this expression's targets [N]
-    int N, D;
+    int N;
     int parts;          // point partitions G (64-point granule g -> partition g mod G)
     int pwaves;         // wavefronts of the workgroup; wave w sums partitions w, w+pwaves, ...
     int wave;           // this wavefront
@@ -854,6 +1027,91 @@ struct PassArgs {
     int part_stride;    // split: doubles between partitions in part (the launch's
                         // widest sums row, which the step kernel reads by)
 };
+
+// The program part of PassArgs from an expression's descriptor. v: the fit's
+// workspace (null: none), uni: this wavefront's scalar area.
+template <typename R, typename F>
+__device__ __forceinline__ void program_args(PassArgs &a, const uint64_t *prog, const ExprDesc &e,
+                                             int Kr, int N, void *v, double *uni) {
+    a.prog = (ProgPtr)(prog + e.prog_off);
+    a.n_c = e.n_c;
+    a.n_v = e.n_v;
+    a.n_m = e.n_m;
+    a.mvars = e.mvars;
+    a.vrows = e.vrows;
+    a.ovars = e.ovars;
+    a.crow = e.crow;
+    a.Kr = Kr;
+    a.map = e.map;
+    a.V = (v && e.vrows > 0) ? (void *)((R *)v + (size_t)e.v_col * N) : nullptr;
+    a.vmode = a.V ? V_LOAD : V_RUN;
+    a.u = uni_lds(uni, Kr, e.cslots);
+    a.N = N;
+}
+
+// The constants M and V read: C's values in place, and in forward AD their
+// tangents in u.t0.
+template <int K, typename R, int JAC, typename F>
+__device__ __forceinline__ const double *pass_constants(const PassArgs &a, const double *cs,
+                                                        int lane) {
+    if (a.n_c == 0) return cs;
+    const_phase<K, R, JAC, F>(a.prog, a.n_c, a.u, cs, lane, a.Kr);
+    return a.u.cm;
+}
+
+// One batch's rows to LDS: M's variables, then V's values (V_LOAD) or V's other
+// variables. Each load is a whole memory latency (1,000 to 2,000 cycles beside
+// other wavefronts), so the loads of kStageRows rows are in flight at once.
+constexpr int kStageRows = 4;
+template <typename R, int P, typename T, typename Src>
+__device__ __forceinline__ void stage_from(const WaveLds<R, P> &w, int first, int n,
+                                           const int (&ic)[P], int lane, const Src &src) {
+    for (int r0 = 0; r0 < n; r0 += kStageRows) {
+        T xv[kStageRows][P];
+#pragma unroll
+        for (int k = 0; k < kStageRows; ++k)
+            if (r0 + k < n) {
+                const T *col = src(r0 + k);
+                CUSR_FOR_P xv[k][p] = col[ic[p]];
+            }
+#pragma unroll
+        for (int k = 0; k < kStageRows; ++k)
+            if (r0 + k < n) CUSR_FOR_P lds_at<R, P>(w.x, first + r0 + k, p, lane) = (R)xv[k][p];
+    }
+}
+template <typename R, int P, typename F>
+__device__ __forceinline__ void stage_rows(const PassArgs &a, const WaveLds<R, P> &w,
+                                           const int (&ic)[P], int lane) {
+    const ProgPtr rows = a.prog + F::kWords * (a.n_c + a.n_v + a.n_m);
+    const auto var = [&](int r) { return a.X + (size_t)F::var(rows, a.map, r) * a.N; };
+    if (a.vmode == V_LOAD) {
+        if constexpr (std::is_same<R, double>::value) {
+            stage_from<R, P, double>(w, 0, a.mvars + a.vrows, ic, lane, [&](int r) {
+                return r < a.mvars ? var(r) : (const double *)a.V + (size_t)(r - a.mvars) * a.N;
+            });
+        } else {
+            stage_from<R, P, double>(w, 0, a.mvars, ic, lane, var);
+            stage_from<R, P, R>(w, a.mvars, a.vrows, ic, lane,
+                                [&](int r) { return (const R *)a.V + (size_t)r * a.N; });
+        }
+    } else {
+        stage_from<R, P, double>(w, 0, a.mvars, ic, lane, var);
+        stage_from<R, P, double>(w, a.mvars + a.vrows, a.ovars, ic, lane,
+                                 [&](int r) { return var(a.mvars + r); });
+    }
+}
+
+// V's values of one batch to the workspace (V_KEEP), for the fit's later
+// passes: the lane that reads a point there is the one that wrote it, or runs
+// in a later launch.
+template <typename R, int P>
+__device__ __forceinline__ void keep_rows(const PassArgs &a, const WaveLds<R, P> &w,
+                                          const int (&ic)[P], const bool (&valid)[P], int lane) {
+    if (a.vmode != V_KEEP) return;
+    R *col = (R *)a.V;
+    for (int r = 0; r < a.vrows; ++r, col += a.N)
+        CUSR_FOR_P if (valid[p]) col[ic[p]] = lds_at<R, P>(w.x, a.mvars + r, p, lane);
+}
 
 // Matrix sums (forward AD, K >= CO_SUMS_MATRIX_MIN_K): v_mfma_f64_16x16x4 takes A[i][k]
 // from lane i + 16k and B[k][j] from lane j + 16k, and returns D[i][j] in
@@ -975,12 +1233,6 @@ __device__ __forceinline__ void wave_reduce_store(const double (&acc)[W], double
     }
 }
 
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_s_waitcnt(0);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-}
-
 // LDS visibility for every wavefront of the workgroup (pwaves uniform).
 __device__ __forceinline__ void block_sync(int pwaves) {
     if (pwaves > 1) __syncthreads();
@@ -1000,6 +1252,12 @@ __device__ __forceinline__ void data_pass(const PassArgs &a, const WaveLds<R, P>
     constexpr int WL = MX ? ((K < 16) ? 1 : 1 + K) : W;
     const int granules = (a.N + kLanes - 1) / kLanes;
     const int last = a.N - 1;
+    cs = pass_constants<K, R, JAC, F>(a, cs, lane);
+    const ProgPtr prog_v = a.prog + F::kWords * a.n_c, prog_m = prog_v + F::kWords * a.n_v;
+    // V and M are one program, run from V's start or from M's
+    const bool load_v = a.vmode == V_LOAD;
+    const ProgPtr run = load_v ? prog_m : prog_v;
+    const int n_run = load_v ? a.n_m : a.n_v + a.n_m;
     for (int part = a.wave; part < a.parts; part += a.pwaves) {
     double acc[WL];
 #pragma unroll
@@ -1022,19 +1280,28 @@ __device__ __forceinline__ void data_pass(const PassArgs &a, const WaveLds<R, P>
             ic[p] = valid[p] ? i : last;
         }
         CUSR_FOR_P yv[p] = a.y[ic[p]];
-#pragma unroll 2
-        for (int v = 0; v < a.D; ++v) {
-            const double *col = a.X + (size_t)v * a.N;
-            double xv[P];
-            CUSR_FOR_P xv[p] = col[ic[p]];
-            CUSR_FOR_P lds_at<R, P>(w.x, v, p, lane) = (R)xv[p];
-        }
+        stage_rows<R, P, F>(a, w, ic, lane);
         R accv[P];
         R T[P * KT];
+        if constexpr (JAC == 1) {
+            if (a.n_c > 0) {
 #pragma unroll
-        for (int j = 0; j < P * KT; ++j) T[j] = (JAC == 1) ? R(1) : R(0);
-        forward_pass<K, R, P, JAC, F>(a.prog, a.n, w, cs, lane, accv, T);
-        if constexpr (JAC == 2) reverse_pass<K, R, P, F>(a.prog, a.n, w, lane, T);
+                for (int j = 0; j < K; ++j) {
+                    const R t = (R)a.u.t0[j];
+                    CUSR_FOR_P T[p * KT + j] = t;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < P * KT; ++j) T[j] = R(1);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < P * KT; ++j) T[j] = R(0);
+        }
+        forward_pass<K, R, P, JAC, F>(run, n_run, w, cs, lane, accv, T);
+        keep_rows<R, P>(a, w, ic, valid, lane);
+        if constexpr (JAC == 2)
+            reverse_pass<K, R, P, F>(prog_m, a.n_m, a.prog, w, a.u.tape, a.crow, lane, T);
         if constexpr (MX) {
             CUSR_FOR_P {
                 const double r = valid[p] ? (double)accv[p] - yv[p] : 0.0;
@@ -1161,6 +1428,11 @@ __device__ __forceinline__ void data_pass_gen(const PassArgs &a, const WaveLds<R
     const int granules = (a.N + kLanes - 1) / kLanes;
     const int last = a.N - 1;
     double *jt = a.jt;
+    cs = pass_constants<K, R, JAC, F>(a, cs, lane);
+    const ProgPtr prog_v = a.prog + F::kWords * a.n_c, prog_m = prog_v + F::kWords * a.n_v;
+    const bool load_v = a.vmode == V_LOAD;
+    const ProgPtr run = load_v ? prog_m : prog_v;
+    const int n_run = load_v ? a.n_m : a.n_v + a.n_m;
     const int c16 = lane & 15;
     const int col0 = c16 < Kr ? c16 : Kr;
     const int col1 = 16 + c16 < Kr ? 16 + c16 : Kr;
@@ -1171,21 +1443,26 @@ __device__ __forceinline__ void data_pass_gen(const PassArgs &a, const WaveLds<R
         for (int gi = 0; gi < ng; ++gi) {
             // points past N read point N-1 (in bounds) and stage a zero row
             const int i = (part + a.parts * gi) * kLanes + lane;
-            const bool valid = i < a.N;
-            const int ic = valid ? i : last;
-            const double yv = a.y[ic];
-            for (int v = 0; v < a.D; ++v)
-                lds_at<R, 1>(w.x, v, 0, lane) = (R)a.X[(size_t)v * a.N + ic];
+            const bool valid[1] = {i < a.N};
+            const int ic[1] = {valid[0] ? i : last};
+            const double yv = a.y[ic[0]];
+            stage_rows<R, 1, F>(a, w, ic, lane);
             R accv[1];
             R T[K];
 #pragma unroll
             for (int j = 0; j < K; ++j) T[j] = (JAC == 1) ? R(1) : R(0);
-            forward_pass<K, R, 1, JAC, F>(a.prog, a.n, w, cs, lane, accv, T);
-            if constexpr (JAC == 2) reverse_pass<K, R, 1, F>(a.prog, a.n, w, lane, T);
-            const double r = valid ? (double)accv[0] - yv : 0.0;
+            if (JAC == 1 && a.n_c > 0) {
+#pragma unroll
+                for (int j = 0; j < K; ++j) T[j] = (R)a.u.t0[j];
+            }
+            forward_pass<K, R, 1, JAC, F>(run, n_run, w, cs, lane, accv, T);
+            keep_rows<R, 1>(a, w, ic, valid, lane);
+            if constexpr (JAC == 2)
+                reverse_pass<K, R, 1, F>(prog_m, a.n_m, a.prog, w, a.u.tape, a.crow, lane, T);
+            const double r = valid[0] ? (double)accv[0] - yv : 0.0;
             double *row = jt + lane * kGenStride;
 #pragma unroll
-            for (int j = 0; j < K; ++j) row[j] = valid ? (double)T[j] : 0.0;
+            for (int j = 0; j < K; ++j) row[j] = valid[0] ? (double)T[j] : 0.0;
             row[Kr] = r;
             wave_sync_lds();
 #pragma unroll
@@ -1405,12 +1682,15 @@ struct FitArgs {
     double *loss_init;      // [M] out
     double *loss_final;     // [M] out
     int32_t *iters;         // [M] out
-    int N, D, max_iter, guard, lm_order;
+    int N, max_iter, guard, lm_order;
     int damp;               // CO_DAMP_* of the solve
     int shared_y;           // 1: Y is one row [N] shared by every expression
     int f32_range;          // 1: constants and losses held to the fp32 range
     double lambda0, xtol;
-    int slots, tape;        // per-wave LDS rows of this launch ([row][P][64] each)
+    int rows, tape;         // per-wave LDS rows of this launch ([row][P][64] each)
+    void *V;                // [columns][N] workspace of the V values (null: run V in
+                            // every pass), of the fit's type
+    int uni_bytes;          // per-wave scalar area of this launch, its first bytes
     int parts;              // point partitions per expression (1, 2 or 4)
     int pwaves;             // wavefronts of the workgroup (divides parts)
     int wave_bytes;         // dynamic LDS of one wavefront; partition sums follow
@@ -1445,10 +1725,10 @@ __device__ __forceinline__ bool loss_ok(const FitArgs &fa, double loss) {
 }
 
 // Static LDS of a fit kernel: current and trial constants, current and trial
-// sums, sized for the kernel family's largest K.
-template <bool GEN>
+// sums of the kernel's K (the general kernel: of the largest).
+template <bool GEN, int K>
 struct FitStatic {
-    static constexpr int KC = GEN ? CO_MAX_K : CO_FAST_MAX_K;
+    static constexpr int KC = GEN ? CO_MAX_K : (K > 0 ? K : 1);
     static constexpr int SW = sums_width(KC);
 };
 
@@ -1471,10 +1751,14 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     typedef typename std::conditional<GEN, WideFmt, FastFmt>::type F;
     constexpr int P = fit_points<GEN, R, K, AD, LN>();
     constexpr int JAC = (K == 0) ? 0 : (AD == CO_AD_REVERSE ? 2 : 1);
-    constexpr int KC = FitStatic<GEN>::KC;
+    constexpr int KC = FitStatic<GEN, K>::KC;
     const int Kr = GEN ? e.K : K;   // the expression's K (wave-uniform)
     char *my_lds = lds_dyn + (size_t)wave * fa.wave_bytes;
     const bool lead = wave == 0;     // the wavefront that writes shared state
+    PassArgs pa;
+    program_args<R, F>(pa, fa.prog, e, Kr, fa.N, fa.max_iter > 0 ? fa.V : nullptr,
+                       (double *)my_lds);
+    my_lds += fa.uni_bytes;
     double *jt = (double *)my_lds;   // matrix sums: the slice's augmented rows first
     // then the K x K Cholesky factor and rhs (the general kernel's solve
     // reuses the rows' bytes: it runs between passes; reverse AD puts both
@@ -1489,17 +1773,11 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     }
     WaveLds<R, P> wl;
     wl.x = (R *)my_lds;
-    wl.slot = wl.x + (size_t)fa.D * P * kLanes;
-    wl.tape = wl.slot + (size_t)fa.slots * P * kLanes;
+    wl.tape = wl.x + (size_t)fa.rows * P * kLanes;
     if constexpr (!GEN && sums_over_tape<K, AD>()) jt = (double *)wl.tape;
     double *lds_l = GEN ? jt : jt + kLanes * kJtStride;
-    PassArgs pa;
-    pa.prog = (ProgPtr)(fa.prog + e.prog_off);
-    pa.n = e.n;
     pa.X = fa.X;
     pa.y = fa.Y + (fa.shared_y ? (size_t)0 : (size_t)e.y_row * fa.N);
-    pa.N = fa.N;
-    pa.D = fa.D;
     pa.parts = fa.parts;
     pa.pwaves = fa.pwaves;
     pa.wave = wave;
@@ -1509,19 +1787,23 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     pa.part_stride = 0;
 
     double *c_cur = lds_c, *c_try = lds_c + KC;
-    double *s_cur = lds_s, *s_try = lds_s + FitStatic<GEN>::SW;
+    double *s_cur = lds_s, *s_try = lds_s + FitStatic<GEN, K>::SW;
     double *sv = fa.state ? fa.state + (size_t)e.y_row * fa.state_stride : nullptr;
     double loss, loss_init, lambda;
     int st, it;
     if (!fa.resume) {
         if (lead && lane < Kr) c_cur[lane] = fa.C0[e.c_off + lane];
         block_sync(fa.pwaves);
+        // the first pass runs V and keeps its values for the others
+        const int vmode = pa.vmode;
+        if (vmode == V_LOAD) pa.vmode = V_KEEP;
         if constexpr (GEN) {
             if (Kr == 0) data_pass<0, R, 1, 0, F>(pa, wl, c_cur, s_cur, lane);
             else data_pass_gen<R, JAC, F>(pa, wl, c_cur, s_cur, lane, Kr);
         } else {
             data_pass<K, R, P, JAC, F>(pa, wl, c_cur, s_cur, lane);
         }
+        pa.vmode = vmode;
         loss = uni(0.5 * s_cur[0]);
         loss_init = loss;
         st = (Kr == 0) ? ST_K0 : (loss_ok(fa, loss) ? ST_RUN : ST_NAN);
@@ -1671,8 +1953,8 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
         constexpr int KA = GEN ? 0 : K;
         WaveLds<double, AP> w64;
         w64.x = (double *)my_lds;
-        w64.slot = w64.x + (size_t)fa.D * AP * kLanes;
-        w64.tape = w64.slot + (size_t)fa.slots * AP * kLanes;
+        w64.tape = w64.x + (size_t)fa.rows * AP * kLanes;
+        pa.vmode = V_RUN;   // the workspace holds the fit's fp32 values
         data_pass<KA, double, AP, 0, F>(pa, w64, c_cur, s_try, lane);
         lf = uni(0.5 * s_try[0]);
         if (fa.pwaves > 1) __syncthreads();
@@ -1750,8 +2032,8 @@ constexpr bool large_n_variant() {
 template <int K, typename R, int AD, int LN = 0>
 __global__ void __launch_bounds__(kLanes * CO_MAX_PARTITIONS, (waves_per_eu<R, K, AD, LN>()))
 lm_fit_kernel(FitArgs fa) {
-    __shared__ double lds_c[2 * FitStatic<false>::KC];
-    __shared__ double lds_s[2 * FitStatic<false>::SW];
+    __shared__ double lds_c[2 * FitStatic<false, K>::KC];
+    __shared__ double lds_s[2 * FitStatic<false, K>::SW];
     extern __shared__ char lds_dyn[];
     const ExprDesc e = fa.desc[blockIdx.x];
     const int lane = (int)threadIdx.x & (kLanes - 1);
@@ -1767,8 +2049,8 @@ lm_fit_kernel(FitArgs fa) {
 template <typename R, int AD>
 __global__ void __launch_bounds__(kLanes * CO_MAX_PARTITIONS, CUSR_WAVES_GEN)
 lm_fit_gen_kernel(FitArgs fa) {
-    __shared__ double lds_c[2 * FitStatic<true>::KC];
-    __shared__ double lds_s[2 * FitStatic<true>::SW];
+    __shared__ double lds_c[2 * FitStatic<true, kGenK>::KC];
+    __shared__ double lds_s[2 * FitStatic<true, kGenK>::SW];
     extern __shared__ char lds_dyn[];
     const ExprDesc e = fa.desc[blockIdx.x];
     const int lane = (int)threadIdx.x & (kLanes - 1);
@@ -1776,38 +2058,51 @@ lm_fit_gen_kernel(FitArgs fa) {
     fit_one<kGenK, R, AD, 0, true>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
 }
 
-// Static LDS bytes of a fit kernel family (kept out of the dynamic budget).
-constexpr size_t fit_static_lds(bool gen) {
-    return gen ? (2 * FitStatic<true>::KC + 2 * FitStatic<true>::SW) * sizeof(double)
-               : (2 * FitStatic<false>::KC + 2 * FitStatic<false>::SW) * sizeof(double);
+// Static LDS bytes of a bin's fit kernel (kept out of the dynamic budget).
+constexpr size_t fit_static_lds(int bin) {
+    const int kc = bin == CO_GENERAL_BIN ? CO_MAX_K : (bin > 0 ? bin : 1);
+    return (2 * kc + 2 * sums_width(kc)) * sizeof(double);
 }
 
-// Dynamic LDS bytes one wavefront of a fit launch needs (the mixed-precision
+// Dynamic LDS bytes one wavefront of a fit launch needs beside its scalar area (the mixed-precision
 // fp64 audit pass reuses the same bytes at audit_points per lane).
 template <typename R, int K, int AD, int LN = 0>
-constexpr size_t fit_lds_bytes_t(int D, int slots, int tape) {
+constexpr size_t fit_lds_bytes_t(int rows, int tape) {
     const size_t row = (size_t)points_per_pass<R, K, AD, LN>() * kLanes * sizeof(R);
     const size_t mx = matrix_sums<K, AD>() ? kJtBytes + (size_t)K * (K + 1) * sizeof(double) : 0;
     const size_t t = sums_over_tape<K, AD>() && mx > (size_t)tape * row ? mx : (size_t)tape * row;
-    const size_t a = (size_t)(D + slots) * row + t;
-    const size_t b = (size_t)(D + slots) * audit_points<R, K, AD, LN>() * kLanes * sizeof(double);
+    const size_t a = (size_t)rows * row + t;
+    const size_t b = (size_t)rows * audit_points<R, K, AD, LN>() * kLanes * sizeof(double);
     return (sums_over_tape<K, AD>() ? 0 : mx) + (a > b ? a : b);
 }
 
 // ... of a general-kernel launch (one point per lane; the fp64 audit at one)
 template <typename R>
-constexpr size_t fit_lds_bytes_gen(int D, int slots, int tape) {
-    const size_t a = (size_t)(D + slots + tape) * kLanes * sizeof(R);
-    const size_t b = (size_t)(D + slots) * kLanes * sizeof(double);
+constexpr size_t fit_lds_bytes_gen(int rows, int tape) {
+    const size_t a = (size_t)(rows + tape) * kLanes * sizeof(R);
+    const size_t b = (size_t)rows * kLanes * sizeof(double);
     return kGenJtBytes + (a > b ? a : b);
 }
 
-// Launch the fit kernel of one bin (k <= CO_FAST_MAX_K: the fast kernel of
-// K = k; CO_GENERAL_BIN: the general kernel) for one (precision, AD mode).
-hipError_t launch_fit_f64_fwd(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_fit_f64_rev(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_fit_f32_fwd(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_fit_f32_rev(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
+// Launch the fit or pass kernel of one bin (k <= CO_FAST_MAX_K: the fast kernel
+// of K = k; CO_GENERAL_BIN: the general kernel) for one (precision, AD mode).
+// fit_kernels.hip defines a launcher for each part of the bins (part_of_bin).
+typedef hipError_t (*Launcher)(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
+constexpr int kParts = 3;
+constexpr int part_of_bin(int bin) { return bin <= 4 ? 0 : bin <= 8 ? 1 : 2; }
+#define CUSR_DECLARE_LAUNCHER(name)                                                  \
+    hipError_t name##_0(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
+    hipError_t name##_1(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
+    hipError_t name##_2(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
+    constexpr Launcher name[kParts] = {name##_0, name##_1, name##_2}
+CUSR_DECLARE_LAUNCHER(launch_fit_f64_fwd);
+CUSR_DECLARE_LAUNCHER(launch_fit_f64_rev);
+CUSR_DECLARE_LAUNCHER(launch_fit_f32_fwd);
+CUSR_DECLARE_LAUNCHER(launch_fit_f32_rev);
+CUSR_DECLARE_LAUNCHER(launch_pass_f64_fwd);
+CUSR_DECLARE_LAUNCHER(launch_pass_f64_rev);
+CUSR_DECLARE_LAUNCHER(launch_pass_f32_fwd);
+CUSR_DECLARE_LAUNCHER(launch_pass_f32_rev);
 
 // ------------------------------------------------------ plain evaluation
 
@@ -1817,7 +2112,8 @@ struct EvalArgs {
     const double *X;   // [D][N]
     const double *C;   // [total_c]
     double *Yout;      // [M][N]
-    int N, D;
+    int N;
+    int uni_bytes;     // scalar area of the staged programs, the first LDS bytes
 };
 
 template <typename R, typename F>
@@ -1828,20 +2124,23 @@ __global__ void __launch_bounds__(kLanes) eval_kernel(EvalArgs ea) {
     const int lane = threadIdx.x;
     const ExprDesc e = ea.desc[blockIdx.x];
     if (lane < e.K) cs[lane] = ea.C[e.c_off + lane];
+    PassArgs a;
+    program_args<R, F>(a, ea.prog, e, e.K, ea.N, nullptr, (double *)lds_dyn);
+    a.X = ea.X;
     WaveLds<R, P> w;
-    w.x = (R *)lds_dyn;
-    w.slot = w.x + (size_t)ea.D * kLanes;
-    w.tape = w.slot;
+    w.x = (R *)(lds_dyn + ea.uni_bytes);
+    w.tape = nullptr;
     wave_sync_lds();
-    const ProgPtr prog = (ProgPtr)(ea.prog + e.prog_off);
+    const double *cv = pass_constants<0, R, 0, F>(a, cs, lane);
     const int batches = (ea.N + kLanes - 1) / kLanes;
     for (int bt = 0; bt < batches; ++bt) {
         const int i = lane + kLanes * bt;
         const bool valid = i < ea.N;
-        for (int v = 0; v < ea.D; ++v)
-            lds_at<R, P>(w.x, v, 0, lane) = valid ? (R)ea.X[(size_t)v * ea.N + i] : R(0);
+        const int ic[P] = {valid ? i : ea.N - 1};
+        stage_rows<R, P, F>(a, w, ic, lane);
         R accv[1], T[1];
-        forward_pass<0, R, P, 0, F>(prog, e.n, w, cs, lane, accv, T);
+        forward_pass<0, R, P, 0, F>(a.prog + F::kWords * e.n_c, e.n_v + e.n_m, w, cv, lane, accv,
+                                    T);
         if (valid) ea.Yout[(size_t)e.y_row * ea.N + i] = (double)accv[0];
     }
 }

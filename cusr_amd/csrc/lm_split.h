@@ -58,7 +58,7 @@ template <int K, typename R, int AD, int LN, bool GEN>
 __global__ void __launch_bounds__(kLanes, (GEN ? CUSR_WAVES_GEN : pass_waves_per_eu<R, (GEN ? 0 : K), AD, LN>()))
 lm_pass_kernel(FitArgs fa) {
     typedef typename std::conditional<GEN, WideFmt, FastFmt>::type F;
-    constexpr int KC = FitStatic<GEN>::KC;
+    constexpr int KC = FitStatic<GEN, K>::KC;
     constexpr int P = fit_points<GEN, R, K, AD, LN>();
     constexpr int AP = fit_audit_points<GEN, R, K, AD, LN>();
     constexpr int JAC = (K == 0) ? 0 : (AD == CO_AD_REVERSE ? 2 : 1);
@@ -77,25 +77,24 @@ lm_pass_kernel(FitArgs fa) {
                         : (kind == SP_AUDIT_CUR ? sv + kSpCCur : sv + kSpCTry);
     if (lane < Kr) cs[lane] = src[lane];
     wave_sync_lds();
-    char *my_lds = lds_dyn;
+    PassArgs pa;
+    program_args<R, F>(pa, fa.prog, e, Kr, fa.N, fa.max_iter > 0 ? fa.V : nullptr,
+                       (double *)lds_dyn);
+    if (kind == SP_INIT && pa.vmode == V_LOAD) pa.vmode = V_KEEP;
+    char *my_lds = lds_dyn + fa.uni_bytes;
     double *jt = (double *)my_lds;
     if constexpr (GEN) {
         my_lds += kGenJtBytes;
     } else if constexpr (sums_over_tape<K, AD>()) {
-        // the rows go to the Jacobian pass's tape bytes (x and slot rows first)
-        jt = (double *)(my_lds + (size_t)(fa.D + fa.slots) * P * kLanes * sizeof(R));
+        // the rows go to the Jacobian pass's tape bytes (after the interpreter's rows)
+        jt = (double *)(my_lds + (size_t)fa.rows * P * kLanes * sizeof(R));
     } else if constexpr (matrix_sums<K, AD>()) {
 #pragma unroll
         for (int j = 0; j < kJtStride; ++j) jt[lane * kJtStride + j] = 0.0;
         my_lds += kJtBytes + (size_t)K * (K + 1) * sizeof(double);
     }
-    PassArgs pa;
-    pa.prog = (ProgPtr)(fa.prog + e.prog_off);
-    pa.n = e.n;
     pa.X = fa.X;
     pa.y = fa.Y + (fa.shared_y ? (size_t)0 : (size_t)e.y_row * fa.N);
-    pa.N = fa.N;
-    pa.D = fa.D;
     pa.parts = G;
     pa.pwaves = G;      // this workgroup's wavefront sums partition `part` only
     pa.wave = part;
@@ -106,8 +105,7 @@ lm_pass_kernel(FitArgs fa) {
     if (kind == SP_INIT || kind == SP_TRIAL) {
         WaveLds<R, P> wl;
         wl.x = (R *)my_lds;
-        wl.slot = wl.x + (size_t)fa.D * P * kLanes;
-        wl.tape = wl.slot + (size_t)fa.slots * P * kLanes;
+        wl.tape = wl.x + (size_t)fa.rows * P * kLanes;
         if constexpr (GEN) {
             if (Kr == 0) data_pass<0, R, 1, 0, F>(pa, wl, cs, nullptr, lane);
             else data_pass_gen<R, JAC, F>(pa, wl, cs, nullptr, lane, Kr);
@@ -118,8 +116,8 @@ lm_pass_kernel(FitArgs fa) {
         constexpr int KA = GEN ? 0 : K;
         WaveLds<double, AP> w64;
         w64.x = (double *)my_lds;
-        w64.slot = w64.x + (size_t)fa.D * AP * kLanes;
-        w64.tape = w64.slot + (size_t)fa.slots * AP * kLanes;
+        w64.tape = w64.x + (size_t)fa.rows * AP * kLanes;
+        pa.vmode = V_RUN;   // the workspace holds the fit's fp32 values
         data_pass<KA, double, AP, 0, F>(pa, w64, cs, nullptr, lane);
     }
 }
@@ -307,11 +305,5 @@ __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) 
     }
 }
 #endif  // CUSR_SPLIT_STEP_KERNELS
-
-// Launch the pass kernel of one bin (as launch_fit_*) for one (precision, AD mode).
-hipError_t launch_pass_f64_fwd(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_pass_f64_rev(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_pass_f32_fwd(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-hipError_t launch_pass_f32_rev(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
 
 }  // namespace cusr

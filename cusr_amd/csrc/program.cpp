@@ -22,59 +22,54 @@
 
 namespace cusr {
 
-static bool unary_op(int f) {
-    switch (f) {
-    case OP_SIN: case OP_COS: case OP_TAN: case OP_SINH: case OP_COSH: case OP_TANH:
-    case OP_LOG: case OP_LOOSE_LOG: case OP_EXP: case OP_INV: case OP_LOOSE_INV:
-    case OP_NEG: case OP_ABS: case OP_SQRT: case OP_LOOSE_SQRT:
-    case OP_CEXP: case OP_SQUARE: case OP_PLOG:
-        return true;
-    default:
-        return false;
+// Per operator id: arity (0: unknown), the relative device cost of one
+// instruction per interpreter pass (VALU instructions per 64 lanes x 4 points,
+// measured with SQ_INSTS_VALU on single-operator expressions; only the launch
+// order within a K bin uses it), and whether its partials have flat branches.
+struct OpInfo {
+    uint8_t arity;
+    bool sel;
+    int16_t cost;
+};
+struct OpTable {
+    OpInfo op[64] = {};
+    constexpr OpTable() {
+        for (int f : {OP_SIN, OP_COS, OP_TAN, OP_SINH, OP_COSH, OP_TANH, OP_LOG, OP_LOOSE_LOG,
+                      OP_EXP, OP_INV, OP_LOOSE_INV, OP_NEG, OP_ABS, OP_SQRT, OP_LOOSE_SQRT,
+                      OP_CEXP, OP_SQUARE, OP_PLOG})
+            op[f].arity = 1;
+        for (int f : {OP_ADD, OP_SUB, OP_MUL, OP_DIV, OP_LOOSE_DIV, OP_POW, OP_LOOSE_POW, OP_MAX,
+                      OP_MIN, OP_LT, OP_GT, OP_LE, OP_GE, OP_PDIV})
+            op[f].arity = 2;
+        for (int f : {OP_MAX, OP_MIN, OP_LT, OP_GT, OP_LE, OP_GE, OP_PDIV, OP_CEXP}) op[f].sel = true;
+        for (OpInfo &o : op) o.cost = 100;
+        for (int f : {OP_ADD, OP_SUB}) op[f].cost = 12;
+        op[OP_MUL].cost = 23;
+        op[OP_SQUARE].cost = 83;
+        for (int f : {OP_DIV, OP_LOOSE_DIV, OP_PDIV, OP_SQRT, OP_LOOSE_SQRT}) op[f].cost = 224;
+        for (int f : {OP_EXP, OP_CEXP}) op[f].cost = 284;
+        for (int f : {OP_SIN, OP_COS}) op[f].cost = 333;
+        for (int f : {OP_LOG, OP_LOOSE_LOG, OP_PLOG}) op[f].cost = 391;
+        for (int f : {OP_TAN, OP_POW, OP_LOOSE_POW}) op[f].cost = 450;
     }
-}
-
-static bool binary_op(int f) {
-    switch (f) {
-    case OP_ADD: case OP_SUB: case OP_MUL: case OP_DIV: case OP_LOOSE_DIV:
-    case OP_POW: case OP_LOOSE_POW: case OP_MAX: case OP_MIN:
-    case OP_LT: case OP_GT: case OP_LE: case OP_GE: case OP_PDIV:
-        return true;
-    default:
-        return false;
-    }
-}
-
-// Relative device cost of one instruction per interpreter pass (VALU
-// instructions per 64 lanes x 4 points, measured with SQ_INSTS_VALU on
-// single-operator expressions); only the launch order within a K bin uses it.
-static int op_cost(int f) {
-    switch (f) {
-    case OP_ADD: case OP_SUB: return 12;
-    case OP_MUL: return 23;
-    case OP_SQUARE: return 83;
-    case OP_DIV: case OP_LOOSE_DIV: case OP_PDIV: case OP_SQRT: case OP_LOOSE_SQRT: return 224;
-    case OP_EXP: case OP_CEXP: return 284;
-    case OP_SIN: case OP_COS: return 333;
-    case OP_LOG: case OP_LOOSE_LOG: case OP_PLOG: return 391;
-    case OP_TAN: case OP_POW: case OP_LOOSE_POW: return 450;
-    default: return 100;
-    }
-}
+};
+static constexpr OpTable kOps;
+static inline bool unary_op(int f) { return f >= 0 && kOps.op[f].arity == 1; }
+static inline bool binary_op(int f) { return f >= 0 && kOps.op[f].arity == 2; }
+static inline int op_cost(int f) { return kOps.op[f].cost; }
 
 // Forward-AD and reverse-AD flags of an instruction: flat-branch select
 // rule, which of its rank ranges get scaled (ADD's partials and SUB's left
 // one are exactly 1; the identity has no partial to apply), and which partials
 // keep a reverse-AD tape slot (read, and not exactly +-1).
 struct Ins {
-    int fid, bin, ak, ai, bk, bi, toslot, di, lo, mid, hi, tape;
-    bool sel, sa, sb, ta, tb;
+    int fid, bin, ak, ai, bk, bi, lo, mid, hi, tape, cidx;
+    bool sel, sa, sb, ta, tb, root;
 };
 
 static void set_flags(Ins &w) {
     const int f = w.fid;
-    w.sel = f == OP_MAX || f == OP_MIN || f == OP_LT || f == OP_GT || f == OP_LE || f == OP_GE ||
-            f == OP_PDIV || f == OP_CEXP;
+    w.sel = kOps.op[f].sel;
     const bool unit_a = w.bin ? (f == OP_ADD || f == OP_SUB) : (f == OP_IDENT);
     const bool unit_b = !w.bin || f == OP_ADD;
     w.sa = !unit_a && w.mid > w.lo;
@@ -86,7 +81,6 @@ static uint64_t encode_fast(const Ins &w) {
     uint64_t x = (uint64_t)w.fid | (uint64_t)w.bin << 6;
     x |= (uint64_t)w.ak << 7 | (uint64_t)(w.ai & 15) << 9;
     x |= (uint64_t)w.bk << 13 | (uint64_t)(w.bi & 15) << 15;
-    x |= (uint64_t)w.toslot << 19 | (uint64_t)(w.di & 15) << 20;
     x |= (uint64_t)w.lo << 24 | (uint64_t)w.mid << 29 | (uint64_t)w.hi << 34;
     x |= (uint64_t)w.tape << 39;
     x |= (uint64_t)w.sel << 47 | (uint64_t)w.sa << 48 | (uint64_t)w.sb << 49;
@@ -98,11 +92,29 @@ static void encode_wide(const Ins &w, uint64_t *out) {
     uint64_t a = (uint64_t)w.fid | (uint64_t)w.bin << 6;
     a |= (uint64_t)w.ak << 7 | (uint64_t)(w.ai & 255) << 9;
     a |= (uint64_t)w.bk << 17 | (uint64_t)(w.bi & 255) << 19;
-    a |= (uint64_t)w.toslot << 27 | (uint64_t)(w.di & 255) << 28;
     a |= (uint64_t)w.sel << 36 | (uint64_t)w.sa << 37 | (uint64_t)w.sb << 38;
     a |= (uint64_t)w.ta << 39 | (uint64_t)w.tb << 40;
     uint64_t b = (uint64_t)w.lo | (uint64_t)w.mid << 8 | (uint64_t)w.hi << 16;
     b |= (uint64_t)(uint32_t)w.tape << 24;
+    out[0] = a;
+    out[1] = b;
+}
+
+// program.h layouts of the staged program; at most `tape` bits of a tape slot
+// are kept (a longer tape fits no LDS and is refused before any launch)
+static void encode_staged(const Ins &w, bool wide, uint64_t *out) {
+    if (!wide) {
+        out[0] = encode_fast(w) | (uint64_t)w.root << 52 | (uint64_t)(w.cidx & 255) << 53;
+        return;
+    }
+    uint64_t a = (uint64_t)w.fid | (uint64_t)w.bin << 6;
+    a |= (uint64_t)w.ak << 7 | (uint64_t)(w.ai & 4095) << 9;
+    a |= (uint64_t)w.sel << 21 | (uint64_t)w.sa << 22 | (uint64_t)w.sb << 23;
+    a |= (uint64_t)w.ta << 24 | (uint64_t)w.tb << 25 | (uint64_t)w.root << 27;
+    a |= (uint64_t)w.bk << 28 | (uint64_t)(w.bi & 4095) << 32;
+    a |= (uint64_t)(w.cidx & kWideCidxMax) << 44;
+    uint64_t b = (uint64_t)w.lo | (uint64_t)w.mid << 8 | (uint64_t)w.hi << 16;
+    b |= (uint64_t)(w.tape & 0xfffff) << 44;
     out[0] = a;
     out[1] = b;
 }
@@ -125,14 +137,32 @@ struct Visit {
     int stage;  // 0: nothing evaluated, 1: first operand done, 2: both done
 };
 
+// A node of a staged program. Operators of its subtree in all (ops) and in M
+// (mops, with every one-class subtree of operators an operand); then, top
+// down: its program, the first instruction of its subtree there, the slots
+// live while it runs, and the slot or row its value goes to (-1: ACC, -2: a C
+// subtree's value).
+struct StagedNode {
+    int ops, mops, start, dest;
+    uint8_t prog, live;
+};
+
 // Per-thread working arrays, grown to the largest expression seen and not
 // cleared between expressions (every entry read is written first).
 struct TreeScratch {
     std::vector<int> size, left, cc, need, depth_stack;
+    // staged programs: bit 0 variables, bit 1 constants in the subtree; slots of
+    // M; and what the emission hands down
+    std::vector<int> cls, needm;
+    std::vector<StagedNode> st;
+    int rows[CO_MAX_VARS + 1];
     std::vector<Operand> res;
     std::vector<Visit> work;
     void reserve(int n) {
         if ((int)size.size() >= n + 1) return;
+        cls.resize(n + 1);
+        needm.resize(n + 1);
+        st.resize(n + 1);
         size.resize(n + 1);
         left.resize(n + 1);
         cc.resize(n + 1);
@@ -148,15 +178,17 @@ static inline bool is_leaf(int t) { return t == NODE_VAR || t == NODE_CONST; }
 // Validate one expression (n nodes, K constants, D variables): node types,
 // operator ids, variable indices, prefix-order constant ranks and stack moves.
 // Returns CO_OK, CO_ERR_BOUNDS (value stack beyond CO_MAX_STACK) or
-// CO_ERR_PROGRAM, and its value-stack depth. Fills s.size / s.left / s.cc and
-// s.need (the spill slots of each subtree in the emission's order) for the
-// emission.
+// CO_ERR_PROGRAM, and its value-stack depth. Fills s.size / s.left / s.cc / s.cls,
+// s.needm, the counts of s.st and s.need (the spill slots of each subtree in the
+// emission's order) for the emission. stage_c: operators over constants alone
+// are class 2, to go to C; else class 3, to stay in M.
 static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int n, int K,
-                      int D, int *stack_depth, TreeScratch &s) {
+                      int D, bool stage_c, int *stack_depth, TreeScratch &s) {
     if (n <= 0) return CO_ERR_PROGRAM;
     s.reserve(n);
     int *size = s.size.data(), *left = s.left.data(), *cc = s.cc.data(), *need = s.need.data();
-    int *st = s.depth_stack.data();
+    int *st = s.depth_stack.data(), *cls = s.cls.data(), *needm = s.needm.data();
+    StagedNode *sn = s.st.data();
     // prefix pass: constant ranks must be 0..K-1 in prefix order
     cc[0] = 0;
     for (int i = 0; i < n; i++) {
@@ -172,15 +204,21 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
         const int t = nt[i];
         if (t == NODE_VAR || t == NODE_CONST) {
             if (t == NODE_VAR && node_int(nv[i], D) < 0) return CO_ERR_PROGRAM;
+            cls[i] = t == NODE_VAR ? 1 : 2;
             size[i] = 1;
-            need[i] = 0;
+            need[i] = needm[i] = 0;
+            sn[i].ops = sn[i].mops = 0;
             st[sp++] = i;
         } else if (t == NODE_UFUNC) {
             if (!unary_op(node_int(nv[i], 64))) return CO_ERR_PROGRAM;
             if (sp < 1) return CO_ERR_PROGRAM;
             const int c = st[sp - 1];
             size[i] = size[c] + 1;
+            cls[i] = cls[c] == 2 && !stage_c ? 3 : cls[c];
             need[i] = need[c];
+            needm[i] = cls[c] == 3 ? needm[c] : 0;
+            sn[i].ops = sn[c].ops + 1;
+            sn[i].mops = cls[c] == 3 ? sn[c].mops + 1 : 1;
             st[sp - 1] = i;
         } else if (t == NODE_BFUNC) {
             if (!binary_op(node_int(nv[i], 64))) return CO_ERR_PROGRAM;
@@ -189,11 +227,19 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
             --sp;
             left[i] = size[l];
             size[i] = size[l] + size[r] + 1;
+            cls[i] = cls[l] | cls[r];
+            if (cls[i] == 2 && !stage_c) cls[i] = 3;
             // the operand that needs more slots runs first; two that both need
             // instructions hold one value in a slot while the other runs
             const int nl = need[l], nr = need[r];
             const int hi = nl > nr ? nl : nr;
             need[i] = (!is_leaf(nt[l]) && !is_leaf(nt[r]) && nl == nr) ? nl + 1 : hi;
+            // the same within M, where subtrees of one class are operands
+            const bool ml = cls[l] == 3, mr = cls[r] == 3;
+            const int a = ml ? needm[l] : 0, b = mr ? needm[r] : 0;
+            needm[i] = (ml && mr && a == b) ? a + 1 : (a > b ? a : b);
+            sn[i].ops = sn[l].ops + sn[r].ops + 1;
+            sn[i].mops = (ml ? sn[l].mops : 0) + (mr ? sn[r].mops : 0) + 1;
             st[sp - 1] = i;
         } else {
             return CO_ERR_PROGRAM;
@@ -206,8 +252,8 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
     return CO_OK;
 }
 
-// An instruction's word(s) in out (fast: one word, wide: two), and the later
-// mark that sends its result to slot di.
+// Instruction k of a plain program, and the later mark that sends its result to
+// slot di.
 static inline void put_ins(uint64_t *out, bool wide, int k, Ins &w) {
     set_flags(w);
     if (wide) encode_wide(w, out + 2 * k);
@@ -217,11 +263,9 @@ static inline void put_spill(uint64_t *out, bool wide, int k, int di) {
     if (wide) out[2 * k] |= (uint64_t)1 << 27 | (uint64_t)(di & 255) << 28;
     else out[k] |= (uint64_t)1 << 19 | (uint64_t)(di & 15) << 20;
 }
-
-// Emit the instructions of a checked expression, encoded, into out in
-// execution order (out holds zeros on entry). max_slots: slots the target
-// format can address. Returns CO_OK, CO_ERR_BOUNDS or CO_ERR_PROGRAM; sets the
-// instruction count, the tape and spill-slot counts and the cost estimate.
+// Emit the plain program of a checked expression (program.h), encoded, into out
+// in execution order (out holds zeros on entry). Returns CO_OK, CO_ERR_BOUNDS or
+// CO_ERR_PROGRAM.
 //
 // Operands are evaluated in Sethi-Ullman order: when both operands of a binary
 // operator need instructions, the one whose subtree needs more spill slots runs
@@ -230,9 +274,8 @@ static inline void put_spill(uint64_t *out, bool wide, int k, int di) {
 // and its constants' tangents and adjoints do not depend on which sibling runs
 // first, and the order keeps the slot count at the minimum (at most
 // log2(nodes + 1)), which is what sizes each wavefront's LDS.
-static int emit_tree(const int32_t *nt, const float *nv, const int32_t *ci, int n, int D,
-                     bool wide, int max_slots_fmt, uint64_t *out, int *n_ins, int *tape_slots,
-                     int *slots_used, int64_t *cost, TreeScratch &s) {
+static int emit_plain(const int32_t *nt, const float *nv, const int32_t *ci, int n, int D,
+                      bool wide, uint64_t *out, TreeScratch &s) {
     const int *left = s.left.data(), *cc = s.cc.data(), *need = s.need.data(),
               *size = s.size.data();
     Operand *res = s.res.data();
@@ -241,8 +284,7 @@ static int emit_tree(const int32_t *nt, const float *nv, const int32_t *ci, int 
         return nt[i] == NODE_VAR ? Operand{OPD_VAR, node_int(nv[i], D), -1}
                                  : Operand{OPD_CONST, ci[i], -1};
     };
-    int k = 0, tape = 0, live_slots = 0, max_slots = 0;
-    int64_t c = 229;   // fixed per-pass cost, then op_cost of each instruction
+    int k = 0, tape = 0, live_slots = 0;
     if (is_leaf(nt[0])) {
         // the expression is one leaf: its value is the identity of that leaf
         const Operand a = leaf_opd(0);
@@ -252,86 +294,361 @@ static int emit_tree(const int32_t *nt, const float *nv, const int32_t *ci, int 
         w.ai = a.idx;
         w.lo = cc[0];
         w.mid = w.hi = cc[n];
-        w.tape = tape;     // the identity's partial is +1: no tape slot
-        put_ins(out, wide, k++, w);
-        c += op_cost(OP_IDENT);
-    } else {
-        int sp = 0;
-        work[sp++] = {0, 0};
-        while (sp > 0) {
-            Visit &fr = work[sp - 1];
-            const int i = fr.node;
-            const bool bin = nt[i] == NODE_BFUNC;
-            const int l = i + 1, r = bin ? i + 1 + left[i] : -1;
-            const bool both = bin && !is_leaf(nt[l]) && !is_leaf(nt[r]);
-            const int first = (!bin || (both && need[l] > need[r])) ? l : r;
-            const int second = !bin ? -1 : (first == l ? r : l);
-            if (fr.stage == 0) {
-                fr.stage = 1;
-                if (!is_leaf(nt[first])) {
-                    work[sp++] = {first, 0};
-                    continue;
-                }
-                res[first] = leaf_opd(first);
+        put_ins(out, wide, k++, w);   // the identity's partial is +1: no tape slot
+        return CO_OK;
+    }
+    int sp = 0;
+    work[sp++] = {0, 0};
+    while (sp > 0) {
+        Visit &fr = work[sp - 1];
+        const int i = fr.node;
+        const bool bin = nt[i] == NODE_BFUNC;
+        const int l = i + 1, r = bin ? i + 1 + left[i] : -1;
+        const bool both = bin && !is_leaf(nt[l]) && !is_leaf(nt[r]);
+        const int first = (!bin || (both && need[l] > need[r])) ? l : r;
+        const int second = !bin ? -1 : (first == l ? r : l);
+        if (fr.stage == 0) {
+            fr.stage = 1;
+            if (!is_leaf(nt[first])) {
+                work[sp++] = {first, 0};
+                continue;
             }
-            if (fr.stage == 1 && bin) {
-                fr.stage = 2;
-                if (both) {
-                    // the first operand's value waits in the next free slot
-                    if (live_slots >= max_slots_fmt) return CO_ERR_BOUNDS;
-                    const int slot = live_slots++;
-                    if (live_slots > max_slots) max_slots = live_slots;
-                    Operand &o = res[first];
-                    if (o.kind != OPD_ACC || o.producer < 0) return CO_ERR_PROGRAM;
-                    put_spill(out, wide, o.producer, slot);
-                    o = {OPD_SLOT, slot, -1};
-                }
-                if (!is_leaf(nt[second])) {
-                    work[sp++] = {second, 0};
-                    continue;
-                }
-                res[second] = leaf_opd(second);
-            }
-            --sp;
-            const Operand a = res[l];
-            const Operand b = bin ? res[r] : Operand{OPD_ACC, 0, -1};
-            // spill slots are used last in, first out
-            if (a.kind == OPD_SLOT) {
-                if (a.idx != live_slots - 1) return CO_ERR_PROGRAM;
-                live_slots--;
-            }
-            if (bin && b.kind == OPD_SLOT) {
-                if (b.idx != live_slots - 1) return CO_ERR_PROGRAM;
-                live_slots--;
-            }
-            Ins w = {};
-            w.fid = (int)nv[i];
-            w.bin = bin ? 1 : 0;
-            w.ak = a.kind;
-            w.ai = a.idx;
-            if (bin) {
-                w.bk = b.kind;
-                w.bi = b.idx;
-            }
-            w.lo = cc[i + 1];
-            w.hi = cc[i + size[i]];
-            w.mid = bin ? cc[i + 1 + left[i]] : w.hi;
-            w.tape = tape;
-            // reverse-AD tape slots only for partials that are read and not exactly +-1
-            const bool unit = bin && (w.fid == OP_ADD || w.fid == OP_SUB);
-            w.ta = a.kind != OPD_VAR && !unit;
-            w.tb = bin && b.kind != OPD_VAR && !unit;
-            tape += (w.ta ? 1 : 0) + (w.tb ? 1 : 0);
-            c += op_cost(w.fid);
-            res[i] = {OPD_ACC, 0, k};
-            put_ins(out, wide, k++, w);
+            res[first] = leaf_opd(first);
         }
+        if (fr.stage == 1 && bin) {
+            fr.stage = 2;
+            if (both) {
+                // the first operand's value waits in the next free slot
+                if (live_slots >= (wide ? kMaxSlotsWide : kMaxSlots)) return CO_ERR_BOUNDS;
+                const int slot = live_slots++;
+                Operand &o = res[first];
+                if (o.kind != OPD_ACC || o.producer < 0) return CO_ERR_PROGRAM;
+                put_spill(out, wide, o.producer, slot);
+                o = {OPD_SLOT, slot, -1};
+            }
+            if (!is_leaf(nt[second])) {
+                work[sp++] = {second, 0};
+                continue;
+            }
+            res[second] = leaf_opd(second);
+        }
+        --sp;
+        const Operand a = res[l];
+        const Operand b = bin ? res[r] : Operand{OPD_ACC, 0, -1};
+        // spill slots are used last in, first out
+        if (a.kind == OPD_SLOT) {
+            if (a.idx != live_slots - 1) return CO_ERR_PROGRAM;
+            live_slots--;
+        }
+        if (bin && b.kind == OPD_SLOT) {
+            if (b.idx != live_slots - 1) return CO_ERR_PROGRAM;
+            live_slots--;
+        }
+        Ins w = {};
+        w.fid = (int)nv[i];
+        w.bin = bin ? 1 : 0;
+        w.ak = a.kind;
+        w.ai = a.idx;
+        if (bin) {
+            w.bk = b.kind;
+            w.bi = b.idx;
+        }
+        w.lo = cc[i + 1];
+        w.hi = cc[i + size[i]];
+        w.mid = bin ? cc[i + 1 + left[i]] : w.hi;
+        w.tape = tape;
+        // reverse-AD tape slots only for partials that are read and not exactly +-1
+        const bool unit = bin && (w.fid == OP_ADD || w.fid == OP_SUB);
+        w.ta = a.kind != OPD_VAR && !unit;
+        w.tb = bin && b.kind != OPD_VAR && !unit;
+        tape += (w.ta ? 1 : 0) + (w.tb ? 1 : 0);
+        res[i] = {OPD_ACC, 0, k};
+        put_ins(out, wide, k++, w);
     }
     if (live_slots != 0) return CO_ERR_PROGRAM;
-    *n_ins = k;
-    *tape_slots = tape;
-    *slots_used = max_slots;
-    *cost = c;
+    return !wide && tape > 255 ? CO_ERR_BOUNDS : CO_OK;   // never: n <= 255 keeps it below
+}
+
+static int64_t program_words(int n_nodes, bool wide, bool staged);
+
+// Rows of a wavefront's LDS that an expression may use (variables, V values,
+// slots): what its plain program takes, n_vars and its slots, or this many.
+// V subtrees beyond stay in M, the last ones first. A row of the fp64 forward
+// kernels to K = 8 is 2 KB (four points per lane), and their registers let four
+// wavefronts on a SIMD at K = 1, three at 2 and 3, two beyond: as many as these
+// rows leave room for in a CU's 160 KB. Elsewhere a row is 512 bytes or 1 KB
+// (from N = 16,384 on two points per lane); more than eight rows cost reverse
+// AD wavefronts (twelve: C3 67.9 -> 70.4 ms).
+static int row_budget(int K, int N) {
+    return K > 3 || N >= 16384 ? 8 : K <= 1 ? 4 : 6;
+}
+// A wide expression with more variable rows than this is not staged: its plain
+// rows may fill the LDS, which then has no room for C's scalars.
+constexpr int kStageVarsMax = 128;
+constexpr int kRowsMax = 160;   // likewise for the rows of a staged one
+
+// Whether C pays at N points: a step of C takes about as long as a step of M
+// (one point per lane against up to four, but both wait mostly on their own
+// chains: 1,300 and 1,400 cycles on the benchmark operators at K = 8), so a
+// pass of one batch of four points per lane has nothing to gain. Measured, 60,000
+// expressions of K 1-5, ten iterations, N = 60: 5.95 ms of device time with C,
+// 5.38 without; N = 1,024 (two batches) with C is faster (16,384 expressions,
+// K 1-8: 9.10 -> 7.67 ms with C and V).
+static bool stage_constants(int N) {
+    const int granules = (N + 63) / 64, parts = co_partitions_for_n(N);
+    return (granules + parts - 1) / parts > 4;
+}
+
+// The staged program of a checked expression (program.h) and its descriptor's
+// counts; out holds zeros on entry. Operands run in emit_plain's order, in one
+// pass over the nodes, parents first: a subtree's instructions are contiguous,
+// its root's last, so each node's place follows from the operator counts.
+static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, int n, int K, int D,
+                       int N, bool wide, bool staged, uint64_t *out, ExprDesc &d, int64_t *cost,
+                       TreeScratch &s) {
+    const int *size = s.size.data(), *left = s.left.data(), *cc = s.cc.data(),
+              *need = s.need.data();
+    int *cls = s.cls.data(), *needm = s.needm.data(), *rows = s.rows;
+    StagedNode *sn = s.st.data();
+    int vars[CO_MAX_VARS + 1];         // variable rows: M's, then V's others
+    const int plain_rows = D + need[0];
+    const int budget = std::min(wide ? 4096 : kFastRows,
+                                std::max(std::min(plain_rows, kRowsMax), row_budget(K, N)));
+    bool stage = staged && K > 0;
+    // class 3 to every operator of [i, end), so that it stays in M
+    auto into_m = [&](int i, int end) {
+        for (; i < end; ++i)
+            if (!is_leaf(nt[i])) cls[i] = 3;
+    };
+    // slots and operators of M after such a change, last node first
+    auto recount = [&] {
+        for (int i = n - 1; i >= 0; i--) {
+            if (is_leaf(nt[i]) || cls[i] != 3) continue;
+            const int l = i + 1, r = nt[i] == NODE_BFUNC ? l + left[i] : -1;
+            const bool ml = cls[l] == 3, mr = r >= 0 && cls[r] == 3;
+            const int a = ml ? needm[l] : 0, b = mr ? needm[r] : 0;
+            needm[i] = ml && mr && a == b ? a + 1 : std::max(a, b);
+            sn[i].mops = (ml ? sn[l].mops : 0) + (mr ? sn[r].mops : 0) + 1;
+        }
+    };
+    if (!stage) {
+        into_m(0, n);
+        recount();
+    }
+    int mv = 0, nvars = 0, nvr = 0, vslots = 0, cslots = 0, n_c = 0, n_v = 0, tail = 0;
+    for (;;) {
+        for (int v = 0; v < D; v++) rows[v] = -1;
+        mv = nvr = vslots = cslots = n_c = n_v = 0;
+        // the variables M reads itself, and the maximal subtrees of operators
+        // over constants or variables alone
+        int last_v = -1;
+        for (int i = 0; i < n;) {
+            if (nt[i] == NODE_VAR) {
+                int &r = rows[(int)nv[i++]];
+                if (r < 0) {
+                    vars[mv] = (int)nv[i - 1];
+                    r = mv++;
+                }
+            } else if (cls[i] == 3 || nt[i] == NODE_CONST) {
+                ++i;
+            } else {
+                if (cls[i] == 2) {
+                    n_c += sn[i].ops;
+                    cslots = std::max(cslots, need[i]);
+                } else {
+                    n_v += sn[i].ops;
+                    vslots = std::max(vslots, need[i]);
+                    last_v = i;
+                    ++nvr;
+                }
+                i += size[i];
+            }
+        }
+        nvars = mv;
+        if (nvr > 0 && mv < D)
+            for (int i = 0; i < n; i++)
+                if (nt[i] == NODE_VAR && rows[(int)nv[i]] < 0) {
+                    vars[nvars] = (int)nv[i];
+                    rows[(int)nv[i]] = nvars++;
+                }
+        tail = mv + nvr;
+        if (stage && (n_c > kWideCidxMax || (wide && nvars > kStageVarsMax))) {
+            stage = false;
+            into_m(0, n);
+            recount();
+            continue;
+        }
+        if (nvr > 0 && tail + std::max(nvars - mv + vslots, cls[0] == 3 ? needm[0] : 0) > budget) {
+            into_m(last_v, last_v + size[last_v]);
+            recount();
+            continue;
+        }
+        break;
+    }
+    // rows: M's variables, V's values, then V's other variables and slots over
+    // M's slots
+    for (int r = mv; r < nvars; r++) rows[vars[r]] = r + nvr;
+    enum { C = 0, V = 1, M = 2, kCRoot = -2 };
+    const int words = wide ? 2 : 1;
+    const bool ident = is_leaf(nt[0]) || cls[0] != 3;
+    const int n_m = ident ? 1 : sn[0].mops;
+    uint64_t *base[3] = {out, out + (size_t)words * n_c, out + (size_t)words * (n_c + n_v)};
+    const int slot0[3] = {0, tail + nvars - mv, tail};
+    int at_c = 0, at_v = 0, at_row = mv;     // next C and V subtree's place
+    int tape[3] = {0, 0, 0};
+    int64_t op_costs[3] = {0, 0, 0};
+    struct Opd {
+        int kind, idx, cidx;   // cidx: C instruction of a C subtree's root, -1
+    };
+    // a leaf or, in M, a hoisted subtree, whose program gets its place
+    auto operand = [&](int i) -> Opd {
+        if (nt[i] == NODE_VAR) return {OPD_VAR, rows[(int)nv[i]], -1};
+        if (nt[i] == NODE_CONST) return {OPD_CONST, ci[i], -1};
+        StagedNode &t = sn[i];
+        t.live = 0;
+        if (cls[i] == 2) {
+            t.prog = C;
+            t.start = at_c;
+            t.dest = kCRoot;
+            at_c += t.ops;
+            return {OPD_CONST, cc[i], at_c - 1};
+        }
+        t.prog = V;
+        t.start = at_v;
+        t.dest = at_row;
+        at_v += t.ops;
+        return {OPD_VAR, at_row++, -1};
+    };
+    auto put = [&](int prog, int k, Ins &w, int dest) {
+        set_flags(w);
+        encode_staged(w, wide, base[prog] + (size_t)words * k);
+        if (dest < 0) return;
+        uint64_t *q = base[prog] + (size_t)words * k;
+        if (!wide) {
+            q[0] |= (uint64_t)1 << 19 | (uint64_t)(dest & 15) << 20;
+        } else {
+            q[0] |= (uint64_t)1 << 26;
+            q[1] |= (uint64_t)(dest & 4095) << 32;
+        }
+    };
+    if (ident) {
+        // one operand: its identity, whose partial is +1 (no tape slot)
+        const Opd a = operand(0);
+        Ins w = {};
+        w.fid = OP_IDENT;
+        w.ak = a.kind;
+        w.ai = a.idx;
+        w.mid = w.hi = cc[n];
+        w.root = a.cidx >= 0;
+        w.cidx = w.root ? a.cidx : 0;
+        op_costs[M] += op_cost(OP_IDENT);
+        put(M, 0, w, -1);
+    } else {
+        sn[0].prog = M;
+        sn[0].start = 0;
+        sn[0].live = 0;
+        sn[0].dest = -1;
+    }
+    for (int i = 0; i < n; i++) {
+        if (is_leaf(nt[i])) continue;
+        const StagedNode t = sn[i];
+        const bool bin = nt[i] == NODE_BFUNC;
+        const int l = i + 1, r = bin ? l + left[i] : l;
+        // an operand that needs instructions of this program
+        const bool il = !is_leaf(nt[l]) && (t.prog != M || cls[l] == 3);
+        const bool ir = bin && !is_leaf(nt[r]) && (t.prog != M || cls[r] == 3);
+        const int *nd = t.prog == M ? needm : need;
+        auto count = [&](int c) { return t.prog == M ? sn[c].mops : sn[c].ops; };
+        const bool both = il && ir, left_first = both && nd[l] > nd[r];
+        const int slot = slot0[t.prog] + t.live;   // where the first of two waits
+        auto place = [&](int c, bool first, int start) {
+            StagedNode &k = sn[c];
+            k.prog = t.prog;
+            k.start = start;
+            k.live = (uint8_t)(t.live + (both && !first));
+            k.dest = both && first ? slot : -1;
+        };
+        Opd a, b = {OPD_ACC, 0, -1};
+        if (il) {
+            place(l, left_first || !both, t.start + (both && !left_first ? count(r) : 0));
+            a = left_first ? Opd{OPD_SLOT, slot, -1} : Opd{OPD_ACC, 0, -1};
+        } else {
+            a = operand(l);
+        }
+        if (ir) {
+            place(r, !left_first, t.start + (left_first ? count(l) : 0));
+            if (both && !left_first) b = {OPD_SLOT, slot, -1};
+        } else if (bin) {
+            b = operand(r);
+        }
+        Ins w = {};
+        w.fid = (int)nv[i];
+        w.bin = bin;
+        w.ak = a.kind;
+        w.ai = a.idx;
+        w.bk = bin ? b.kind : 0;
+        w.bi = bin ? b.idx : 0;
+        w.lo = cc[l];
+        w.hi = cc[i + size[i]];
+        w.mid = bin ? cc[r] : w.hi;
+        w.tape = tape[t.prog];
+        const bool unit = bin && (w.fid == OP_ADD || w.fid == OP_SUB);
+        w.ta = a.kind != OPD_VAR && !unit;
+        w.tb = bin && b.kind != OPD_VAR && !unit;
+        tape[t.prog] += w.ta + w.tb;
+        op_costs[t.prog] += op_cost(w.fid);
+        // M: the operand that is a C subtree; C: a subtree's last instruction
+        const int k = t.start + count(i) - 1;
+        const bool c_root = t.dest == kCRoot;
+        w.root = c_root || a.cidx >= 0 || b.cidx >= 0;
+        w.cidx = c_root ? t.ops : a.cidx >= 0 ? a.cidx : b.cidx >= 0 ? b.cidx : 0;
+        put(t.prog, k, w, t.dest);
+    }
+    if (!wide && tape[M] > 255) return CO_ERR_BOUNDS;   // never: n <= 255 keeps it below
+    d.map = 0;
+    if (wide) {
+        uint64_t *vm = base[M] + 2 * (size_t)n_m;
+        for (int r = 0; r < nvars; r++) vm[r] = (uint64_t)vars[r];
+    } else {
+        for (int r = 0; r < nvars; r++) d.map |= (uint64_t)vars[r] << (4 * r);
+    }
+    const int mslots = ident ? 0 : needm[0];
+    d.n_c = n_c;
+    d.n_v = n_v;
+    d.n_m = n_m;
+    d.K = K;
+    d.mvars = mv;
+    d.vrows = nvr;
+    d.ovars = nvars - mv;
+    d.crow = tail + mslots;
+    d.rows = tail + std::max(nvars - mv + vslots, mslots);
+    d.rows_rev = std::max(d.rows, d.crow + cslots);
+    d.cslots = cslots;
+    d.ctape = tape[C];
+    d.tape = tape[M];
+    // V runs once in a fit and C once per pass, by one point per lane
+    *cost = 229 + op_costs[M] + op_costs[C] / 4;
+    if (wide && stage) {
+        // a wavefront's LDS in reverse AD (512 bytes a row or tape slot) must
+        // not pass what the plain program took where that may have been the
+        // device's limit
+        int plain_tape = 0;
+        for (int i = 0; i < n; i++) {
+            if (is_leaf(nt[i])) continue;
+            const bool bin = nt[i] == NODE_BFUNC;
+            const int f = (int)nv[i];
+            if (bin && (f == OP_ADD || f == OP_SUB)) continue;
+            plain_tape += nt[i + 1] != NODE_VAR;
+            if (bin) plain_tape += nt[i + 1 + left[i]] != NODE_VAR;
+        }
+        const size_t row = 64 * sizeof(double);
+        const size_t now = (d.rows_rev + d.tape) * row +
+                           uni_doubles(K, d.cslots, d.ctape) * sizeof(double);
+        if (now > (64u << 10) && now > (plain_rows + (size_t)plain_tape) * row) {
+            memset(out, 0, sizeof(uint64_t) * program_words(n, true, true));
+            return emit_staged(nt, nv, ci, n, K, D, N, wide, false, out, d, cost, s);
+        }
+    }
     return CO_OK;
 }
 
@@ -444,14 +761,26 @@ int check_header(const PopHeader *h, const int32_t *nt, const float *nv, const i
     return CO_OK;
 }
 
-// Decode the M expressions at metas (rows row_base.. of the population whose
-// header h is checked): programs into prog (word 0 of this range at word
-// word_base of the device program buffer), descriptors in launch order.
-static int decode_core(const PopHeader *h, const int32_t *nt, const float *nv,
-                       const int32_t *ci, const TreeMeta *metas, int M, int row_base,
-                       int64_t word_base, uint64_t *prog, int32_t *order, int32_t *bin_start,
-                       ExprDesc *descs, int32_t *stack, int32_t *n_ins, int32_t *prog_off,
-                       int32_t *route, Plan *plan, int64_t nodes_per_thread) {
+// Per-expression bounds of the M expressions at metas, then their kernel by a
+// count over the node types (the stack depth check_tree finds for a valid tree;
+// the full check runs with the emission, before anything is used), and their
+// program offsets: expression after expression, n_nodes words in the fast
+// format, 2 * n_nodes in the wide one (node_offset order would let overlapping
+// metas alias each other's instructions); a wide staged program of one leaf
+// takes a third word for its variable.
+static int64_t program_words(int n_nodes, bool wide, bool staged) {
+    if (!wide) return n_nodes;
+    return staged && n_nodes == 1 ? 3 : 2 * (int64_t)n_nodes;
+}
+
+struct Layout {
+    std::vector<int32_t> depth, gen, poff, rcs;
+    int64_t words = 0;
+    int n_gen = 0, nthreads = 1;
+};
+
+static int lay_out(const PopHeader *h, const int32_t *nt, const TreeMeta *metas, int M,
+                   bool staged, Layout &lo) {
     const int D = h->n_vars;
     long nsum = 0;
     for (int m = 0; m < M; m++) nsum += metas[m].n_nodes;
@@ -463,96 +792,161 @@ static int decode_core(const PopHeader *h, const int32_t *nt, const float *nv,
             return CO_ERR_PROGRAM;
         if (t.K > CO_MAX_K) return CO_ERR_BOUNDS;
     }
-    std::vector<int32_t> depth(M, 0), tapes(M, 0), poff(M), nins(M, 0), slots(M, 0);
-    std::vector<int32_t> rcs(M, CO_OK), gen(M, 0);
-    std::vector<int64_t> cost(descs ? M : 0);
+    lo.words = 0;
+    lo.n_gen = 0;
+    lo.depth.resize(M);
+    lo.gen.resize(M);
+    lo.poff.resize(M);
+    lo.rcs.assign(M, CO_OK);
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    const int nthreads = (int)std::min<int64_t>(std::min(16u, hw), nsum / nodes_per_thread + 1);
-    // phase 1: every expression's stack depth and so its kernel, by a count
-    // over the node types (the depth check_tree finds for a valid tree); the
-    // full check runs in phase 2, which still ends before anything is used
+    lo.nthreads = (int)std::min<int64_t>(std::min(16u, hw), nsum / kDecodeNodes + 1);
     auto depth_range = [&](int m0, int m1) {
         for (int m = m0; m < m1; m++) {
             const TreeMeta &t = metas[m];
             const int32_t *tnt = nt + t.node_offset;
             int sp = 0, dmax = 0;
             for (int i = t.n_nodes - 1; i >= 0; i--) {
-                if (tnt[i] == NODE_BFUNC) sp -= 1;          // two operands in, one out
-                else if (tnt[i] != NODE_UFUNC) sp += 1;     // a leaf
-                if (sp > dmax) dmax = sp;
+                // a leaf pushes one; a binary takes two and gives one
+                sp += (tnt[i] != NODE_UFUNC) - 2 * (tnt[i] == NODE_BFUNC);
+                dmax = sp > dmax ? sp : dmax;
             }
-            depth[m] = dmax;
-            gen[m] = co_fast_path(t.K, depth[m], t.n_nodes, D) ? 0 : 1;
+            lo.depth[m] = dmax;
+            lo.gen[m] = co_fast_path(t.K, dmax, t.n_nodes, D) ? 0 : 1;
         }
     };
-    chunked(M, nthreads, depth_range, depth_range);
-    // programs are laid out expression after expression: n_nodes words in the
-    // fast format, 2 * n_nodes in the wide one (node_offset order would let
-    // overlapping metas alias each other's instructions)
-    int64_t run = 0;
-    int n_gen = 0;
+    chunked(M, lo.nthreads, depth_range, depth_range);
     for (int m = 0; m < M; m++) {
-        poff[m] = (int32_t)run;
-        run += (int64_t)metas[m].n_nodes * (gen[m] ? 2 : 1);
-        n_gen += gen[m];
+        lo.poff[m] = (int32_t)lo.words;
+        lo.words += program_words(metas[m].n_nodes, lo.gen[m] != 0, staged);
+        lo.n_gen += lo.gen[m];
     }
-    // phase 2: emit and encode (expressions decode independently; C5's 1.7 M
-    // nodes take 32 ms on one thread)
-    auto emit_range = [&](int m0, int m1) {
+    return CO_OK;
+}
+
+// Check and emit every expression: emit(m, out, scratch) returns its code.
+// Expressions decode independently (C5's 1.7 M nodes take 32 ms on one thread).
+template <typename Emit>
+static int emit_all(const int32_t *nt, const float *nv, const int32_t *ci, const TreeMeta *metas,
+                    int M, int D, bool staged, bool stage_c, uint64_t *prog, Layout &lo,
+                    const Emit &emit) {
+    auto range = [&](int m0, int m1) {
         TreeScratch s;
         for (int m = m0; m < m1; m++) {
             const TreeMeta &t = metas[m];
-            const int32_t *tnt = nt + t.node_offset;
-            const float *tnv = nv + t.node_offset;
-            const int32_t *tci = ci + t.node_offset;
-            uint64_t *out = prog + poff[m];
-            const int words = t.n_nodes * (gen[m] ? 2 : 1);
+            uint64_t *out = prog + lo.poff[m];
+            const int64_t words = program_words(t.n_nodes, lo.gen[m] != 0, staged);
             if (words > 0) memset(out, 0, sizeof(uint64_t) * words);
             int dd = 0;
-            rcs[m] = check_tree(tnt, tnv, tci, t.n_nodes, t.K, D, &dd, s);
-            if (rcs[m] == CO_OK && dd != depth[m]) rcs[m] = CO_ERR_PROGRAM;   // never, for a valid tree
-            int64_t c = 0;
-            int ni = 0;
-            if (rcs[m] == CO_OK)
-                rcs[m] = emit_tree(tnt, tnv, tci, t.n_nodes, D, gen[m] != 0,
-                                   gen[m] ? kMaxSlotsWide : kMaxSlots, out, &ni, &tapes[m],
-                                   &slots[m], &c, s);
-            if (rcs[m] != CO_OK) return;
-            nins[m] = ni;
-            if (!gen[m] && tapes[m] > 255) {   // 8-bit tape field (n <= 255 keeps it below)
-                rcs[m] = CO_ERR_BOUNDS;
-                return;
-            }
-            if (descs) cost[m] = c;
+            int rc = check_tree(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset,
+                                t.n_nodes, t.K, D, stage_c, &dd, s);
+            if (rc == CO_OK && dd != lo.depth[m]) rc = CO_ERR_PROGRAM;   // never, for a valid tree
+            if (rc == CO_OK) rc = emit(m, out, s);
+            lo.rcs[m] = rc;
+            if (rc != CO_OK) return;
         }
     };
-    auto emit_all = [&](int m0, int m1) {
-        std::fill(rcs.begin(), rcs.end(), CO_OK);
-        emit_range(m0, m1);
+    auto redo = [&](int m0, int m1) {
+        std::fill(lo.rcs.begin(), lo.rcs.end(), CO_OK);
+        range(m0, m1);
     };
-    chunked(M, nthreads, emit_range, emit_all);
-    int max_tape = 0, max_n = 0, max_slots = 0;
-    std::vector<int> count(CO_MAX_K + 1, 0);
-    for (int m = 0; m < M; m++) {
-        if (rcs[m] != CO_OK) return rcs[m];
-        if (tapes[m] > max_tape) max_tape = tapes[m];
-        if (nins[m] > max_n) max_n = nins[m];
-        if (slots[m] > max_slots) max_slots = slots[m];
-        count[metas[m].K]++;
-    }
-    // stable K bins, ascending
-    std::vector<int32_t> start(CO_MAX_K + 2, 0);
-    for (int k = 0; k <= CO_MAX_K; k++) start[k + 1] = start[k] + count[k];
+    chunked(M, lo.nthreads, range, redo);
+    for (int m = 0; m < M; m++)
+        if (lo.rcs[m] != CO_OK) return lo.rcs[m];
+    return CO_OK;
+}
+
+// Stable K bins, ascending.
+static void k_bins(const TreeMeta *metas, int M, std::vector<int32_t> &start,
+                   std::vector<int32_t> &ord) {
+    start.assign(CO_MAX_K + 2, 0);
+    for (int m = 0; m < M; m++) start[metas[m].K + 1]++;
+    for (int k = 0; k <= CO_MAX_K; k++) start[k + 1] += start[k];
     std::vector<int32_t> fill(start.begin(), start.end() - 1);
-    std::vector<int32_t> ord(M);
+    ord.resize(M);
     for (int m = 0; m < M; m++) ord[fill[metas[m].K]++] = m;
+}
+
+int decode_population(const PopHeader *h, const int32_t *nt, const float *nv,
+                      const int32_t *ci, const TreeMeta *metas, uint64_t *prog,
+                      int32_t *order, int32_t *bin_start, int32_t *stack, int32_t *prog_off,
+                      int32_t *route) {
+    int rc = check_header(h, nt, nv, ci, metas);
+    if (rc != CO_OK) return rc;
+    const int M = h->M_prob, D = h->n_vars;
+    std::vector<uint64_t> tmp;
+    if (!prog) {
+        tmp.assign(h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1, 0);
+        prog = tmp.data();
+    }
+    Layout lo;
+    rc = lay_out(h, nt, metas, M, false, lo);
+    if (rc != CO_OK) return rc;
+    rc = emit_all(nt, nv, ci, metas, M, D, false, true, prog, lo,
+                  [&](int m, uint64_t *out, TreeScratch &s) {
+        const TreeMeta &t = metas[m];
+        return emit_plain(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset, t.n_nodes, D,
+                          lo.gen[m] != 0, out, s);
+    });
+    if (rc != CO_OK) return rc;
+    std::vector<int32_t> start, ord;
+    k_bins(metas, M, start, ord);
     if (order) memcpy(order, ord.data(), sizeof(int32_t) * M);
     if (bin_start) memcpy(bin_start, start.data(), sizeof(int32_t) * (CO_MAX_K + 2));
-    if (stack) memcpy(stack, depth.data(), sizeof(int32_t) * M);
-    if (n_ins) memcpy(n_ins, nins.data(), sizeof(int32_t) * M);
-    if (prog_off) memcpy(prog_off, poff.data(), sizeof(int32_t) * M);
-    if (route) memcpy(route, gen.data(), sizeof(int32_t) * M);
-    if (descs) {
+    if (stack) memcpy(stack, lo.depth.data(), sizeof(int32_t) * M);
+    if (prog_off) memcpy(prog_off, lo.poff.data(), sizeof(int32_t) * M);
+    if (route) memcpy(route, lo.gen.data(), sizeof(int32_t) * M);
+    return CO_OK;
+}
+
+// The arrays of decode_range.
+struct RangeScratch {
+    Layout lo;
+    std::vector<ExprDesc> desc;
+    std::vector<int64_t> cost;
+    std::vector<int32_t> start, ord, a, launch;
+};
+
+int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const int32_t *ci,
+                 const TreeMeta *all_metas, int m0, int m1, int64_t word_base, uint64_t *all_prog,
+                 ExprDesc *all_descs, Plan *plan) {
+    const TreeMeta *metas = all_metas + m0;
+    const int M = m1 - m0, D = h->n_vars;
+    uint64_t *prog = all_prog + word_base;
+    ExprDesc *descs = all_descs + m0;
+    // working arrays kept per calling thread: for large populations fresh pages
+    // cost a tenth of the decode
+    static thread_local RangeScratch rs;
+    Layout &lo = rs.lo;
+    int rc = lay_out(h, nt, metas, M, true, lo);
+    if (rc != CO_OK) return rc;
+    if ((int)rs.desc.size() < M) rs.desc.resize(M);
+    if ((int)rs.cost.size() < M) rs.cost.resize(M);
+    ExprDesc *desc = rs.desc.data();
+    int64_t *cost = rs.cost.data();
+    rc = emit_all(nt, nv, ci, metas, M, D, true, stage_constants(h->N), prog, lo,
+                  [&](int m, uint64_t *out, TreeScratch &s) {
+        const TreeMeta &t = metas[m];
+        ExprDesc &d = desc[m];
+        d.prog_off = (int32_t)(word_base + lo.poff[m]);
+        d.c_off = t.c_offset;
+        d.y_row = m0 + m;
+        d.gen = lo.gen[m];
+        return emit_staged(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset, t.n_nodes,
+                           t.K, D, h->N, lo.gen[m] != 0, true, out, d, &cost[m], s);
+    });
+    if (rc != CO_OK) return rc;
+    int max_rows = 0, max_cslots = 0;
+    int64_t vcols = 0;
+    for (int m = 0; m < M; m++) {
+        ExprDesc &d = desc[m];
+        if (d.rows > max_rows) max_rows = d.rows;
+        if (d.cslots > max_cslots) max_cslots = d.cslots;
+        d.v_col = (int32_t)vcols;
+        vcols += d.vrows;
+    }
+    std::vector<int32_t> &start = rs.start, &ord = rs.ord;
+    k_bins(metas, M, start, ord);
+    {
         // launch positions: the general kernel's bin first, then the fast K
         // bins, largest K first; within a bin by K descending (the general
         // bin) and the costliest programs first (fixed per-pass cost plus
@@ -562,7 +956,9 @@ static int decode_core(const PopHeader *h, const int32_t *nt, const float *nv,
         // kCostBuckets), by K descending, by kernel (general first); ties keep
         // the order of ord reversed
         constexpr int kCostBuckets = 1 << 15;
-        std::vector<int32_t> a(M), launch(M);
+        std::vector<int32_t> &a = rs.a, &launch = rs.launch;
+        a.resize(M);
+        launch.resize(M);
         for (int p = 0; p < M; p++) a[p] = ord[M - 1 - p];
         std::vector<int32_t> next(kCostBuckets + 1, 0);
         auto bucket = [&](int32_t m) {
@@ -576,60 +972,24 @@ static int decode_core(const PopHeader *h, const int32_t *nt, const float *nv,
         for (int p = 0; p < M; p++) knext[CO_MAX_K - metas[launch[p]].K + 1]++;
         for (int i = 0; i <= CO_MAX_K; i++) knext[i + 1] += knext[i];
         for (int p = 0; p < M; p++) a[knext[CO_MAX_K - metas[launch[p]].K]++] = launch[p];
-        int gpos = 0, fpos = n_gen;
-        for (int p = 0; p < M; p++) launch[gen[a[p]] ? gpos++ : fpos++] = a[p];
-        for (int p = 0; p < M; p++) {
-            const int m = launch[p];
-            ExprDesc &d = descs[p];
-            d.prog_off = (int32_t)(word_base + poff[m]);
-            d.n = nins[m];
-            d.c_off = metas[m].c_offset;
-            d.K = metas[m].K;
-            d.y_row = row_base + m;
-            d.tape = tapes[m];
-            d.slots = slots[m];
-            d.gen = gen[m];
-        }
+        int gpos = 0, fpos = lo.n_gen;
+        for (int p = 0; p < M; p++) launch[lo.gen[a[p]] ? gpos++ : fpos++] = a[p];
+        const auto put = [&](int p0, int p1) {
+            for (int p = p0; p < p1; p++) descs[p] = desc[launch[p]];
+        };
+        chunked(M, M >= 4096 ? lo.nthreads : 1, put, put);
     }
-    if (plan) {
-        plan->M = M;
-        plan->N = h->N;
-        plan->D = h->n_vars;
-        plan->total_nodes = h->total_nodes;
-        plan->total_c = h->total_c;
-        plan->max_tape = max_tape;
-        plan->max_n = max_n;
-        plan->max_slots = max_slots;
-        plan->words = run;
-        plan->n_gen = n_gen;
-    }
+    plan->M = M;
+    plan->N = h->N;
+    plan->D = D;
+    plan->total_nodes = h->total_nodes;
+    plan->total_c = h->total_c;
+    plan->max_rows = max_rows;
+    plan->max_cslots = max_cslots;
+    plan->words = lo.words;
+    plan->vcols = vcols;
+    plan->n_gen = lo.n_gen;
     return CO_OK;
-}
-
-int decode_population(const PopHeader *h, const int32_t *nt, const float *nv,
-                      const int32_t *ci, const TreeMeta *metas, uint64_t *prog,
-                      int32_t *order, int32_t *bin_start, ExprDesc *descs,
-                      int32_t *stack, int32_t *n_ins, int32_t *prog_off, int32_t *route,
-                      Plan *plan) {
-    const int rc = check_header(h, nt, nv, ci, metas);
-    if (rc != CO_OK) return rc;
-    std::vector<uint64_t> tmp;
-    if (!prog) {
-        tmp.assign(h->total_nodes > 0 ? 2 * (size_t)h->total_nodes : 1, 0);
-        prog = tmp.data();
-    }
-    return decode_core(h, nt, nv, ci, metas, h->M_prob, 0, 0, prog, order, bin_start, descs,
-                       stack, n_ins, prog_off, route, plan, 65536);
-}
-
-int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const int32_t *ci,
-                 const TreeMeta *metas, int m0, int m1, int64_t word_base, uint64_t *prog,
-                 ExprDesc *descs, Plan *plan) {
-    // a range is decoded while the device fits the ones before it: more
-    // threads per node than a whole population gets
-    return decode_core(h, nt, nv, ci, metas + m0, m1 - m0, m0, word_base, prog + word_base,
-                       nullptr, nullptr, descs + m0, nullptr, nullptr, nullptr, nullptr, plan,
-                       16384);
 }
 
 }  // namespace cusr

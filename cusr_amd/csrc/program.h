@@ -58,6 +58,7 @@
 //           bits 24..55  tape
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include "../../include/cusr_co.h"
@@ -69,15 +70,61 @@ constexpr int OP_IDENT = 63;
 constexpr int kMaxSlots = 16;                    // fast format (4-bit slot index)
 constexpr int kMaxSlotsWide = CO_MAX_STACK;      // wide format
 
+// The staged program, which the device runs. Of an expression's operators, those
+// over constants alone give the same value at every point, and those over
+// variables alone the same value at every iteration. On the benchmark
+// populations they are a quarter to a third of the operators each (a fifth to
+// 40 % of their cost each), so neither is evaluated per point and pass:
+//   C  the maximal constant-only subtrees, run once per pass with one value per
+//      wavefront: each leaves its value in place of its first constant (rank
+//      lo) and, in forward AD, the tangents of its constants, from which the
+//      per-point rows start instead of from 1;
+//   V  the maximal variable-only subtrees, run in the first pass of a fit:
+//      each value goes to a row of LDS and to a column of the fit's workspace,
+//      which later passes load like an input variable;
+//   M  everything else, run per point and pass; a C subtree is a CONST operand
+//      of it, a V subtree a VAR operand.
+// Every value, tangent and adjoint goes through the operations it went through
+// before, in the same order, so results are bit-identical to the plain program.
+// An expression without constants is one M program.
+//
+// The instructions are the words above with these differences: VAR and SLOT
+// operands and the destination index a row of the wavefront's LDS (variables of
+// M, V values, then a shared tail: V's other variables and slots, M's slots);
+// in C, SLOT operands and destinations index the wavefront's scalar slots, and
+// tape slots the scalar tape. The fast word adds
+//   bit  52      root   C: the subtree's last instruction; M: an operand is a C
+//                       subtree
+//   bits 53..60  cidx   C root: the subtree's instructions; M with root: the C
+//                       instruction of that subtree's root (at most one operand
+//                       of an M operator is a C subtree: with two it were in C)
+// and the wide words are laid out as
+//   word 0: bits  0..5   fid          bit  6 binary
+//           bits  7..8   a_kind       bits  9..20 a_idx
+//           bits 21..27  sel, scale_a, scale_b, tape_a, tape_b, to_slot, root
+//           bits 28..29  b_kind       bits 32..43 b_idx      bits 44..63 cidx
+//   word 1: bits  0..7   lo           bits  8..15 mid        bits 16..23 hi
+//           bits 32..43  d_idx        bits 44..63 tape
+// A wide program is followed by one word per variable row, the variable's index;
+// a fast one has them in ExprDesc.map, four bits each.
 struct ExprDesc {          // one per expression, device-resident
-    int32_t prog_off;      // first program word
-    int32_t n;             // instructions
+    int32_t prog_off;      // first program word: C, then V, then M
+    int32_t n_c, n_v, n_m; // instructions of each
     int32_t c_off;         // constants offset
     int32_t K;             // constants
     int32_t y_row;         // row of ym / output index (original expression index)
-    int32_t tape;          // reverse-mode tape slots
-    int32_t slots;         // spill slots
+    int32_t v_col;         // first workspace column of its V values
+    int32_t mvars;         // rows of variables that M reads
+    int32_t vrows;         // rows of V values
+    int32_t ovars;         // rows of the other variables, that V reads
+    int32_t rows;          // rows in all; forward AD and values
+    int32_t rows_rev;      // rows in all; reverse AD
+    int32_t crow;          // reverse AD: first row of C's adjoint slots
+    int32_t cslots;        // scalar slots of C
+    int32_t ctape;         // scalar reverse-AD tape slots of C
+    int32_t tape;          // reverse-mode tape slots of M
     int32_t gen;           // 1: wide program, general kernel
+    uint64_t map;          // fast: variable index of each variable row
 };
 
 static inline __host__ __device__ int ins_fid(uint64_t w) { return (int)(w & 63u); }
@@ -101,64 +148,76 @@ static inline __host__ __device__ int ins_scale_b(uint64_t w) { return (int)((in
 static inline __host__ __device__ int ins_tape_a(uint64_t w) { return (int)((ins_w1(w) >> 18) & 1u); }
 static inline __host__ __device__ int ins_tape_b(uint64_t w) { return (int)((ins_w1(w) >> 19) & 1u); }
 
-// wide-format fields (word 0 a, word 1 b)
+// wide staged fields (word 0 a, word 1 b), each within one 32-bit half
 struct Wide {
     uint64_t a, b;
 };
-static inline __host__ __device__ int wins_fid(uint64_t a) { return (int)(a & 63u); }
-static inline __host__ __device__ int wins_binary(uint64_t a) { return (int)((a >> 6) & 1u); }
-static inline __host__ __device__ int wins_akind(uint64_t a) { return (int)((a >> 7) & 3u); }
-static inline __host__ __device__ int wins_aidx(uint64_t a) { return (int)((a >> 9) & 255u); }
-static inline __host__ __device__ int wins_bkind(uint64_t a) { return (int)((a >> 17) & 3u); }
-static inline __host__ __device__ int wins_bidx(uint64_t a) { return (int)((a >> 19) & 255u); }
-static inline __host__ __device__ int wins_toslot(uint64_t a) { return (int)((a >> 27) & 1u); }
-static inline __host__ __device__ int wins_didx(uint64_t a) { return (int)((a >> 28) & 255u); }
-static inline __host__ __device__ int wins_sel(uint64_t a) { return (int)((ins_w1(a) >> 4) & 1u); }
-static inline __host__ __device__ int wins_scale_a(uint64_t a) { return (int)((ins_w1(a) >> 5) & 1u); }
-static inline __host__ __device__ int wins_scale_b(uint64_t a) { return (int)((ins_w1(a) >> 6) & 1u); }
-static inline __host__ __device__ int wins_tape_a(uint64_t a) { return (int)((ins_w1(a) >> 7) & 1u); }
-static inline __host__ __device__ int wins_tape_b(uint64_t a) { return (int)((ins_w1(a) >> 8) & 1u); }
-static inline __host__ __device__ int wins_lo(uint64_t b) { return (int)(b & 255u); }
-static inline __host__ __device__ int wins_mid(uint64_t b) { return (int)((b >> 8) & 255u); }
-static inline __host__ __device__ int wins_hi(uint64_t b) { return (int)((b >> 16) & 255u); }
-static inline __host__ __device__ int wins_tape(uint64_t b) { return (int)((b >> 24) & 0xffffffffu); }
+static inline __host__ __device__ int wst_fid(uint64_t a) { return (int)(a & 63u); }
+static inline __host__ __device__ int wst_bit(uint64_t a, int i) { return (int)(((uint32_t)a >> i) & 1u); }
+static inline __host__ __device__ int wst_akind(uint64_t a) { return (int)(((uint32_t)a >> 7) & 3u); }
+static inline __host__ __device__ int wst_aidx(uint64_t a) { return (int)(((uint32_t)a >> 9) & 4095u); }
+static inline __host__ __device__ int wst_bkind(uint64_t a) { return (int)(((uint32_t)a >> 28) & 3u); }
+static inline __host__ __device__ int wst_bidx(uint64_t a) { return (int)(ins_w1(a) & 4095u); }
+static inline __host__ __device__ int wst_cidx(uint64_t a) { return (int)(ins_w1(a) >> 12); }
+static inline __host__ __device__ int wst_lo(uint64_t b) { return (int)((uint32_t)b & 255u); }
+static inline __host__ __device__ int wst_mid(uint64_t b) { return (int)(((uint32_t)b >> 8) & 255u); }
+static inline __host__ __device__ int wst_hi(uint64_t b) { return (int)(((uint32_t)b >> 16) & 255u); }
+static inline __host__ __device__ int wst_didx(uint64_t b) { return (int)(ins_w1(b) & 4095u); }
+static inline __host__ __device__ int wst_tape(uint64_t b) { return (int)(ins_w1(b) >> 12); }
+// Doubles of a wavefront's scalar area (LDS): the constants with C's values in
+// place, the tangents C leaves, C's slots and its reverse-AD tape.
+static inline __host__ __device__ int uni_doubles(int K, int cslots, int ctape) {
+    return 2 * K + cslots + ctape;
+}
+constexpr int kWideCidxMax = (1 << 20) - 1;   // C instructions a wide word can address
+constexpr int kFastRows = 16;                 // rows a fast word can address
 
 struct Plan {
     int32_t M, N, D, total_nodes, total_c;
-    int32_t max_tape, max_n, max_slots;
-    int64_t words;         // program words (fast: 1 per instruction, wide: 2)
+    int32_t max_rows;      // LDS rows of a value pass
+    int32_t max_cslots;
+    int64_t words;         // program words (fast: n_nodes per expression, wide: 2 n_nodes)
+    int64_t vcols;         // workspace columns of the V values
     int32_t n_gen;         // expressions of the general kernel
 };
 
-// Check a population and decode it. Returns a CO_* code. On success fills
-// prog[2 * total_nodes] (expression m's program starts at word prog_off[m]:
-// programs are laid out expression after expression, n_nodes words for the
-// fast format and 2 * n_nodes for the wide one; words past its instructions
-// are 0), order[M] (stable K bins, ascending), bin_start[CO_MAX_K+2],
-// descs[M] (by launch position: the general kernel's bin first, then the fast
-// K bins, largest K first), stack[M] (value-stack depth, by expression),
-// n_ins[M] (instructions per expression), prog_off[M], route[M] (1: general
-// kernel). Any output pointer may be null.
+// Check a population and decode it into plain programs (co_decode). Returns a
+// CO_* code. On success fills prog[2 * total_nodes] (expression m's program
+// starts at word prog_off[m]: programs are laid out expression after
+// expression, n_nodes words for the fast format and 2 * n_nodes for the wide
+// one; words past its instructions are 0), order[M] (stable K bins, ascending),
+// bin_start[CO_MAX_K+2], stack[M] (value-stack depth, by expression),
+// prog_off[M], route[M] (1: general kernel). Any output pointer may be null.
 int decode_population(const PopHeader *h, const int32_t *nt, const float *nv,
                       const int32_t *ci, const TreeMeta *metas, uint64_t *prog,
-                      int32_t *order, int32_t *bin_start, ExprDesc *descs,
-                      int32_t *stack, int32_t *n_ins, int32_t *prog_off, int32_t *route,
-                      Plan *plan);
+                      int32_t *order, int32_t *bin_start, int32_t *stack, int32_t *prog_off,
+                      int32_t *route);
 
-// The header-level checks decode_population makes first: null inputs, device
+// The header-level checks every decode makes first: null inputs, device
 // bounds on K_max / max_stack / n_vars, and the sums of K and of n_nodes.
 int check_header(const PopHeader *h, const int32_t *nt, const float *nv, const int32_t *ci,
                  const TreeMeta *metas);
 
 // Decode expressions [m0, m1) of a population whose header passed
-// check_header, for an upload that decodes a population in pieces: their
-// programs go to prog from word word_base on (the range's layout as
-// decode_population's, its descriptors' prog_off counting from word 0 of
-// prog), their descriptors to descs[m0..m1) in launch order within the range
-// (y_row the population row). plan describes the range (M, words, slots,
-// tape); the same per-expression checks and error codes as decode_population.
+// check_header into staged programs, for an upload of the population as a
+// whole or in pieces: the programs go to prog from word word_base on (laid out
+// expression after expression as above, the descriptors' prog_off counting
+// from word 0 of prog), the descriptors to descs[m0..m1) by launch position
+// within the range (the general kernel's bin first, then the fast K bins,
+// largest K first; y_row the population row, v_col counting from the range's
+// first column). plan describes the range. The same per-expression checks and error codes as
+// decode_population.
 int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const int32_t *ci,
                  const TreeMeta *metas, int m0, int m1, int64_t word_base, uint64_t *prog,
                  ExprDesc *descs, Plan *plan);
+
+// Words that the staged programs of total_nodes nodes take at most.
+static inline size_t staged_words_max(int total_nodes, int n_vars) {
+    return total_nodes > 0 ? (size_t)total_nodes * (n_vars > CO_FAST_MAX_VARS ? 3 : 2) : 1;
+}
+
+// Nodes a decode thread takes at least: waking the pool's threads costs about
+// what one thread decodes in 20 us.
+constexpr int64_t kDecodeNodes = 4096;
 
 }  // namespace cusr
