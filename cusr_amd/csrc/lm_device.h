@@ -895,7 +895,7 @@ __device__ __forceinline__ void const_phase(ProgPtr prog, int n, const UniLds &u
         double t = 0.0;
 #pragma unroll
         for (int j = 0; j < K; ++j) t = lane == j ? (double)T[j] : t;
-        if (lane < K) u.t0[lane] = t;
+        if (lane < Kr) u.t0[lane] = t;
     }
     wave_order_lds();
 }
@@ -1126,9 +1126,8 @@ template <int K, int AD>
 constexpr bool matrix_sums() {
     return AD == CO_AD_FORWARD ? K >= CO_SUMS_MATRIX_MIN_K : K >= CO_SUMS_MATRIX_MIN_K_REV;
 }
-// Reverse AD stages the rows (and the solve's K x K factor) in the tape's LDS:
-// a batch's rows are written after its reverse sweep has read the tape, and
-// the solve runs between passes. Every column the matrix instruction reads
+// Reverse AD stages the rows in the tape's LDS: a batch's rows are written
+// after its reverse sweep has read the tape. Every column the matrix instruction reads
 // (0..15) is rewritten for each batch, the ones past r with zeros.
 template <int K, int AD>
 constexpr bool sums_over_tape() { return AD == CO_AD_REVERSE && matrix_sums<K, AD>(); }
@@ -1549,123 +1548,103 @@ __device__ __forceinline__ bool damp_pivot(double &sj, double lambda, int damp) 
 
 // Damped Cholesky solve of (J^T J + damping) delta = -J^T r from pass sums s
 // (cusr/kernel/batch_lm_ad.cu:149-191) under damping variant damp; false when
-// the pivot rule fails the step. Every lane computes the same result.
-template <int K, bool REL>
-__device__ __forceinline__ bool damped_solve(const double *s, double lambda, int damp,
-                                             double (&delta)[K]) {
-    double L[K][K];
-    double b[K];
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        b[i] = -s[1 + i];
-#pragma unroll
-        for (int j = 0; j <= i; ++j) {
-            // upper-triangle element (j, i): row j starts at j*K - j*(j-1)/2
-            L[i][j] = s[1 + K + j * K - (j * (j - 1)) / 2 + (i - j)];
-        }
-        L[i][i] = damp_diag<REL>(L[i][i], lambda, damp);
-    }
-    bool ok = true;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        double sj = L[j][j];
-#pragma unroll
-        for (int k = 0; k < j; ++k) sj = fma(-L[j][k], L[j][k], sj);
-        if (!damp_pivot<REL>(sj, lambda, damp)) ok = false;
-        const double dj = ::sqrt(sj);
-        L[j][j] = dj;
-#pragma unroll
-        for (int i = j + 1; i < K; ++i) {
-            double t = L[i][j];
-#pragma unroll
-            for (int k = 0; k < j; ++k) t = fma(-L[i][k], L[j][k], t);
-            L[i][j] = t / dj;
-        }
-    }
-    if (!ok) return false;
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-        double t = b[i];
-#pragma unroll
-        for (int k = 0; k < i; ++k) t = fma(-L[i][k], b[k], t);
-        b[i] = t / L[i][i];
-    }
-#pragma unroll
-    for (int i = K - 1; i >= 0; --i) {
-        double t = b[i];
-#pragma unroll
-        for (int k = i + 1; k < K; ++k) t = fma(-L[k][i], b[k], t);
-        b[i] = t / L[i][i];
-    }
-#pragma unroll
-    for (int i = 0; i < K; ++i) delta[i] = b[i];
-    return true;
+// the pivot rule fails the step. KM: the most constants, Kr: the expression's,
+// KL: the K by which s is laid out. x: delta on every lane; mine: entry `lane`.
+//
+// Lane i holds row i of the factor in registers (a[j], j < i; its diagonal in
+// dg, its right-hand side in t), and column k is finished for all rows at once:
+// one square root and one division per column, its entries broadcast from their
+// lanes (v_readlane). Row by row every element still goes through the updates
+// k = 0, 1, ... of the textbook's inner product in that order, and the back
+// substitution through its terms in ascending order, so the bits are those of
+// the scalar algorithm. It replaces the solve unrolled on every lane alike (K(K-1)/2
+// + 2K divisions; at K = 8 a third of a fit pass's vector instructions) and the
+// one with its factor in LDS for larger K, a chain of LDS round trips and waits
+// (16,384 expressions x 1,024 points, K 1-8: 7.67 -> 7.38 ms; 4,000 x 1,000, K 1-28:
+// 37.5 -> 35.9 ms).
+// The entries above the diagonal and the lanes past Kr hold unused values.
+// sched_barrier keeps a column's broadcasts from being scheduled all at once,
+// which overflows the scalar registers.
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
-
-// The same solve with L in LDS, K at run time (the general kernel, and the
-// fast kernels with matrix sums, where K(K+1)/2 doubles per lane of the
-// register version would set the kernel's register count). Every element gets
-// exactly the arithmetic of damped_solve: column j's pivot is computed by
-// every lane, the entries below it by lane i; the substitutions run on every
-// lane with L read by broadcast. The solution is left in L[K*K .. K*K+K).
-template <bool REL>
-__device__ __forceinline__ bool damped_solve_rt(const double *s, double lambda, int damp, int K,
-                                                double *L, int lane) {
-    double *b = L + K * K;   // right-hand side, then the solution (LDS, K doubles)
-    // L[i][j] = upper-triangle element (j, i) of J^T J for j <= i; diagonal damped
-    if (lane < K) {
-        const int i = lane;
-        for (int j = 0; j <= i; ++j) {
-            double v = s[1 + K + j * K - (j * (j - 1)) / 2 + (i - j)];
-            if (j == i) v = damp_diag<REL>(v, lambda, damp);
-            L[i * K + j] = v;
-        }
-        b[i] = -s[1 + i];
-    }
-    wave_sync_lds();
-    bool ok = true;
-#pragma unroll 1
-    for (int j = 0; j < K; ++j) {
-        double sj = L[j * K + j];
-        for (int k = 0; k < j; ++k) sj = fma(-L[j * K + k], L[j * K + k], sj);
-        if (!damp_pivot<REL>(sj, lambda, damp)) ok = false;
-        const double dj = ::sqrt(sj);
-        if (lane > j && lane < K) {
-            const int i = lane;
-            double t = L[i * K + j];
-            for (int k = 0; k < j; ++k) t = fma(-L[i * K + k], L[j * K + k], t);
-            L[i * K + j] = t / dj;
-        }
-        wave_sync_lds();
-        if (lane == j) L[j * K + j] = dj;
-        wave_sync_lds();
-    }
-    if (!ok) return false;
-#pragma unroll 1
-    for (int i = 0; i < K; ++i) {
-        double t = b[i];
-        for (int k = 0; k < i; ++k) t = fma(-L[i * K + k], b[k], t);
-        wave_sync_lds();
-        if (lane == 0) b[i] = t / L[i * K + i];
-        wave_sync_lds();
-    }
-#pragma unroll 1
-    for (int i = K - 1; i >= 0; --i) {
-        double t = b[i];
-        for (int k = i + 1; k < K; ++k) t = fma(-L[k * K + i], b[k], t);
-        wave_sync_lds();
-        if (lane == 0) b[i] = t / L[i * K + i];
-        wave_sync_lds();
-    }
-    return true;
+// v with lane l set to w; the opaque copy of the lane keeps the compiler from
+// holding one 64-bit lane mask per column for all its uses
+__device__ __forceinline__ double with_lane(double v, double w, int l, int lane) {
+    __asm__("" : "+v"(lane));
+    return lane == l ? w : v;
 }
-
-template <int K, bool REL>
-__device__ __forceinline__ bool damped_solve_lds(const double *s, double lambda, int damp,
-                                                 double (&delta)[K], double *L, int lane) {
-    if (!damped_solve_rt<REL>(s, lambda, damp, K, L, lane)) return false;
-#pragma unroll
-    for (int i = 0; i < K; ++i) delta[i] = L[K * K + i];
+template <int B, int E, typename Fn>
+__device__ __forceinline__ void static_for(const Fn &f) {
+    if constexpr (B < E) {
+        f(std::integral_constant<int, B>{});
+        static_for<B + 1, E>(f);
+    }
+}
+template <int KM, bool REL>
+__device__ __forceinline__ bool damped_solve(const double *s, int KL, int Kr, double lambda,
+                                             int damp, int lane, double (&x)[KM], double &mine) {
+    constexpr int GS = 4, NG = (KM + GS - 1) / GS;   // columns behind one test of Kr
+    const int i = lane < Kr ? lane : Kr - 1;
+    const double *row = s + 1 + KL + i;   // entry (j, i) of the upper triangle at j KL - j (j+1) / 2
+    double a[KM];
+    static_for<0, NG>([&](auto g) {
+        if (g * GS < Kr)
+            static_for<g * GS, (g * GS + GS < KM ? g * GS + GS : KM)>(
+                [&](auto j) { a[j] = row[j * KL - (j * (j + 1)) / 2]; });
+    });
+    double dg = damp_diag<REL>(row[i * KL - (i * (i + 1)) / 2], lambda, damp);
+    double t = -s[1 + i];
+    double dv = 1.0, bv = 0.0;   // lane k: the factor's diagonal and the forward solution
+    bool ok = true;
+    static_for<0, KM>([&](auto k) {
+        if (k < Kr && ok) {
+            double sk = lane_value(dg, k);
+            ok = damp_pivot<REL>(sk, lambda, damp);
+            ok = uni((int)ok) != 0;
+            const double dk = ::sqrt(sk);
+            // rows below: L[i][k]; row k: its right-hand side
+            const double q = with_lane(a[k], t, k, lane) / dk;
+            const double bk = lane_value(q, k);
+            a[k] = q;
+            dv = with_lane(dv, dk, k, lane);
+            bv = with_lane(bv, q, k, lane);
+            dg = fma(-q, q, dg);
+            t = fma(-q, bk, t);
+            static_for<(k + 1) / GS, NG>([&](auto g) {
+                if (g * GS < Kr) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    static_for<(g * GS > k ? g * GS : k + 1), (g * GS + GS < KM ? g * GS + GS : KM)>(
+                        [&](auto j) { a[j] = fma(-q, lane_value(q, j), a[j]); });
+                }
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    });
+    if (!ok) return false;
+    mine = 0.0;
+    static_for<0, KM>([&](auto down) {
+        constexpr int r = KM - 1 - down;
+        x[r] = 0.0;
+        if (r < Kr) {
+            double v = lane_value(bv, r);
+            static_for<(r + 1) / GS, NG>([&](auto g) {
+                if (g * GS < Kr) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    static_for<(g * GS > r ? g * GS : r + 1), (g * GS + GS < KM ? g * GS + GS : KM)>(
+                        [&](auto k) {
+                            if (k < Kr) v = fma(-lane_value(a[r], k), x[k], v);
+                        });
+                }
+            });
+            x[r] = v / lane_value(dv, r);
+            mine = with_lane(mine, x[r], r, lane);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    });
     return true;
 }
 
@@ -1760,22 +1739,19 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
                        (double *)my_lds);
     my_lds += fa.uni_bytes;
     double *jt = (double *)my_lds;   // matrix sums: the slice's augmented rows first
-    // then the K x K Cholesky factor and rhs (the general kernel's solve
-    // reuses the rows' bytes: it runs between passes; reverse AD puts both
-    // in the tape's bytes)
+    // (reverse AD puts them in the tape's bytes)
     if constexpr (GEN) {
         my_lds += kGenJtBytes;
     } else if constexpr (matrix_sums<K, AD>() && !sums_over_tape<K, AD>()) {
         // columns K+1.. of every row stay zero for the whole fit
 #pragma unroll
         for (int j = 0; j < kJtStride; ++j) jt[lane * kJtStride + j] = 0.0;
-        my_lds += kJtBytes + (size_t)K * (K + 1) * sizeof(double);
+        my_lds += kJtBytes;
     }
     WaveLds<R, P> wl;
     wl.x = (R *)my_lds;
     wl.tape = wl.x + (size_t)fa.rows * P * kLanes;
     if constexpr (!GEN && sums_over_tape<K, AD>()) jt = (double *)wl.tape;
-    double *lds_l = GEN ? jt : jt + kLanes * kJtStride;
     pa.X = fa.X;
     pa.y = fa.Y + (fa.shared_y ? (size_t)0 : (size_t)e.y_row * fa.N);
     pa.parts = fa.parts;
@@ -1827,21 +1803,11 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     if constexpr (K > 0) {
         while (uni(st) == ST_RUN && it < fa.it_end) {
             ++it;
-            double delta[GEN ? 1 : K];
-            bool solved;
-            if constexpr (GEN)
-                solved = fa.damp == CO_DAMP_RELATIVE
-                             ? damped_solve_rt<true>(s_cur, lambda, 0, Kr, lds_l, lane)
-                             : damped_solve_rt<false>(s_cur, lambda, fa.damp, Kr, lds_l, lane);
-            else if constexpr (matrix_sums<K, AD>())
-                solved = fa.damp == CO_DAMP_RELATIVE
-                             ? damped_solve_lds<K, true>(s_cur, lambda, 0, delta, lds_l, lane)
-                             : damped_solve_lds<K, false>(s_cur, lambda, fa.damp, delta, lds_l,
-                                                          lane);
-            else
-                solved = fa.damp == CO_DAMP_RELATIVE
-                             ? damped_solve<K, true>(s_cur, lambda, 0, delta)
-                             : damped_solve<K, false>(s_cur, lambda, fa.damp, delta);
+            double delta[K], mine;
+            const bool solved =
+                fa.damp == CO_DAMP_RELATIVE
+                    ? damped_solve<K, true>(s_cur, Kr, Kr, lambda, 0, lane, delta, mine)
+                    : damped_solve<K, false>(s_cur, Kr, Kr, lambda, fa.damp, lane, delta, mine);
             if (!solved) {
                 lambda = lambda * 10.0;
                 if (lambda > 1e12) st = ST_CHOL;
@@ -1850,32 +1816,21 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
             // every wavefront is done reading c_try (the norm below) before
             // the lead overwrites it
             if (fa.pwaves > 1) __syncthreads();
+            if (lead && lane < Kr) {
+                const double v = c_cur[lane] + mine;
+                c_try[lane] = fa.f32_range ? (double)(float)v : v;
+            }
+            block_sync(fa.pwaves);
+            // the step norms, before the pass: only their comparison is kept over it
             double dn2 = 0.0, cn2 = 0.0;
-            if constexpr (GEN) {
-                // the solution sits in the rows' bytes, which the pass
-                // overwrites: the step norms are formed before it
-                const double *db = lds_l + Kr * Kr;
-                if (lead && lane < Kr) {
-                    const double v = c_cur[lane] + db[lane];
-                    c_try[lane] = fa.f32_range ? (double)(float)v : v;
-                }
-                block_sync(fa.pwaves);
-                for (int j = 0; j < Kr; ++j) {
-                    dn2 = fma(db[j], db[j], dn2);
+#pragma unroll
+            for (int j = 0; j < K; ++j)
+                if (j < Kr) {
+                    dn2 = fma(delta[j], delta[j], dn2);
                     cn2 = fma(c_try[j], c_try[j], cn2);
                 }
-            } else {
-                if (lead && lane < K) {
-#pragma unroll
-                    for (int j = 0; j < K; ++j) {
-                        if (j == lane) {
-                            const double v = c_cur[j] + delta[j];
-                            c_try[j] = fa.f32_range ? (double)(float)v : v;
-                        }
-                    }
-                }
-                block_sync(fa.pwaves);
-            }
+            const double dn = ::sqrt(dn2), cn = ::sqrt(cn2);
+            const int small = uni((int)(dn < fa.xtol * (cn + fa.xtol)));
             if (fa.f32_range) {
                 // trial constants are held in fp32, as the reference's are; one
                 // beyond the fp32 range makes its trial loss non-finite
@@ -1891,16 +1846,9 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
                 data_pass_gen<R, JAC, F>(pa, wl, c_try, s_try, lane, Kr);
             } else {
                 data_pass<K, R, P, JAC, F>(pa, wl, c_try, s_try, lane);
-#pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    dn2 = fma(delta[j], delta[j], dn2);
-                    cn2 = fma(c_try[j], c_try[j], cn2);
-                }
             }
             const double loss_try = uni(0.5 * s_try[0]);
             if (!loss_ok(fa, loss_try)) { st = ST_NAN; continue; }
-            const double dn = ::sqrt(dn2), cn = ::sqrt(cn2);
-            const bool small = dn < fa.xtol * (cn + fa.xtol);
             bool accept, conv;
             if (fa.lm_order == CO_ORDER_CONVERGE_FIRST) {
                 // FD variant (co_lib.cu:457-473): a small step converges
@@ -2069,7 +2017,7 @@ constexpr size_t fit_static_lds(int bin) {
 template <typename R, int K, int AD, int LN = 0>
 constexpr size_t fit_lds_bytes_t(int rows, int tape) {
     const size_t row = (size_t)points_per_pass<R, K, AD, LN>() * kLanes * sizeof(R);
-    const size_t mx = matrix_sums<K, AD>() ? kJtBytes + (size_t)K * (K + 1) * sizeof(double) : 0;
+    const size_t mx = matrix_sums<K, AD>() ? kJtBytes : 0;
     const size_t t = sums_over_tape<K, AD>() && mx > (size_t)tape * row ? mx : (size_t)tape * row;
     const size_t a = (size_t)rows * row + t;
     const size_t b = (size_t)rows * audit_points<R, K, AD, LN>() * kLanes * sizeof(double);

@@ -91,7 +91,7 @@ lm_pass_kernel(FitArgs fa) {
     } else if constexpr (matrix_sums<K, AD>()) {
 #pragma unroll
         for (int j = 0; j < kJtStride; ++j) jt[lane * kJtStride + j] = 0.0;
-        my_lds += kJtBytes + (size_t)K * (K + 1) * sizeof(double);
+        my_lds += kJtBytes;
     }
     pa.X = fa.X;
     pa.y = fa.Y + (fa.shared_y ? (size_t)0 : (size_t)e.y_row * fa.N);
@@ -126,16 +126,13 @@ lm_pass_kernel(FitArgs fa) {
 // One LM step of one expression (a wavefront): the G partition sums of its
 // pending pass added in partition order, then fit_one's decisions. The state
 // row is worked on in LDS and written back.
-// KS > 0: every expression of the launch has K = KS (a fast kernel's bin), and
-// the solve is damped_solve<KS>, unrolled in registers; KS = 0: the runtime-K
-// solve in LDS (the general bin). Both give the same bits; the unrolled one has
-// no chain of LDS round trips (C3's step launches: the solves of K <= 16).
+// KS > 0: every expression of the launch has K = KS (a fast kernel's bin); KS = 0:
+// K at run time (the general bin, K = 0).
 template <int KS>
 __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) {
     __shared__ double s_new[sums_width(CO_MAX_K)];
     __shared__ double s_cur[sums_width(CO_MAX_K)];
     __shared__ double c_cur[CO_MAX_K], c_try[CO_MAX_K];
-    __shared__ double L[CO_MAX_K * CO_MAX_K + CO_MAX_K];
     const int idx = blockIdx.x;
     const int lane = (int)threadIdx.x;
     const ExprDesc e = fa.desc[idx];
@@ -222,37 +219,28 @@ __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) 
         double dn = 0.0, cn = 0.0;
         while (st == ST_RUN && it < fa.max_iter) {
             ++it;
-            bool solved;
-            if constexpr (KS > 0) {
-                double delta[KS];
-                solved = fa.damp == CO_DAMP_RELATIVE
-                             ? damped_solve<KS, true>(s_cur, lambda, 0, delta)
-                             : damped_solve<KS, false>(s_cur, lambda, fa.damp, delta);
-                if (solved && lane == 0) {
-#pragma unroll
-                    for (int j = 0; j < KS; ++j) L[KS * KS + j] = delta[j];
-                }
-                wave_sync_lds();
-            } else {
-                solved = fa.damp == CO_DAMP_RELATIVE
-                             ? damped_solve_rt<true>(s_cur, lambda, 0, K, L, lane)
-                             : damped_solve_rt<false>(s_cur, lambda, fa.damp, K, L, lane);
-            }
+            constexpr int KM = KS > 0 ? KS : CO_MAX_K;
+            double delta[KM], mine;
+            const bool solved =
+                fa.damp == CO_DAMP_RELATIVE
+                    ? damped_solve<KM, true>(s_cur, K, K, lambda, 0, lane, delta, mine)
+                    : damped_solve<KM, false>(s_cur, K, K, lambda, fa.damp, lane, delta, mine);
             if (!solved) {
                 lambda = lambda * 10.0;
                 if (lambda > 1e12) st = ST_CHOL;
                 continue;
             }
-            const double *db = L + K * K;
             if (lane < K) {
-                const double v = c_cur[lane] + db[lane];
+                const double v = c_cur[lane] + mine;
                 c_try[lane] = fa.f32_range ? (double)(float)v : v;
             }
             wave_sync_lds();
             double dn2 = 0.0, cn2 = 0.0;
             int over = 0;
-            for (int j = 0; j < K; ++j) {
-                dn2 = fma(db[j], db[j], dn2);
+#pragma unroll
+            for (int j = 0; j < KM; ++j) {
+                if (j >= K) break;
+                dn2 = fma(delta[j], delta[j], dn2);
                 cn2 = fma(c_try[j], c_try[j], cn2);
                 over |= !isfinite(c_try[j]) ? 1 : 0;
             }
