@@ -127,7 +127,7 @@ def build(jobs: int | None = None, verbose: bool = False, defines=(), out: Path 
     jobs = jobs or min(8, os.cpu_count() or 4)
     compiles = []
     for rtype, ad, name in FIT_VARIANTS:
-        for kind, part in [(k, p) for p in (2, 1, 0) for k in ("fit", "pass")]:
+        for kind, part in [(k, p) for p in (2, 1, 3, 0) for k in ("fit", "pass")]:
             obj = bdir / f"fit_{kind}_{name}_{part}.o"
             compiles.append([HIPCC, *flags, *extra, REMARKS, "-x", "hip",
                              f"-DCUSR_FIT_R={rtype}", f"-DCUSR_FIT_AD={ad}",

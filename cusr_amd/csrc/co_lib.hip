@@ -93,6 +93,8 @@ struct HostBuf {
 // (C2: 20.5 ms, the sum of the two streams' bins). So four streams in all.
 constexpr int kExtraStreams = 3;
 constexpr int kStreams = kExtraStreams + 1;
+// wavefronts of a K bin below which bins are grouped (in-workgroup, split path)
+constexpr int kGroupWaves = 1024, kGroupWavesSplit = 4096;
 constexpr int kMaxRanges = 2;   // launch ranges of one fit (the upload pipeline's two)
 
 // launchers per (precision, AD mode) come from fit_kernels.hip, each variant
@@ -124,7 +126,7 @@ struct Ctx {
     // per bin and launch range (a pipelined co_optimize launches each bin once
     // per range): a bin's time is the sum of its launches' durations
     hipEvent_t ev_b0[kMaxRanges][CO_BINS] = {}, ev_b1[kMaxRanges][CO_BINS] = {};
-    bool bin_launched[kMaxRanges][CO_BINS] = {};
+    uint32_t launched[kMaxRanges][CO_BINS] = {};   // the bins of the launch timed there
     Plan plan = {};
     bool resident = false;
     std::vector<int> ranges;   // launch-order ranges of the resident descriptors: [r[i], r[i+1])
@@ -443,6 +445,8 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
 // anything is launched, so a launch that cannot fit is refused up front).
 struct LaunchPlan {
     int bin, pos, cnt, rows, tape, uni, kmax, stream;   // uni: doubles of the scalar area
+    uint32_t bins;   // the bins it covers, bit by bit (a group: several)
+    bool group;      // run by the padded kernel of group_top
     size_t wave_bytes;
     int pwaves[2];
     size_t lds[2];
@@ -463,8 +467,22 @@ template <int KS>
 static void launch_step_k(unsigned n, hipStream_t s, const FitArgs &fa, int mixed) {
     lm_step_kernel<KS><<<n, kLanes, 0, s>>>(fa, mixed);
 }
-static void launch_step(int bin, unsigned n, hipStream_t s, const FitArgs &fa, int mixed) {
+static void launch_step(int bin, bool group, unsigned n, hipStream_t s, const FitArgs &fa,
+                        int mixed) {
     static_assert(CO_FAST_MAX_K == 16, "one step instance per fast K");
+    if (group) {
+        constexpr int kFwd = group_top(9, false), kRev = group_top(9, true);
+        static_assert(kFwd != kRev && kFwd > 8 && kFwd < 15 && kRev > 8 && kRev < 15,
+                      "one step instance per group");
+        switch (bin) {
+        case 4: lm_step_kernel<4, true><<<n, kLanes, 0, s>>>(fa, mixed); break;
+        case 8: lm_step_kernel<8, true><<<n, kLanes, 0, s>>>(fa, mixed); break;
+        case kFwd: lm_step_kernel<kFwd, true><<<n, kLanes, 0, s>>>(fa, mixed); break;
+        case kRev: lm_step_kernel<kRev, true><<<n, kLanes, 0, s>>>(fa, mixed); break;
+        default: lm_step_kernel<15, true><<<n, kLanes, 0, s>>>(fa, mixed); break;
+        }
+        return;
+    }
     switch (bin) {
     case 1: launch_step_k<1>(n, s, fa, mixed); break;
     case 2: launch_step_k<2>(n, s, fa, mixed); break;
@@ -494,6 +512,7 @@ struct FitRun {
     CoOptions opt = {};
     FitArgs fa = {};
     bool rev = false, mixed = false, split = false, started = false;
+    bool group = true;   // small bins may be launched in groups
     int parts = 0, nseg = 1, pwidth = 0;
     Segment seg[2] = {};
     bool lane_used[kExtraStreams] = {};
@@ -519,7 +538,7 @@ struct FitRun {
         const Plan &plan = ctx->plan;
         ctx->last_kernel_ms = 0.0;
         for (int k = 0; k < CO_BINS; ++k) {
-            for (int r = 0; r < kMaxRanges; ++r) ctx->bin_launched[r][k] = false;
+            for (int r = 0; r < kMaxRanges; ++r) ctx->launched[r][k] = 0;
             ctx->last_bin_ms[k] = -1.0;
         }
         parts = co_partitions_resolve(&opt, plan.N);
@@ -581,15 +600,27 @@ struct FitRun {
     // dealt over the other three (a GP-generation population, a fifth of it
     // general: the fast bins dealt behind it on stream 0 had waited for it,
     // 74.6 ms per fit against the general bin's 45 ms).
+    // Bins too small to fill the chip four at a time are launched in groups
+    // (group_top), by the padded kernel of the group's largest K: queued behind
+    // each other, every bin waits for the slowest expression of the one before.
+    // Measured, one launch per bin -> groups: 700 x 777 reverse AD, K 2-14: 14.2
+    // -> 5.0 ms; 24 x 1,000,003: 12.3 -> 5.0 ms; 1,000 x 1,000, K 0-8: 2.67 -> 1.77
+    // ms; 4,000 x 1,000, K 1-28: 35.9 -> 29.6 ms. Larger bins keep their own
+    // kernels, with fewer registers and no padded sums: at 2,000 wavefronts a bin
+    // 4.24 ms against 4.60 grouped (K 1-8, N = 1,024), at 1,000 equal. On the split
+    // path every launch waits for all of the one before, pass and step in turn, so
+    // groups pay for longer: 1,024 x 100,000 (2,048 a bin) 27.2 -> 22.0 ms, 3,000 x
+    // 2,048 reverse AD (1,850) 26.5 -> 24.8 ms, 8,192 x 2,048 (5,040) 66.9 against
+    // 68.6 grouped.
     int plan_range(int p0, int p1, LaunchPlan *lp, int *nl_out, int *kmax_out) const {
         const Plan &plan = ctx->plan;
-        int nl = 0, kmax = 0, pos = p0;
-        bool gen_alone = false;
+        int nl = 0, kmax = 0, pos = p0, fast = 0, fast_bins = 0;
         for (int i = 0; i < CO_BINS; ++i) {
             const int bin = i == 0 ? CO_GENERAL_BIN : CO_FAST_MAX_K - (i - 1);
             const bool gen = bin == CO_GENERAL_BIN;
             LaunchPlan b = {};
             b.bin = bin;
+            b.bins = 1u << bin;
             b.pos = pos;
             while (pos < p1 && (gen ? ctx->h_desc[pos].gen != 0
                                     : (!ctx->h_desc[pos].gen && ctx->h_desc[pos].K == bin))) {
@@ -605,17 +636,53 @@ struct FitRun {
             }
             if (b.cnt == 0) continue;
             if (!rev) b.tape = 0;
+            if (!gen) {
+                fast += b.cnt;
+                ++fast_bins;
+            }
+            lp[nl++] = b;
+        }
+        if (pos != p1) return CO_ERR_PROGRAM;   // descriptors out of launch order: never
+        if (group && nseg == 1 && (long)fast * parts < (long)fast_bins * (split ? kGroupWavesSplit : kGroupWaves)) {
+            int n = 0;
+            for (int i = 0; i < nl; ++i) {
+                const LaunchPlan b = lp[i];
+                const int top = b.bin == CO_GENERAL_BIN ? -1 : group_top(b.bin, rev);
+                if (n > 0 && top >= 0 && lp[n - 1].bin != CO_GENERAL_BIN &&
+                    group_top(lp[n - 1].bin, rev) == top) {
+                    LaunchPlan &g = lp[n - 1];
+                    g.bin = top;
+                    g.group = true;
+                    g.bins |= b.bins;
+                    g.cnt += b.cnt;
+                    g.rows = g.rows > b.rows ? g.rows : b.rows;
+                    g.tape = g.tape > b.tape ? g.tape : b.tape;
+                    g.uni = g.uni > b.uni ? g.uni : b.uni;
+                    g.kmax = top;
+                } else {
+                    lp[n++] = b;
+                }
+            }
+            nl = n;
+        }
+        bool gen_alone = false;
+        for (int i = 0; i < nl; ++i) {
+            LaunchPlan &b = lp[i];
+            const bool gen = b.bin == CO_GENERAL_BIN;
             if (b.kmax > kmax) kmax = b.kmax;
             if (gen) gen_alone = (long)b.cnt * 16 >= (long)(p1 - p0) && b.cnt < p1 - p0;
-            b.stream = !gen_alone ? nl % kStreams : (gen ? 0 : 1 + (nl - 1) % (kStreams - 1));
+            // the handle's own stream first: a fit of one launch waits for no other
+            const int lane = !gen_alone ? i % kStreams : (gen ? 0 : 1 + (i - 1) % (kStreams - 1));
+            b.stream = (lane + kExtraStreams) % kStreams;
             // per-wavefront areas, then the partition sums; fewer wavefronts per
             // workgroup (each summing several partitions) when LDS is short. The
             // split path's pass workgroups are one wavefront with no partition
             // sums in LDS.
-            b.wave_bytes = uni_bytes(b) + ((fit_lds_bytes(mixed, rev, bin, plan.N, b.rows, b.tape) +
+            const int N = b.group ? 0 : plan.N;   // a group has no large-N instance
+            b.wave_bytes = uni_bytes(b) + ((fit_lds_bytes(mixed, rev, b.bin, N, b.rows, b.tape) +
                                             15) & ~(size_t)15);
-            const size_t cap = max_dyn_lds(ctx, bin);
-            const int ks = gen ? b.kmax : bin;
+            const size_t cap = max_dyn_lds(ctx, b.bin);
+            const int ks = gen ? b.kmax : b.bin;
             for (int g = 0; g < (b.kmax == 0 || split ? 1 : nseg); ++g) {
                 const int sp = split ? 1 : seg[g].parts;
                 const size_t part_bytes = sp > 1 ? (size_t)sp * sums_width(ks) * 8 : 0;
@@ -625,9 +692,7 @@ struct FitRun {
                 b.lds[g] = pw * b.wave_bytes + part_bytes;
                 if (b.lds[g] > cap) return CO_ERR_BOUNDS;   // before any launch
             }
-            lp[nl++] = b;
         }
-        if (pos != p1) return CO_ERR_PROGRAM;   // descriptors out of launch order: never
         *nl_out = nl;
         *kmax_out = kmax;
         return CO_OK;
@@ -727,8 +792,8 @@ struct FitRun {
                 fk.it_end = opt.max_iter;
                 fk.resume = 0;
                 for (int r = 0; r < rounds; ++r) {
-                    CO_LAUNCH_HIP(launch_pass[part_of_bin(b.bin)](b.bin, (unsigned)b.cnt * parts, b.lds[0], ks, fk));
-                    launch_step(b.bin, (unsigned)b.cnt, ks, fk, mixed ? 1 : 0);
+                    CO_LAUNCH_HIP(launch_pass[part_of_bin(b.bin, b.group)](b.bin, (unsigned)b.cnt * parts, b.lds[0], ks, fk));
+                    launch_step(b.bin, b.group, (unsigned)b.cnt, ks, fk, mixed ? 1 : 0);
                     CO_LAUNCH_HIP(hipGetLastError());
                 }
             } else {
@@ -745,11 +810,11 @@ struct FitRun {
                     fk.wave_bytes = (int)b.wave_bytes;
                     fk.it_end = seg[g].it_end;
                     fk.resume = seg[g].resume;
-                    CO_LAUNCH_HIP(launch[part_of_bin(b.bin)](b.bin, (unsigned)b.cnt, b.lds[g], ks, fk));
+                    CO_LAUNCH_HIP(launch[part_of_bin(b.bin, b.group)](b.bin, (unsigned)b.cnt, b.lds[g], ks, fk));
                 }
             }
             CO_LAUNCH_HIP(hipEventRecord(ctx->ev_b1[range][b.bin], ks));
-            ctx->bin_launched[range][b.bin] = true;
+            ctx->launched[range][b.bin] = b.bins;
         }
         ++range;
         return CO_OK;
@@ -808,13 +873,15 @@ struct FitRun {
         CO_HIP(hipEventElapsedTime(&ms, ctx->ev_t0, ctx->ev_t1));
         ctx->last_kernel_ms = ms;
         for (int k = 0; k < CO_BINS; ++k) {
-            double sum = -1.0;
             for (int r = 0; r < kMaxRanges; ++r) {
-                if (!ctx->bin_launched[r][k]) continue;
+                if (!ctx->launched[r][k]) continue;
                 CO_HIP(hipEventElapsedTime(&ms, ctx->ev_b0[r][k], ctx->ev_b1[r][k]));
-                sum = (sum < 0.0 ? 0.0 : sum) + ms;
+                for (int i = 0; i < CO_BINS; ++i) {
+                    if (!(ctx->launched[r][k] >> i & 1)) continue;
+                    double &sum = ctx->last_bin_ms[i];
+                    sum = (sum < 0.0 ? 0.0 : sum) + ms;
+                }
             }
-            ctx->last_bin_ms[k] = sum;
         }
         return CO_OK;
     }
@@ -838,15 +905,23 @@ int run_fit(Ctx *ctx, const CoOptions &opt, double *c_out, int32_t *status_out, 
     const int nr = (int)ctx->ranges.size() - 1;
     std::vector<LaunchPlan> lp((size_t)nr * CO_BINS);
     std::vector<int> nl(nr, 0);
-    int kmax = 0;
-    for (int r = 0; r < nr; ++r) {
-        int km = 0;
-        rc = fr.plan_range(ctx->ranges[r], ctx->ranges[r + 1], lp.data() + (size_t)r * CO_BINS,
-                           &nl[r], &km);
-        if (rc != CO_OK) return rc;
-        if (km > kmax) kmax = km;
+    const auto plan = [&] {
+        int kmax = 0;
+        for (int r = 0; r < nr; ++r) {
+            int km = 0;
+            const int e = fr.plan_range(ctx->ranges[r], ctx->ranges[r + 1],
+                                        lp.data() + (size_t)r * CO_BINS, &nl[r], &km);
+            if (e != CO_OK) return e;
+            if (km > kmax) kmax = km;
+        }
+        return fr.set_scratch(kmax, sc);
+    };
+    rc = plan();
+    if (rc == CO_ERR_BOUNDS || rc == CO_ERR_OOM) {
+        // groups of bins lay their sums out by their largest K
+        fr.group = false;
+        rc = plan();
     }
-    rc = fr.set_scratch(kmax, sc);
     if (rc != CO_OK) return rc;
     for (int r = 0; r < nr; ++r) {
         rc = fr.issue(lp.data() + (size_t)r * CO_BINS, nl[r]);

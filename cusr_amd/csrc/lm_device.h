@@ -1724,14 +1724,17 @@ constexpr int fit_audit_points() {
     else return audit_points<R, K, AD, LN>();
 }
 
-template <int K, typename R, int AD, int LN, bool GEN = false>
+// PAD: expressions of fewer constants than K run in K's kernel (group_top): the
+// tangents, sums and solve of the entries past theirs are formed and not read.
+template <int K, typename R, int AD, int LN, bool GEN = false, bool PAD = false>
 __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, double *lds_c, double *lds_s,
                         char *lds_dyn, int lane, int wave) {
     typedef typename std::conditional<GEN, WideFmt, FastFmt>::type F;
     constexpr int P = fit_points<GEN, R, K, AD, LN>();
     constexpr int JAC = (K == 0) ? 0 : (AD == CO_AD_REVERSE ? 2 : 1);
     constexpr int KC = FitStatic<GEN, K>::KC;
-    const int Kr = GEN ? e.K : K;   // the expression's K (wave-uniform)
+    const int Kr = (GEN || PAD) ? e.K : K;   // the expression's K (wave-uniform)
+    const int KL = GEN ? Kr : K;             // the K by which its sums are laid out
     char *my_lds = lds_dyn + (size_t)wave * fa.wave_bytes;
     const bool lead = wave == 0;     // the wavefront that writes shared state
     PassArgs pa;
@@ -1806,8 +1809,8 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
             double delta[K], mine;
             const bool solved =
                 fa.damp == CO_DAMP_RELATIVE
-                    ? damped_solve<K, true>(s_cur, Kr, Kr, lambda, 0, lane, delta, mine)
-                    : damped_solve<K, false>(s_cur, Kr, Kr, lambda, fa.damp, lane, delta, mine);
+                    ? damped_solve<K, true>(s_cur, KL, Kr, lambda, 0, lane, delta, mine)
+                    : damped_solve<K, false>(s_cur, KL, Kr, lambda, fa.damp, lane, delta, mine);
             if (!solved) {
                 lambda = lambda * 10.0;
                 if (lambda > 1e12) st = ST_CHOL;
@@ -1977,7 +1980,7 @@ constexpr bool large_n_variant() {
     return points_per_pass<R, K, AD, 1>() != points_per_pass<R, K, AD, 0>() ||
            waves_per_eu<R, K, AD, 1>() != waves_per_eu<R, K, AD, 0>();
 }
-template <int K, typename R, int AD, int LN = 0>
+template <int K, typename R, int AD, int LN = 0, bool PAD = false>
 __global__ void __launch_bounds__(kLanes * CO_MAX_PARTITIONS, (waves_per_eu<R, K, AD, LN>()))
 lm_fit_kernel(FitArgs fa) {
     __shared__ double lds_c[2 * FitStatic<false, K>::KC];
@@ -1986,7 +1989,7 @@ lm_fit_kernel(FitArgs fa) {
     const ExprDesc e = fa.desc[blockIdx.x];
     const int lane = (int)threadIdx.x & (kLanes - 1);
     const int wave = uni((int)threadIdx.x >> 6);
-    fit_one<K, R, AD, LN>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
+    fit_one<K, R, AD, LN, false, PAD>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
 }
 
 // The general kernel: runtime K <= CO_MAX_K, wide programs, one point per
@@ -2004,6 +2007,15 @@ lm_fit_gen_kernel(FitArgs fa) {
     const int lane = (int)threadIdx.x & (kLanes - 1);
     const int wave = uni((int)threadIdx.x >> 6);
     fit_one<kGenK, R, AD, 0, true>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
+}
+
+// The K whose kernel runs a group of bins in one launch, padded: the largest of
+// 0..4, 5..8, or of the larger K with per-lane sums, with matrix sums (K = 16,
+// whose sums differ, stands alone). Sums of one kind only, so that every entry
+// keeps its order.
+constexpr int group_top(int K, bool rev) {
+    const int lane_top = (rev ? CO_SUMS_MATRIX_MIN_K_REV : CO_SUMS_MATRIX_MIN_K) - 1;
+    return K <= 4 ? 4 : K <= 8 ? 8 : K <= lane_top ? lane_top : K <= 15 ? 15 : 16;
 }
 
 // Static LDS bytes of a bin's fit kernel (kept out of the dynamic budget).
@@ -2034,15 +2046,19 @@ constexpr size_t fit_lds_bytes_gen(int rows, int tape) {
 
 // Launch the fit or pass kernel of one bin (k <= CO_FAST_MAX_K: the fast kernel
 // of K = k; CO_GENERAL_BIN: the general kernel) for one (precision, AD mode).
-// fit_kernels.hip defines a launcher for each part of the bins (part_of_bin).
+// fit_kernels.hip defines a launcher for each part of the bins (part_of_bin); the
+// last part takes a group of bins (group_top) by its largest K.
 typedef hipError_t (*Launcher)(int bin, unsigned grid, size_t lds, hipStream_t s, const FitArgs &fa);
-constexpr int kParts = 3;
-constexpr int part_of_bin(int bin) { return bin <= 4 ? 0 : bin <= 8 ? 1 : 2; }
+constexpr int kParts = 4;
+constexpr int part_of_bin(int bin, bool group) {
+    return group ? 3 : bin <= 4 ? 0 : bin <= 8 ? 1 : 2;
+}
 #define CUSR_DECLARE_LAUNCHER(name)                                                  \
     hipError_t name##_0(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
     hipError_t name##_1(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
     hipError_t name##_2(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
-    constexpr Launcher name[kParts] = {name##_0, name##_1, name##_2}
+    hipError_t name##_3(int, unsigned, size_t, hipStream_t, const FitArgs &);        \
+    constexpr Launcher name[kParts] = {name##_0, name##_1, name##_2, name##_3}
 CUSR_DECLARE_LAUNCHER(launch_fit_f64_fwd);
 CUSR_DECLARE_LAUNCHER(launch_fit_f64_rev);
 CUSR_DECLARE_LAUNCHER(launch_fit_f32_fwd);

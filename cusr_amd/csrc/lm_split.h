@@ -54,7 +54,7 @@ __global__ void __launch_bounds__(kLanes) lm_split_init_kernel(FitArgs fa) {
 // launch's expression b / G. SP_INIT and SP_TRIAL are Jacobian passes at
 // c_try (value only for K = 0); the audits are fp64 value passes at c_cur and
 // c_init.
-template <int K, typename R, int AD, int LN, bool GEN>
+template <int K, typename R, int AD, int LN, bool GEN, bool PAD = false>
 __global__ void __launch_bounds__(kLanes, (GEN ? CUSR_WAVES_GEN : pass_waves_per_eu<R, (GEN ? 0 : K), AD, LN>()))
 lm_pass_kernel(FitArgs fa) {
     typedef typename std::conditional<GEN, WideFmt, FastFmt>::type F;
@@ -72,7 +72,7 @@ lm_pass_kernel(FitArgs fa) {
     const double *sv = fa.state + (size_t)e.y_row * fa.state_stride;
     const int kind = (int)uni(sv[kSpPending]);
     if (kind == SP_NONE) return;
-    const int Kr = GEN ? e.K : K;
+    const int Kr = (GEN || PAD) ? e.K : K;
     const double *src = kind == SP_AUDIT_INIT ? fa.C0 + e.c_off
                         : (kind == SP_AUDIT_CUR ? sv + kSpCCur : sv + kSpCTry);
     if (lane < Kr) cs[lane] = src[lane];
@@ -126,9 +126,10 @@ lm_pass_kernel(FitArgs fa) {
 // One LM step of one expression (a wavefront): the G partition sums of its
 // pending pass added in partition order, then fit_one's decisions. The state
 // row is worked on in LDS and written back.
-// KS > 0: every expression of the launch has K = KS (a fast kernel's bin); KS = 0:
-// K at run time (the general bin, K = 0).
-template <int KS>
+// KS > 0: every expression of the launch has K = KS (a fast kernel's bin), or, with
+// PAD, at most KS (a group of bins, its sums laid out by KS); KS = 0: K at run time
+// (the general bin, K = 0).
+template <int KS, bool PAD = false>
 __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) {
     __shared__ double s_new[sums_width(CO_MAX_K)];
     __shared__ double s_cur[sums_width(CO_MAX_K)];
@@ -139,10 +140,10 @@ __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) 
     double *sv = fa.state + (size_t)e.y_row * fa.state_stride;
     const int kind = (int)uni(sv[kSpPending]);
     if (kind == SP_NONE) return;
-    const int K = KS > 0 ? KS : e.K;
+    const int K = (KS > 0 && !PAD) ? KS : e.K, KL = KS > 0 ? KS : K;
     const int G = fa.parts;
     const bool audit = kind == SP_AUDIT_CUR || kind == SP_AUDIT_INIT;
-    const int W = (audit || K == 0) ? 1 : sums_width(K);
+    const int W = (audit || K == 0) ? 1 : sums_width(KL);
     const double *ps = fa.psum + (size_t)idx * G * fa.psum_width;
     for (int q = lane; q < W; q += kLanes) {
         double v = ps[q];
@@ -223,8 +224,8 @@ __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) 
             double delta[KM], mine;
             const bool solved =
                 fa.damp == CO_DAMP_RELATIVE
-                    ? damped_solve<KM, true>(s_cur, K, K, lambda, 0, lane, delta, mine)
-                    : damped_solve<KM, false>(s_cur, K, K, lambda, fa.damp, lane, delta, mine);
+                    ? damped_solve<KM, true>(s_cur, KL, K, lambda, 0, lane, delta, mine)
+                    : damped_solve<KM, false>(s_cur, KL, K, lambda, fa.damp, lane, delta, mine);
             if (!solved) {
                 lambda = lambda * 10.0;
                 if (lambda > 1e12) st = ST_CHOL;

@@ -412,7 +412,8 @@ int co_last_kernel_ms(void *handle, double *fit_ms_out);
 /* Per-launch device time of the last fit: bin_ms_out[k] (CO_BINS entries)
  * is the duration of the fit launches of bin k (k <= CO_FAST_MAX_K: the fast
  * kernel of K = k; CO_GENERAL_BIN: the general kernel), from HIP events
- * recorded around them on the stream they ran on; -1 for bins with no
+ * recorded around them on the stream they ran on (bins launched together: of
+ * their common launch); -1 for bins with no
  * expressions. No counterpart in the reference (measurement only). */
 int co_last_bin_ms(void *handle, double *bin_ms_out);
 
