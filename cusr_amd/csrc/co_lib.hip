@@ -216,8 +216,7 @@ int grow_needed(Ctx *ctx, DevBuf &b, size_t bytes) {
         if (r_ != CO_OK) return r_;                    \
     } while (0)
 
-// The workspace of range r for `cols` columns of N values (fp64; fp32 fits use
-// half of it), grown with a quarter of headroom and kept. ctx->v_ptr[r] stays
+// The workspace of range r for `cols` columns of N values of 8 bytes, grown with a quarter of headroom and kept. ctx->v_ptr[r] stays
 // null, and no error is returned, where it would pass v_max or does not fit.
 void set_vwork(Ctx *ctx, int r, int64_t cols, int N) {
     DevBuf &b = ctx->vwork[r];

@@ -117,7 +117,9 @@ lm_pass_kernel(FitArgs fa) {
         WaveLds<double, AP> w64;
         w64.x = (double *)my_lds;
         w64.tape = w64.x + (size_t)fa.rows * AP * kLanes;
-        pa.vmode = V_RUN;   // the workspace holds the fit's fp32 values
+        // the first audit keeps V's fp64 values for the second, over the fit's
+        // fp32 ones
+        pa.vmode = !pa.V ? V_RUN : kind == SP_AUDIT_CUR ? V_KEEP : V_LOAD;
         data_pass<KA, double, AP, 0, F>(pa, w64, cs, nullptr, lane);
     }
 }
