@@ -45,9 +45,11 @@ constexpr float kCexpCap32 = 485165184.0f;         // exp(20) rounded to float
 // Points per lane per interpreter pass: more amortises the scalar fetch and
 // dispatch, fewer keeps registers (the J^T J sums dominate for large K) and
 // the reverse-AD tape in LDS small.
-// Per-K tables for fp64 forward AD, K = 0..16 (overridable for tuning).
+// Per-K tables for fp64 forward AD, K = 0..16 (overridable for tuning). Two points
+// per lane from K = 9 (one before: with the solve out of every lane's registers
+// the second point's tangents fit; 4,000 x 1,000, K 1-28: 27.9 -> 26.3 ms).
 #ifndef CUSR_P64_TABLE
-#define CUSR_P64_TABLE 4, 4, 4, 4, 4, 4, 4, 4, 4, 1, 1, 1, 1, 1, 1, 1, 1
+#define CUSR_P64_TABLE 4, 4, 4, 4, 4, 4, 4, 4, 4, 2, 2, 2, 2, 2, 2, 2, 2
 #endif
 #ifndef CUSR_P32_TABLE
 #define CUSR_P32_TABLE 4, 4, 4, 4, 4, 4, 4, 4, 4, 2, 2, 2, 2, 2, 2, 2, 2
@@ -58,10 +60,11 @@ constexpr float kCexpCap32 = 485165184.0f;         // exp(20) rounded to float
 // fp64 forward AD from kLargeN points on (C4's N = 100,000): each pass streams
 // y from memory, and two points per lane with three waves per SIMD hide the
 // loads better (C4 on the split path: 187 -> 179.5 ms with every K = 1..8 so,
-// against K = 5, 6 only; at N = 1,024 four points measured faster). Points per
-// pass do not change any summation order.
+// against K = 5, 6 only; at N = 1,024 four points measured faster; with the staged
+// programs again: 6,000 expressions x 70,000 44.7 ms against 46.2 with four points
+// and two waves). Points per pass do not change any summation order.
 #ifndef CUSR_P64_LARGE_N_TABLE
-#define CUSR_P64_LARGE_N_TABLE 2, 2, 2, 2, 2, 2, 2, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1
+#define CUSR_P64_LARGE_N_TABLE 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2, 2
 #endif
 constexpr int kLargeN = 16384;
 constexpr int kP64[CO_FAST_MAX_K + 1] = {CUSR_P64_TABLE};
