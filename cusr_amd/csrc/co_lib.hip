@@ -1416,7 +1416,7 @@ extern "C" int co_eval_ex(void *handle, const PopHeader *h, const int32_t *nt, c
     const int N = h->N, D = h->n_vars, C = h->total_c;
     const size_t nX = (size_t)N * D, nY = (size_t)M * N, words = (size_t)plan.words;
     // one workgroup per expression: C's scalars, then the rows of 64 points in LDS
-    const int uni = (uni_doubles(h->K_max > 0 ? CO_MAX_K : 0, plan.max_cslots, 0) * (int)sizeof(double) + 15) & ~15;
+    const int uni = (eval_uni_doubles(plan) * (int)sizeof(double) + 15) & ~15;
     const size_t lds = uni + (size_t)plan.max_rows * kLanes * (precision == CO_PREC_FP64 ? 8 : 4);
     if (lds + sizeof(double) * CO_MAX_K > ctx->lds_per_block) return CO_ERR_BOUNDS;
     CO_GROW(ctx->prog, sizeof(uint64_t) * words);

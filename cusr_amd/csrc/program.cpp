@@ -935,11 +935,12 @@ int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const i
                            t.K, D, h->N, lo.gen[m] != 0, true, out, d, &cost[m], s);
     });
     if (rc != CO_OK) return rc;
-    int max_rows = 0, max_cslots = 0;
+    int max_rows = 0, max_ck = 0, max_cslots = 0;
     int64_t vcols = 0;
     for (int m = 0; m < M; m++) {
         ExprDesc &d = desc[m];
         if (d.rows > max_rows) max_rows = d.rows;
+        if (d.n_c > 0 && d.K > max_ck) max_ck = d.K;
         if (d.cslots > max_cslots) max_cslots = d.cslots;
         d.v_col = (int32_t)vcols;
         vcols += d.vrows;
@@ -985,6 +986,7 @@ int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const i
     plan->total_nodes = h->total_nodes;
     plan->total_c = h->total_c;
     plan->max_rows = max_rows;
+    plan->max_ck = max_ck;
     plan->max_cslots = max_cslots;
     plan->words = lo.words;
     plan->vcols = vcols;

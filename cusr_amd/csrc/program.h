@@ -175,11 +175,17 @@ constexpr int kFastRows = 16;                 // rows a fast word can address
 struct Plan {
     int32_t M, N, D, total_nodes, total_c;
     int32_t max_rows;      // LDS rows of a value pass
-    int32_t max_cslots;
+    int32_t max_ck;        // most constants of an expression with a C program (0: none)
+    int32_t max_cslots;    // most scalar slots of one
     int64_t words;         // program words (fast: n_nodes per expression, wide: 2 n_nodes)
     int64_t vcols;         // workspace columns of the V values
     int32_t n_gen;         // expressions of the general kernel
 };
+// Doubles of the scalar area of a launch that evaluates a whole plan: sized by the
+// decoded expressions, not by the header's K_max, which no check holds to them.
+static inline int eval_uni_doubles(const Plan &p) {
+    return p.max_ck > 0 ? uni_doubles(p.max_ck, p.max_cslots, 0) : 0;
+}
 
 // Check a population and decode it into plain programs (co_decode). Returns a
 // CO_* code. On success fills prog[2 * total_nodes] (expression m's program

@@ -1,0 +1,116 @@
+// layout_check.cpp -- host checks of the sizes and indices that the host plans
+// launches by against what the device reads and writes by them
+// (cusr_amd/csrc/program.h). Built and run by tests/test_layout.py with the
+// check's name; prints "layout ok".
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include <random>
+#include <vector>
+
+#include "../cusr_amd/csrc/program.h"
+
+using namespace cusr;
+
+#define CHECK(c)                                        \
+    do {                                                \
+        if (!(c)) {                                     \
+            printf("%s fails at line %d\n", #c, __LINE__); \
+            exit(1);                                    \
+        }                                               \
+    } while (0)
+
+// A population built tree by tree; operators and leaves in prefix order.
+struct Pop {
+    std::vector<int32_t> nt, ci;
+    std::vector<float> nv;
+    std::vector<TreeMeta> metas;
+    PopHeader h = {};
+    std::vector<uint64_t> prog;
+    std::vector<ExprDesc> desc;
+    Plan plan = {};
+
+    void op(int f, bool binary) {
+        nt.push_back(binary ? NODE_BFUNC : NODE_UFUNC);
+        nv.push_back((float)f);
+        ci.push_back(-1);
+        metas.back().n_nodes++;
+    }
+    void var(int v) {
+        nt.push_back(NODE_VAR);
+        nv.push_back((float)v);
+        ci.push_back(-1);
+        metas.back().n_nodes++;
+    }
+    void con() {
+        nt.push_back(NODE_CONST);
+        nv.push_back(0.0f);
+        ci.push_back(metas.back().K++);
+        metas.back().n_nodes++;
+        h.total_c++;
+    }
+    void tree() { metas.push_back({(int32_t)nt.size(), 0, h.total_c, 0}); }
+    int decode(int N, int D, int k_max) {
+        h.magic = POP_MAGIC;
+        h.version = POP_VERSION;
+        h.M_prob = (int)metas.size();
+        h.total_nodes = (int)nt.size();
+        h.N = N;
+        h.n_vars = D;
+        h.K_max = k_max;
+        prog.assign(staged_words_max(h.total_nodes, D), 0);
+        desc.assign(metas.size(), ExprDesc{});
+        const int rc = check_header(&h, nt.data(), nv.data(), ci.data(), metas.data());
+        return rc != CO_OK ? rc
+                           : decode_range(&h, nt.data(), nv.data(), ci.data(), metas.data(), 0,
+                                          h.M_prob, 0, prog.data(), desc.data(), &plan);
+    }
+};
+
+// sin(c) * x with k constants summed under the sine: a C program of k operators
+static void sine_of_constants(Pop &p, int k) {
+    p.tree();
+    p.op(OP_MUL, true);
+    p.op(OP_SIN, false);
+    for (int i = 1; i < k; i++) p.op(OP_ADD, true);
+    for (int i = 0; i < k; i++) p.con();
+    p.var(0);
+}
+
+// An evaluation's scalar area holds every expression's constants and slots, with
+// a header that claims fewer constants than the expressions have, or none.
+static void check_eval() {
+    for (int k_max : {0, 1, 8, 20})
+        for (int D : {1, 12}) {
+            Pop p;
+            sine_of_constants(p, 3);
+            sine_of_constants(p, 20);
+            p.tree();
+            p.var(0);
+            CHECK(p.decode(1024, D, k_max) == CO_OK);
+            const int room = eval_uni_doubles(p.plan);
+            bool any = false;
+            for (const ExprDesc &d : p.desc) {
+                if (d.n_c == 0) continue;
+                any = true;
+                CHECK(uni_doubles(d.K, d.cslots, 0) <= room);
+            }
+            CHECK(any);
+        }
+    Pop none;
+    none.tree();
+    none.op(OP_MUL, true);
+    none.con();
+    none.var(0);
+    CHECK(none.decode(1024, 1, 1) == CO_OK);
+    CHECK(eval_uni_doubles(none.plan) == 0);
+}
+
+int main(int argc, char **argv) {
+    CHECK(argc == 2);
+    if (!strcmp(argv[1], "eval")) check_eval();
+    else CHECK(!"check's name");
+    puts("layout ok");
+    return 0;
+}

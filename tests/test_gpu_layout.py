@@ -1,0 +1,43 @@
+"""Launches whose LDS is sized by the decoded expressions, against the CPU oracle
+(the sizes themselves: tests/test_layout.py)."""
+import numpy as np
+import pytest
+
+from cusr_amd.benchmark import popio
+from oracle import lm_oracle
+from tests.helpers import f64
+
+pytestmark = pytest.mark.gpu
+
+VAR, CONST, UN, BIN = popio.NODE_VAR, popio.NODE_CONST, popio.NODE_UFUNC, popio.NODE_BFUNC
+ADD, MUL, SIN = 1, 3, 14
+
+
+def _tree(k, D):
+    """sin(c0 + ... + c_{k-1}) * x_{D-1}"""
+    nt = [BIN, UN] + [BIN] * (k - 1) + [CONST] * k + [VAR]
+    nv = [float(MUL), float(SIN)] + [float(ADD)] * (k - 1) + [0.0] * k + [float(D - 1)]
+    return nt, nv, [-1] * (k + 1) + list(range(k)) + [-1]
+
+
+@pytest.mark.parametrize("D", [3, 12])     # fast and wide programs
+@pytest.mark.parametrize("k_max", [0, 2])
+def test_evaluate_with_understated_k_max(co, D, k_max):
+    """The header's K_max is no bound on the expressions' own: constants and C's
+    values keep their place beside the rows."""
+    rng = np.random.default_rng(5)
+    xs = rng.uniform(-2, 2, (700, D)).astype(np.float32)
+    slots = [(*_tree(k, D), rng.standard_normal(k).astype(np.float32)) for k in (1, 3, 7, 16, 20)]
+    pop = popio.build_pop(slots, xs, np.zeros((len(slots), 700)))
+    c0, x64, _ = f64(pop)
+    under = dict(pop, K_max=k_max)
+    print(f"evaluate D={D} K_max={k_max} of {pop['K_max']}", flush=True)
+    want = lm_oracle.eval_pop(pop, c=c0, xs=x64)
+    assert np.array_equal(co.evaluate(under, c0, x64), want)
+    # fp32: k - 1 sums, each within 2^-24 of a partial sum of at most sum |c|, go through
+    # the sine (slope at most 1) and the factor x; the sine, the product and the
+    # operands' own rounding are a few 2^-24 of |x|
+    single = co.evaluate(under, c0, x64, precision=1)
+    for m, (_, _, _, c) in enumerate(slots):
+        bound = (len(c) * np.abs(c).sum() + 8) * 2.0 ** -24 * np.abs(x64[:, D - 1])
+        assert np.all(np.abs(single[m] - want[m]) <= bound), m
