@@ -1140,8 +1140,6 @@ constexpr bool matrix_sums() {
 template <int K, int AD>
 constexpr bool sums_over_tape() { return AD == CO_AD_REVERSE && matrix_sums<K, AD>(); }
 
-constexpr int sums_width(int K) { return 1 + K + K * (K + 1) / 2; }
-
 // Cross-lane exchange of a double with lane ^ S (S = 32, 16, 8, 4, 2, 1):
 // ds_bpermute for 32, ds_swizzle (xor mask) for 16, DPP moves below: row_ror:8
 // is the xor-8 partner within a row of 16, row_half_mirror then the reversed
@@ -1595,9 +1593,9 @@ __device__ __forceinline__ void static_for(const Fn &f) {
 template <int KM, bool REL>
 __device__ __forceinline__ bool damped_solve(const double *s, int KL, int Kr, double lambda,
                                              int damp, int lane, double (&x)[KM], double &mine) {
-    constexpr int GS = 4, NG = (KM + GS - 1) / GS;   // columns behind one test of Kr
+    constexpr int GS = kSolveCols, NG = (KM + GS - 1) / GS;   // columns behind one test of Kr
     const int i = lane < Kr ? lane : Kr - 1;
-    const double *row = s + 1 + KL + i;   // entry (j, i) of the upper triangle at j KL - j (j+1) / 2
+    const double *row = s + sums_row(KL, 0) + i;   // entry (j, i) at j KL - j (j+1) / 2
     double a[KM];
     static_for<0, NG>([&](auto g) {
         if (g * GS < Kr)
@@ -1711,12 +1709,14 @@ __device__ __forceinline__ bool loss_ok(const FitArgs &fa, double loss) {
     return isfinite(loss) && (!fa.f32_range || isfinite((float)loss));
 }
 
-// Static LDS of a fit kernel: current and trial constants, current and trial
-// sums of the kernel's K (the general kernel: of the largest).
+// Static LDS of a fit kernel, one array: current and trial constants, then current
+// and trial sums of the kernel's K (the general kernel: of the largest).
 template <bool GEN, int K>
 struct FitStatic {
     static constexpr int KC = GEN ? CO_MAX_K : (K > 0 ? K : 1);
     static constexpr int SW = sums_width(KC);
+    static constexpr int size = 2 * KC + 2 * SW;
+    static_assert(2 * KC >= kSolveBefore, "the solve's loads before the sums");
 };
 
 // Points per lane of a fit's passes and of its fp64 audit passes: the
@@ -1735,7 +1735,7 @@ constexpr int fit_audit_points() {
 // PAD: expressions of fewer constants than K run in K's kernel (group_top): the
 // tangents, sums and solve of the entries past theirs are formed and not read.
 template <int K, typename R, int AD, int LN, bool GEN = false, bool PAD = false>
-__device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, double *lds_c, double *lds_s,
+__device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, double *lds,
                         char *lds_dyn, int lane, int wave) {
     typedef typename std::conditional<GEN, WideFmt, FastFmt>::type F;
     constexpr int P = fit_points<GEN, R, K, AD, LN>();
@@ -1773,8 +1773,8 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     pa.split = 0;
     pa.part_stride = 0;
 
-    double *c_cur = lds_c, *c_try = lds_c + KC;
-    double *s_cur = lds_s, *s_try = lds_s + FitStatic<GEN, K>::SW;
+    double *c_cur = lds, *c_try = lds + KC;
+    double *s_cur = lds + 2 * KC, *s_try = s_cur + FitStatic<GEN, K>::SW;
     double *sv = fa.state ? fa.state + (size_t)e.y_row * fa.state_stride : nullptr;
     double loss, loss_init, lambda;
     int st, it;
@@ -1994,13 +1994,12 @@ constexpr bool large_n_variant() {
 template <int K, typename R, int AD, int LN = 0, bool PAD = false>
 __global__ void __launch_bounds__(kLanes * CO_MAX_PARTITIONS, (waves_per_eu<R, K, AD, LN>()))
 lm_fit_kernel(FitArgs fa) {
-    __shared__ double lds_c[2 * FitStatic<false, K>::KC];
-    __shared__ double lds_s[2 * FitStatic<false, K>::SW];
+    __shared__ double lds[FitStatic<false, K>::size];
     extern __shared__ char lds_dyn[];
     const ExprDesc e = fa.desc[blockIdx.x];
     const int lane = (int)threadIdx.x & (kLanes - 1);
     const int wave = uni((int)threadIdx.x >> 6);
-    fit_one<K, R, AD, LN, false, PAD>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
+    fit_one<K, R, AD, LN, false, PAD>(fa, e, lds, lds_dyn, lane, wave);
 }
 
 // The general kernel: runtime K <= CO_MAX_K, wide programs, one point per
@@ -2011,13 +2010,12 @@ lm_fit_kernel(FitArgs fa) {
 template <typename R, int AD>
 __global__ void __launch_bounds__(kLanes * CO_MAX_PARTITIONS, CUSR_WAVES_GEN)
 lm_fit_gen_kernel(FitArgs fa) {
-    __shared__ double lds_c[2 * FitStatic<true, kGenK>::KC];
-    __shared__ double lds_s[2 * FitStatic<true, kGenK>::SW];
+    __shared__ double lds[FitStatic<true, kGenK>::size];
     extern __shared__ char lds_dyn[];
     const ExprDesc e = fa.desc[blockIdx.x];
     const int lane = (int)threadIdx.x & (kLanes - 1);
     const int wave = uni((int)threadIdx.x >> 6);
-    fit_one<kGenK, R, AD, 0, true>(fa, e, lds_c, lds_s, lds_dyn, lane, wave);
+    fit_one<kGenK, R, AD, 0, true>(fa, e, lds, lds_dyn, lane, wave);
 }
 
 // The K whose kernel runs a group of bins in one launch, padded: the largest of
@@ -2032,7 +2030,7 @@ constexpr int group_top(int K, bool rev) {
 // Static LDS bytes of a bin's fit kernel (kept out of the dynamic budget).
 constexpr size_t fit_static_lds(int bin) {
     const int kc = bin == CO_GENERAL_BIN ? CO_MAX_K : (bin > 0 ? bin : 1);
-    return (2 * kc + 2 * sums_width(kc)) * sizeof(double);
+    return (2 * kc + 2 * sums_width(kc)) * sizeof(double);   // FitStatic::size
 }
 
 // Dynamic LDS bytes one wavefront of a fit launch needs beside its scalar area (the mixed-precision

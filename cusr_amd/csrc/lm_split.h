@@ -134,8 +134,11 @@ lm_pass_kernel(FitArgs fa) {
 template <int KS, bool PAD = false>
 __global__ void __launch_bounds__(kLanes) lm_step_kernel(FitArgs fa, int mixed) {
     __shared__ double s_new[sums_width(CO_MAX_K)];
-    __shared__ double s_cur[sums_width(CO_MAX_K)];
-    __shared__ double c_cur[CO_MAX_K], c_try[CO_MAX_K];
+    __shared__ double c_try[CO_MAX_K];
+    // one array: the solve may read kSolveBefore entries before the sums
+    __shared__ double lds_cur[CO_MAX_K + sums_width(CO_MAX_K)];
+    static_assert(CO_MAX_K >= kSolveBefore, "the solve's loads before the sums");
+    double *c_cur = lds_cur, *s_cur = lds_cur + CO_MAX_K;
     const int idx = blockIdx.x;
     const int lane = (int)threadIdx.x;
     const ExprDesc e = fa.desc[idx];

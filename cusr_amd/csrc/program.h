@@ -172,6 +172,18 @@ static inline __host__ __device__ int uni_doubles(int K, int cslots, int ctape) 
 constexpr int kWideCidxMax = (1 << 20) - 1;   // C instructions a wide word can address
 constexpr int kFastRows = 16;                 // rows a fast word can address
 
+// The sums vector of a Jacobian pass over K constants: r^2, J^T r, then the upper
+// triangle of J^T J row by row; entry (j, i), i >= j, is at sums_row(K, j) + i.
+static inline constexpr __host__ __device__ int sums_width(int K) { return 1 + K + K * (K + 1) / 2; }
+static inline constexpr __host__ __device__ int sums_row(int K, int j) {
+    return 1 + K + j * K - (j * (j + 1)) / 2;
+}
+// The damped solve takes columns in fours (kSolveCols), so up to three past a
+// runtime K are loaded from sums_row and not used. They lie within the vector but
+// for column 3 at K = 1, which starts kSolveBefore entries before it: the kernels
+// keep the constants there, in one array with the sums, and test no column.
+constexpr int kSolveCols = 4, kSolveBefore = 1;
+
 struct Plan {
     int32_t M, N, D, total_nodes, total_c;
     int32_t max_rows;      // LDS rows of a value pass

@@ -107,9 +107,35 @@ static void check_eval() {
     CHECK(eval_uni_doubles(none.plan) == 0);
 }
 
+// The damped solve's loads stay within its sums and the kSolveBefore entries that
+// every kernel holds before them: at every K of the kernel whose K is
+// known at run time only (the sums laid out by it), and for every group of K
+// bins in a padded kernel (laid out by the kernel's K).
+static void check_solve() {
+    auto loads = [](int KM, int KL, int Kr) {
+        for (int g = 0; g * kSolveCols < Kr; g++)
+            for (int j = g * kSolveCols; j < (g + 1) * kSolveCols && j < KM; j++)
+                for (int i = 0; i < Kr; i++) {
+                    const int at = sums_row(KL, j) + i;
+                    CHECK(at >= -kSolveBefore && at < sums_width(KL));
+                    // a column that is used holds its own entries
+                    if (j < Kr && i >= j) {
+                        int q = 1 + KL;
+                        for (int a = 0; a < j; a++) q += KL - a;
+                        CHECK(at == q + i - j);
+                    }
+                }
+        for (int i = 0; i < Kr; i++) CHECK(sums_row(KL, i) + i < sums_width(KL));
+    };
+    for (int K = 1; K <= CO_MAX_K; K++) loads(CO_MAX_K, K, K);
+    for (int top = 1; top <= CO_FAST_MAX_K; top++)
+        for (int K = 1; K <= top; K++) loads(top, top, K);
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
+    else if (!strcmp(argv[1], "solve")) check_solve();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;
