@@ -1,6 +1,6 @@
-// layout_check.cpp -- host checks of the sizes and indices that the host plans
+// layout_check.hip -- host checks of the sizes and indices that the host plans
 // launches by against what the device reads and writes by them
-// (cusr_amd/csrc/program.h). Built and run by tests/test_layout.py with the
+// (cusr_amd/csrc/program.h, launch_plan.h). Built and run by tests/test_layout.py with the
 // check's name; prints "layout ok".
 #include <stdio.h>
 #include <stdlib.h>
@@ -9,6 +9,7 @@
 #include <random>
 #include <vector>
 
+#include "../cusr_amd/csrc/launch_plan.h"
 #include "../cusr_amd/csrc/program.h"
 
 using namespace cusr;

@@ -1,5 +1,6 @@
 """What the host plans a launch's LDS and indices by, against what the device uses
-(tests/layout_check.cpp, on the host)."""
+(tests/layout_check.hip, compiled for the host)."""
+import shutil
 import subprocess
 from pathlib import Path
 
@@ -10,11 +11,16 @@ REPO = Path(__file__).resolve().parents[1]
 
 @pytest.fixture(scope="module")
 def exe(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not available")
     out = tmp_path_factory.mktemp("layout") / "layout_check"
-    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Wno-unused-function", "-pthread",
-                    "-ffp-contract=off", "-D__host__=", "-D__device__=", "-o", str(out),
-                    str(REPO / "tests" / "layout_check.cpp"),
-                    str(REPO / "cusr_amd" / "csrc" / "program.cpp")], check=True)
+    subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-Wall",
+                    "-Wno-unused-function", "-ffp-contract=off", "-Xclang", "-target-feature",
+                    "-Xclang", "-packed-fp32-ops", f"-I{REPO / 'include'}",
+                    str(REPO / "tests" / "layout_check.hip"),
+                    str(REPO / "cusr_amd" / "csrc" / "program.cpp"), "-pthread", "-o", str(out)],
+                   check=True, capture_output=True, timeout=300)
     return out
 
 
