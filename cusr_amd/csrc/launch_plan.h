@@ -67,6 +67,10 @@ struct LaunchPlan {
     size_t lds[2];
 };
 
+// The K of a launch's kernel, by which it holds tangents (sums: by the expression's
+// own in the general kernel).
+static inline int kernel_k(const LaunchPlan &b) { return b.bin == CO_GENERAL_BIN ? kGenK : b.bin; }
+
 // Bytes of a launch's per-wavefront scalar area.
 static inline int uni_bytes(const LaunchPlan &b) { return (b.uni * (int)sizeof(double) + 15) & ~15; }
 
@@ -118,7 +122,7 @@ static inline int plan_launches(const ExprDesc *desc, int p0, int p1, const Plan
                                 : (!desc[pos].gen && desc[pos].K == bin))) {
             const ExprDesc &d = desc[pos];
             const int rows = rev ? d.rows_rev : d.rows;
-            const int uni = d.n_c ? uni_doubles(d.K, d.cslots, rev ? d.ctape : 0) : 0;
+            const int uni = d.n_c ? uni_at(d.K, 0, d.cslots, rev ? d.ctape : 0).size : 0;
             if (rows > b.rows) b.rows = rows;
             if (uni > b.uni) b.uni = uni;
             if (d.tape > b.tape) b.tape = d.tape;
@@ -167,6 +171,8 @@ static inline int plan_launches(const ExprDesc *desc, int p0, int p1, const Plan
         // the handle's own stream first: a fit of one launch waits for no other
         const int lane = !gen_alone ? i % kStreams : (gen ? 0 : 1 + (i - 1) % (kStreams - 1));
         b.stream = (lane + kExtraStreams) % kStreams;
+        // forward AD: the tangents that C leaves, to the kernel's K
+        if (b.uni > 0 && !rev) b.uni += kernel_k(b);
         // per-wavefront areas, then the partition sums; fewer wavefronts per
         // workgroup (each summing several partitions) when LDS is short. The
         // split path's pass workgroups are one wavefront with no partition

@@ -819,20 +819,16 @@ __device__ __forceinline__ void forward_pass(ProgPtr prog, int n, const WaveLds<
     }
 }
 
-// LDS of one wavefront for the scalar program C (program.h, uni_doubles).
+// LDS of one wavefront for the scalar program C (program.h, uni_at).
 struct UniLds {
-    double *cm;      // [K] the constants, then C's values in place
-    double *t0;      // [K] forward AD: the tangents M starts from
+    double *cm;      // [Kr] the constants, then C's values in place
+    double *t0;      // [K] forward AD: the tangents M starts from, 1 past the expression's Kr
     double *slot;    // C's spill slots
     double *tape;    // reverse AD: C's partials
 };
-__device__ __forceinline__ UniLds uni_lds(double *base, int K, int cslots) {
-    UniLds u;
-    u.cm = base;
-    u.t0 = base + K;
-    u.slot = base + 2 * K;
-    u.tape = u.slot + cslots;
-    return u;
+__device__ __forceinline__ UniLds uni_lds(double *base, int K, int t0, int cslots) {
+    const UniAt at = uni_at(K, t0, cslots, 0);
+    return {base, base + at.t0, base + at.slot, base + at.tape};
 }
 
 // The scalar program C at constants cs: every lane computes the same single
@@ -897,11 +893,12 @@ __device__ __forceinline__ void const_phase(ProgPtr prog, int n, const UniLds &u
         acc[0] = o[0];
     }
     if constexpr (JAC == 1) {
-        // all lanes hold the same row: entry j from lane j, in one store
+        // all lanes hold the same row: entry j from lane j, in one store, to the
+        // kernel's K (the entries past Kr, still 1, are read there too)
         double t = 0.0;
 #pragma unroll
         for (int j = 0; j < K; ++j) t = lane == j ? (double)T[j] : t;
-        if (lane < Kr) u.t0[lane] = t;
+        if (lane < K) u.t0[lane] = t;
     }
     wave_order_lds();
 }
@@ -1035,10 +1032,10 @@ struct PassArgs {
 };
 
 // The program part of PassArgs from an expression's descriptor. v: the fit's
-// workspace (null: none), uni: this wavefront's scalar area.
+// workspace (null: none), uni: this wavefront's scalar area, t0: its tangents.
 template <typename R, typename F>
 __device__ __forceinline__ void program_args(PassArgs &a, const uint64_t *prog, const ExprDesc &e,
-                                             int Kr, int N, void *v, double *uni) {
+                                             int Kr, int t0, int N, void *v, double *uni) {
     a.prog = (ProgPtr)(prog + e.prog_off);
     a.n_c = e.n_c;
     a.n_v = e.n_v;
@@ -1053,7 +1050,7 @@ __device__ __forceinline__ void program_args(PassArgs &a, const uint64_t *prog, 
     // audits of a mixed fit keep theirs over its own fp32 ones
     a.V = (v && e.vrows > 0) ? (void *)((double *)v + (size_t)e.v_col * N) : nullptr;
     a.vmode = a.V ? V_LOAD : V_RUN;
-    a.u = uni_lds(uni, Kr, e.cslots);
+    a.u = uni_lds(uni, Kr, t0, e.cslots);
     a.N = N;
 }
 
@@ -1746,8 +1743,8 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     char *my_lds = lds_dyn + (size_t)wave * fa.wave_bytes;
     const bool lead = wave == 0;     // the wavefront that writes shared state
     PassArgs pa;
-    program_args<R, F>(pa, fa.prog, e, Kr, fa.N, fa.max_iter > 0 ? fa.V : nullptr,
-                       (double *)my_lds);
+    program_args<R, F>(pa, fa.prog, e, Kr, JAC == 1 ? K : 0, fa.N,
+                       fa.max_iter > 0 ? fa.V : nullptr, (double *)my_lds);
     my_lds += fa.uni_bytes;
     double *jt = (double *)my_lds;   // matrix sums: the slice's augmented rows first
     // (reverse AD puts them in the tape's bytes)
@@ -2098,7 +2095,7 @@ __global__ void __launch_bounds__(kLanes) eval_kernel(EvalArgs ea) {
     const ExprDesc e = ea.desc[blockIdx.x];
     if (lane < e.K) cs[lane] = ea.C[e.c_off + lane];
     PassArgs a;
-    program_args<R, F>(a, ea.prog, e, e.K, ea.N, nullptr, (double *)lds_dyn);
+    program_args<R, F>(a, ea.prog, e, e.K, 0, ea.N, nullptr, (double *)lds_dyn);
     a.X = ea.X;
     WaveLds<R, P> w;
     w.x = (R *)(lds_dyn + ea.uni_bytes);

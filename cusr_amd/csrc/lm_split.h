@@ -78,8 +78,8 @@ lm_pass_kernel(FitArgs fa) {
     if (lane < Kr) cs[lane] = src[lane];
     wave_sync_lds();
     PassArgs pa;
-    program_args<R, F>(pa, fa.prog, e, Kr, fa.N, fa.max_iter > 0 ? fa.V : nullptr,
-                       (double *)lds_dyn);
+    program_args<R, F>(pa, fa.prog, e, Kr, JAC == 1 ? K : 0, fa.N,
+                       fa.max_iter > 0 ? fa.V : nullptr, (double *)lds_dyn);
     if (kind == SP_INIT && pa.vmode == V_LOAD) pa.vmode = V_KEEP;
     char *my_lds = lds_dyn + fa.uni_bytes;
     double *jt = (double *)my_lds;

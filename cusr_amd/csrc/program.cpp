@@ -643,7 +643,7 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
         }
         const size_t row = 64 * sizeof(double);
         const size_t now = (d.rows_rev + d.tape) * row +
-                           uni_doubles(K, d.cslots, d.ctape) * sizeof(double);
+                           uni_at(K, 0, d.cslots, d.ctape).size * sizeof(double);
         if (now > (64u << 10) && now > (plain_rows + (size_t)plain_tape) * row) {
             memset(out, 0, sizeof(uint64_t) * program_words(n, true, true));
             return emit_staged(nt, nv, ci, n, K, D, N, wide, false, out, d, cost, s);

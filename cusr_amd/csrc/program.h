@@ -164,10 +164,15 @@ static inline __host__ __device__ int wst_mid(uint64_t b) { return (int)(((uint3
 static inline __host__ __device__ int wst_hi(uint64_t b) { return (int)(((uint32_t)b >> 16) & 255u); }
 static inline __host__ __device__ int wst_didx(uint64_t b) { return (int)(ins_w1(b) & 4095u); }
 static inline __host__ __device__ int wst_tape(uint64_t b) { return (int)(ins_w1(b) >> 12); }
-// Doubles of a wavefront's scalar area (LDS): the constants with C's values in
-// place, the tangents C leaves, C's slots and its reverse-AD tape.
-static inline __host__ __device__ int uni_doubles(int K, int cslots, int ctape) {
-    return 2 * K + cslots + ctape;
+// A wavefront's scalar area (LDS), in doubles: the constants with C's values in
+// place, the tangents C leaves (forward AD: t0 of them, the kernel's own K, which a
+// padded or the general kernel reads whatever the expression's), C's slots and its
+// reverse-AD tape.
+struct UniAt {
+    int t0, slot, tape, size;
+};
+static inline constexpr __host__ __device__ UniAt uni_at(int K, int t0, int cslots, int ctape) {
+    return {K, K + t0, K + t0 + cslots, K + t0 + cslots + ctape};
 }
 constexpr int kWideCidxMax = (1 << 20) - 1;   // C instructions a wide word can address
 constexpr int kFastRows = 16;                 // rows a fast word can address
@@ -196,7 +201,7 @@ struct Plan {
 // Doubles of the scalar area of a launch that evaluates a whole plan: sized by the
 // decoded expressions, not by the header's K_max, which no check holds to them.
 static inline int eval_uni_doubles(const Plan &p) {
-    return p.max_ck > 0 ? uni_doubles(p.max_ck, p.max_cslots, 0) : 0;
+    return p.max_ck > 0 ? uni_at(p.max_ck, 0, p.max_cslots, 0).size : 0;
 }
 
 // Check a population and decode it into plain programs (co_decode). Returns a

@@ -95,7 +95,7 @@ static void check_eval() {
             for (const ExprDesc &d : p.desc) {
                 if (d.n_c == 0) continue;
                 any = true;
-                CHECK(uni_doubles(d.K, d.cslots, 0) <= room);
+                CHECK(uni_at(d.K, 0, d.cslots, 0).size <= room);
             }
             CHECK(any);
         }
@@ -133,10 +133,74 @@ static void check_solve() {
         for (int K = 1; K <= top; K++) loads(top, top, K);
 }
 
+// Plans the decoded population's launches at the default options of its N.
+static int plan(const Pop &p, bool rev, bool mixed, int parts, std::vector<LaunchPlan> &lp,
+                bool group = true) {
+    PlanArgs a = {};
+    a.rev = rev;
+    a.mixed = mixed;
+    a.split = parts > CO_MAX_PARTITIONS;
+    a.group = group;
+    a.N = p.h.N;
+    a.parts = a.seg_parts[0] = parts;
+    a.nseg = 1;
+    a.lds_per_block = 160 << 10;
+    lp.resize(CO_BINS);
+    int nl = 0, kmax = 0;
+    const int rc = plan_launches(p.desc.data(), 0, p.h.M_prob, a, lp.data(), &nl, &kmax);
+    lp.resize(rc == CO_OK ? nl : 0);
+    return rc;
+}
+
+// Every launch's scalar area holds its expressions' constants, the tangents that
+// its kernel reads (its own K of them, padded and general kernels too), the
+// slots and the tape; rows of one point for the rest of the launch's LDS.
+static void check_scalars() {
+    for (int N : {60, 1024, 70000})
+        for (int D : {1, 12})
+            for (bool vars : {false, true}) {
+                Pop p;
+                for (int k : {1, 1, 2, 3, 4, 5, 7, 9, 11, 12, 13, 15, 16, 20, 32}) {
+                    if (vars) {
+                        sine_of_constants(p, k);
+                        continue;
+                    }
+                    // constants alone: a scalar area and no rows beside it
+                    p.tree();
+                    p.op(OP_SIN, false);
+                    for (int i = 1; i < k; i++) p.op(OP_ADD, true);
+                    for (int i = 0; i < k; i++) p.con();
+                }
+                CHECK(p.decode(N, D, 32) == CO_OK);
+                for (int parts : {1, 4, 8})
+                    for (int mode = 0; mode < 8; mode++) {
+                        const bool rev = mode & 1, mixed = mode & 2, group = mode & 4;
+                        std::vector<LaunchPlan> lp;
+                        CHECK(plan(p, rev, mixed, parts, lp, group) == CO_OK);
+                        int n = 0;
+                        for (const LaunchPlan &b : lp) {
+                            for (int q = b.pos; q < b.pos + b.cnt; q++, n++) {
+                                const ExprDesc &d = p.desc[q];
+                                CHECK(b.bin == CO_GENERAL_BIN ? d.gen : !d.gen && d.K <= b.bin);
+                                if (d.n_c == 0) continue;
+                                const int t0 = rev ? 0 : kernel_k(b);
+                                const UniAt at = uni_at(d.K, t0, d.cslots, rev ? d.ctape : 0);
+                                CHECK(at.t0 >= d.K && at.slot - at.t0 >= t0);
+                                CHECK(at.size * (int)sizeof(double) <= uni_bytes(b));
+                                CHECK(uni_bytes(b) + (rev ? d.rows_rev : d.rows) * 256 <=
+                                      (int)b.wave_bytes);
+                            }
+                        }
+                        CHECK(n == p.h.M_prob);
+                    }
+            }
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
     else if (!strcmp(argv[1], "solve")) check_solve();
+    else if (!strcmp(argv[1], "scalars")) check_scalars();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;

@@ -41,3 +41,28 @@ def test_evaluate_with_understated_k_max(co, D, k_max):
     for m, (_, _, _, c) in enumerate(slots):
         bound = (len(c) * np.abs(c).sum() + 8) * 2.0 ** -24 * np.abs(x64[:, D - 1])
         assert np.all(np.abs(single[m] - want[m]) <= bound), m
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(ad_mode=1), dict(partitions=8),
+                                  dict(partitions=1, precision=1)])
+def test_constants_alone_in_padded_kernels(co, opts):
+    """Expressions without variables in groups of K bins: a scalar area and no rows,
+    whose tangents a padded kernel reads up to its own K."""
+    rng = np.random.default_rng(11)
+    xs = rng.uniform(-2, 2, (1100, 3)).astype(np.float32)
+    slots = []
+    for k in (1, 1, 2, 3, 5, 7, 9, 11, 13, 14, 20):
+        nt, nv, ci = _tree(k, 3)
+        slots.append((nt[1:-1], nv[1:-1], ci[1:-1], rng.standard_normal(k).astype(np.float32)))
+        slots.append((*_tree(k, 3), rng.standard_normal(k).astype(np.float32)))
+    y = rng.standard_normal((len(slots), 1100)).astype(np.float32)
+    pop = popio.build_pop(slots, xs, y)
+    print(f"constants alone M={pop['M']} {opts}", flush=True)
+    g = co.optimize_ex(pop, 6, **opts)
+    o = lm_oracle.fit(pop, max_iter=6, **opts)
+    if opts.get("precision"):
+        # fp32 partials: each step's path may differ; the fp64 losses at the start do not
+        assert np.array_equal(g["loss_init"], o["loss_init"])
+        return
+    for k in ("status", "loss_init", "loss_final", "iters", "c_final"):
+        assert np.array_equal(g[k], o[k], equal_nan=True), k
