@@ -60,6 +60,7 @@ static inline size_t max_dyn_lds(size_t lds_per_block, int bin) {
 // anything is launched, so a launch that cannot fit is refused up front).
 struct LaunchPlan {
     int bin, pos, cnt, rows, tape, uni, kmax, stream;   // uni: doubles of the scalar area
+    size_t gen_bytes;   // general bin: the LDS of its largest expression's wavefront
     uint32_t bins;   // the bins it covers, bit by bit (a group: several)
     bool group;      // run by the padded kernel of group_top
     size_t wave_bytes;
@@ -126,6 +127,11 @@ static inline int plan_launches(const ExprDesc *desc, int p0, int p1, const Plan
             if (rows > b.rows) b.rows = rows;
             if (uni > b.uni) b.uni = uni;
             if (d.tape > b.tape) b.tape = d.tape;
+            if (gen) {
+                const size_t own = (size_t)uni_bytes_of(d, rev, kGenK) +
+                                   fit_lds_bytes(mixed, rev, bin, a.N, rows, rev ? d.tape : 0);
+                if (own > b.gen_bytes) b.gen_bytes = own;
+            }
             if (d.K > b.kmax) b.kmax = d.K;
             ++b.cnt;
             ++pos;
@@ -178,8 +184,9 @@ static inline int plan_launches(const ExprDesc *desc, int p0, int p1, const Plan
         // split path's pass workgroups are one wavefront with no partition
         // sums in LDS.
         const int N = b.group ? 0 : a.N;   // a group has no large-N instance
-        b.wave_bytes = uni_bytes(b) + ((fit_lds_bytes(mixed, rev, b.bin, N, b.rows, b.tape) +
-                                        15) & ~(size_t)15);
+        const size_t own = gen ? b.gen_bytes
+                               : uni_bytes(b) + fit_lds_bytes(mixed, rev, b.bin, N, b.rows, b.tape);
+        b.wave_bytes = (own + 15) & ~(size_t)15;
         const size_t cap = max_dyn_lds(a.lds_per_block, b.bin);
         const int ks = gen ? b.kmax : b.bin;
         for (int g = 0; g < (b.kmax == 0 || split ? 1 : a.nseg); ++g) {

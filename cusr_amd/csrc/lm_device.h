@@ -1669,10 +1669,11 @@ struct FitArgs {
     int shared_y;           // 1: Y is one row [N] shared by every expression
     int f32_range;          // 1: constants and losses held to the fp32 range
     double lambda0, xtol;
-    int rows, tape;         // per-wave LDS rows of this launch ([row][P][64] each)
+    int rows, tape;         // per-wave LDS rows of this launch ([row][P][64] each; the
+                            // general kernel takes its expression's own)
     void *V;                // [columns][N] workspace of the V values (null: run V in
                             // every pass), of the fit's type
-    int uni_bytes;          // per-wave scalar area of this launch, its first bytes
+    int uni_bytes;          // per-wave scalar area of this launch, its first bytes (likewise)
     int parts;              // point partitions per expression (1, 2 or 4)
     int pwaves;             // wavefronts of the workgroup (divides parts)
     int wave_bytes;         // dynamic LDS of one wavefront; partition sums follow
@@ -1745,7 +1746,11 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     PassArgs pa;
     program_args<R, F>(pa, fa.prog, e, Kr, JAC == 1 ? K : 0, fa.N,
                        fa.max_iter > 0 ? fa.V : nullptr, (double *)my_lds);
-    my_lds += fa.uni_bytes;
+    // the general kernel's areas are laid out by the expression itself, so that a
+    // launch needs the LDS of its largest expression, not the sum of each area's
+    // largest (plan_launches)
+    const int rows = !GEN ? fa.rows : JAC == 2 ? e.rows_rev : e.rows;
+    my_lds += GEN ? uni_bytes_of(e, JAC == 2, K) : fa.uni_bytes;
     double *jt = (double *)my_lds;   // matrix sums: the slice's augmented rows first
     // (reverse AD puts them in the tape's bytes)
     if constexpr (GEN) {
@@ -1758,7 +1763,7 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     }
     WaveLds<R, P> wl;
     wl.x = (R *)my_lds;
-    wl.tape = wl.x + (size_t)fa.rows * P * kLanes;
+    wl.tape = wl.x + (size_t)rows * P * kLanes;
     if constexpr (!GEN && sums_over_tape<K, AD>()) jt = (double *)wl.tape;
     pa.X = fa.X;
     pa.y = fa.Y + (fa.shared_y ? (size_t)0 : (size_t)e.y_row * fa.N);
@@ -1909,7 +1914,7 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
         constexpr int KA = GEN ? 0 : K;
         WaveLds<double, AP> w64;
         w64.x = (double *)my_lds;
-        w64.tape = w64.x + (size_t)fa.rows * AP * kLanes;
+        w64.tape = w64.x + (size_t)rows * AP * kLanes;
         // the first audit keeps V's fp64 values for the second, over the fit's
         // fp32 ones (every wavefront is past its last pass)
         pa.vmode = pa.V ? V_KEEP : V_RUN;

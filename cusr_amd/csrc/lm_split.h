@@ -81,13 +81,14 @@ lm_pass_kernel(FitArgs fa) {
     program_args<R, F>(pa, fa.prog, e, Kr, JAC == 1 ? K : 0, fa.N,
                        fa.max_iter > 0 ? fa.V : nullptr, (double *)lds_dyn);
     if (kind == SP_INIT && pa.vmode == V_LOAD) pa.vmode = V_KEEP;
-    char *my_lds = lds_dyn + fa.uni_bytes;
+    const int rows = !GEN ? fa.rows : JAC == 2 ? e.rows_rev : e.rows;
+    char *my_lds = lds_dyn + (GEN ? uni_bytes_of(e, JAC == 2, K) : fa.uni_bytes);
     double *jt = (double *)my_lds;
     if constexpr (GEN) {
         my_lds += kGenJtBytes;
     } else if constexpr (sums_over_tape<K, AD>()) {
         // the rows go to the Jacobian pass's tape bytes (after the interpreter's rows)
-        jt = (double *)(my_lds + (size_t)fa.rows * P * kLanes * sizeof(R));
+        jt = (double *)(my_lds + (size_t)rows * P * kLanes * sizeof(R));
     } else if constexpr (matrix_sums<K, AD>()) {
 #pragma unroll
         for (int j = 0; j < kJtStride; ++j) jt[lane * kJtStride + j] = 0.0;
@@ -105,7 +106,7 @@ lm_pass_kernel(FitArgs fa) {
     if (kind == SP_INIT || kind == SP_TRIAL) {
         WaveLds<R, P> wl;
         wl.x = (R *)my_lds;
-        wl.tape = wl.x + (size_t)fa.rows * P * kLanes;
+        wl.tape = wl.x + (size_t)rows * P * kLanes;
         if constexpr (GEN) {
             if (Kr == 0) data_pass<0, R, 1, 0, F>(pa, wl, cs, nullptr, lane);
             else data_pass_gen<R, JAC, F>(pa, wl, cs, nullptr, lane, Kr);
@@ -116,7 +117,7 @@ lm_pass_kernel(FitArgs fa) {
         constexpr int KA = GEN ? 0 : K;
         WaveLds<double, AP> w64;
         w64.x = (double *)my_lds;
-        w64.tape = w64.x + (size_t)fa.rows * AP * kLanes;
+        w64.tape = w64.x + (size_t)rows * AP * kLanes;
         // the first audit keeps V's fp64 values for the second, over the fit's
         // fp32 ones
         pa.vmode = !pa.V ? V_RUN : kind == SP_AUDIT_CUR ? V_KEEP : V_LOAD;

@@ -629,9 +629,10 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
     // V runs once in a fit and C once per pass, by one point per lane
     *cost = 229 + op_costs[M] + op_costs[C] / 4;
     if (wide && stage) {
-        // a wavefront's LDS in reverse AD (512 bytes a row or tape slot) must
-        // not pass what the plain program took where that may have been the
-        // device's limit
+        // what the general kernel's wavefront takes for it in reverse AD must not
+        // pass what the plain program took where that may have been the device's
+        // limit (at 512 bytes a row and tape slot in fp64; measured by the 256 of
+        // fp32, which hold for both)
         int plain_tape = 0;
         for (int i = 0; i < n; i++) {
             if (is_leaf(nt[i])) continue;
@@ -641,10 +642,10 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
             plain_tape += nt[i + 1] != NODE_VAR;
             if (bin) plain_tape += nt[i + 1 + left[i]] != NODE_VAR;
         }
-        const size_t row = 64 * sizeof(double);
-        const size_t now = (d.rows_rev + d.tape) * row +
-                           uni_at(K, 0, d.cslots, d.ctape).size * sizeof(double);
-        if (now > (64u << 10) && now > (plain_rows + (size_t)plain_tape) * row) {
+        const size_t row = 64 * sizeof(float), rows = (size_t)d.rows_rev + d.tape;
+        const size_t uni = (size_t)uni_bytes_of(d, true, K);
+        if (2 * rows * row + uni > (64u << 10) &&
+            rows * row + uni > (plain_rows + (size_t)plain_tape) * row) {
             memset(out, 0, sizeof(uint64_t) * program_words(n, true, true));
             return emit_staged(nt, nv, ci, n, K, D, N, wide, false, out, d, cost, s);
         }

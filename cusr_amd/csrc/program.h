@@ -174,6 +174,12 @@ struct UniAt {
 static inline constexpr __host__ __device__ UniAt uni_at(int K, int t0, int cslots, int ctape) {
     return {K, K + t0, K + t0 + cslots, K + t0 + cslots + ctape};
 }
+// Bytes of the scalar area that an expression takes in a kernel of K kernel_k.
+static inline __host__ __device__ int uni_bytes_of(const ExprDesc &d, bool rev, int kernel_k) {
+    if (d.n_c == 0) return 0;
+    const UniAt at = uni_at(d.K, rev ? 0 : kernel_k, d.cslots, rev ? d.ctape : 0);
+    return (at.size * (int)sizeof(double) + 15) & ~15;
+}
 constexpr int kWideCidxMax = (1 << 20) - 1;   // C instructions a wide word can address
 constexpr int kFastRows = 16;                 // rows a fast word can address
 

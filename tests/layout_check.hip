@@ -186,9 +186,10 @@ static void check_scalars() {
                                 const int t0 = rev ? 0 : kernel_k(b);
                                 const UniAt at = uni_at(d.K, t0, d.cslots, rev ? d.ctape : 0);
                                 CHECK(at.t0 >= d.K && at.slot - at.t0 >= t0);
-                                CHECK(at.size * (int)sizeof(double) <= uni_bytes(b));
-                                CHECK(uni_bytes(b) + (rev ? d.rows_rev : d.rows) * 256 <=
-                                      (int)b.wave_bytes);
+                                const int ub = b.bin == CO_GENERAL_BIN
+                                                   ? uni_bytes_of(d, rev, kGenK) : uni_bytes(b);
+                                CHECK(at.size * (int)sizeof(double) <= ub);
+                                CHECK(ub + (rev ? d.rows_rev : d.rows) * 256 <= (int)b.wave_bytes);
                             }
                         }
                         CHECK(n == p.h.M_prob);
@@ -196,11 +197,112 @@ static void check_scalars() {
             }
 }
 
+// Rows (variables and spill slots) and reverse-AD tape of the plain programs, the
+// largest of each over the population.
+static void plain_lds(const Pop &p, int *rows, int *tape) {
+    std::vector<uint64_t> w(2 * p.nt.size());
+    std::vector<int32_t> off(p.metas.size());
+    CHECK(decode_population(&p.h, p.nt.data(), p.nv.data(), p.ci.data(), p.metas.data(), w.data(),
+                            nullptr, nullptr, nullptr, off.data(), nullptr) == CO_OK);
+    int slots = 0;
+    *tape = 0;
+    for (size_t m = 0; m < p.metas.size(); m++) {
+        int t = 0;
+        for (int k = 0; k < p.metas[m].n_nodes; k++) {
+            const uint64_t a = w[off[m] + 2 * k];
+            t += (int)(a >> 39 & 1) + (int)(a >> 40 & 1);
+            if (a >> 27 & 1 && (int)(a >> 28 & 255) + 1 > slots) slots = (int)(a >> 28 & 255) + 1;
+        }
+        if (t > *tape) *tape = t;
+    }
+    *rows = p.h.n_vars + slots;
+}
+
+// A sum of K constants times functions of x, some of them subtrees of variables
+// alone (v of them), and one subtree of constants alone.
+static void sum_with_subtrees(Pop &p, int K, int v, int D) {
+    p.tree();
+    for (int i = 0; i < K; i++) p.op(OP_ADD, true);
+    p.op(OP_MUL, true);
+    p.op(OP_EXP, false);
+    p.op(OP_SIN, false);
+    p.op(OP_MUL, true);
+    p.con();
+    p.con();
+    p.var(0);
+    for (int i = 2; i < K + 2; i++) {
+        if (i < K) {
+            p.op(OP_MUL, true);
+            p.con();
+        }
+        if (i - 2 < v) {
+            p.op(i & 1 ? OP_SIN : OP_COS, false);
+            p.op(OP_SQUARE, false);
+        }
+        p.var(i % D);
+    }
+}
+
+// A population of the general kernel whose plain programs fit the LDS is planned,
+// whatever staging adds to one expression's rows beside another's tape; the
+// planned bytes hold every expression.
+static void check_limit() {
+    const size_t limit = 160 << 10;
+    int at_limit = 0;
+    for (int D : {1, 2, 12, 60})
+        for (int parts : {1, 2, 4, 8})
+            for (int mode = 0; mode < 4; mode++)
+                for (int v : {0, 3, 12})
+                    for (int slack = 0; slack < 6; slack++) {
+                        const bool rev = mode & 1, mixed = mode & 2;
+                        const size_t row = 64 * (mixed ? 4 : 8);
+                        const int sp = parts > CO_MAX_PARTITIONS ? 1 : parts;
+                        const size_t fixed = fit_static_lds(CO_GENERAL_BIN) + kGenJtBytes +
+                                             (sp > 1 ? sp * sums_width(20) * 8 : 0);
+                        Pop p;
+                        sum_with_subtrees(p, 20, v, D);
+                        sum_with_subtrees(p, 17, v / 2, D);
+                        // a chain whose tape takes what is left, down to a slot of slack
+                        p.h.N = 1000;
+                        p.h.n_vars = D;
+                        const int rows0 = D + 1;
+                        const int chain = (int)((limit - fixed) / row) - rows0 - slack;
+                        p.tree();
+                        for (int i = 0; i < chain; i++) p.op(i & 1 ? OP_SIN : OP_COS, false);
+                        p.op(OP_MUL, true);
+                        p.con();
+                        p.var(0);
+                        CHECK(p.decode(1000, D, 20) == CO_OK);
+                        int rows, tape;
+                        plain_lds(p, &rows, &tape);
+                        if (!rev) tape = 0;
+                        size_t was = (size_t)(rows + tape) * row;
+                        if (mixed && was < (size_t)rows * 512) was = (size_t)rows * 512;
+                        was += fixed;
+                        std::vector<LaunchPlan> lp;
+                        const int rc = plan(p, rev, mixed, parts, lp);
+                        CHECK(was > limit || rc == CO_OK);
+                        at_limit += rev && was <= limit && was + 8 * row > limit;
+                        if (rc != CO_OK) continue;
+                        CHECK(lp[0].bin == CO_GENERAL_BIN && lp[0].cnt >= 2);
+                        CHECK(lp[0].lds[0] + fit_static_lds(CO_GENERAL_BIN) <= limit);
+                        for (const ExprDesc &d : p.desc) {
+                            if (!d.gen) continue;   // a chain of at most 255 nodes
+                            const size_t r = rev ? d.rows_rev : d.rows, t = rev ? d.tape : 0;
+                            const size_t need = uni_bytes_of(d, rev, kGenK) + kGenJtBytes;
+                            CHECK(need + (r + t) * row <= lp[0].wave_bytes);
+                            CHECK(!mixed || need + r * 512 <= lp[0].wave_bytes);
+                        }
+                    }
+    CHECK(at_limit > 50);
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
     else if (!strcmp(argv[1], "solve")) check_solve();
     else if (!strcmp(argv[1], "scalars")) check_scalars();
+    else if (!strcmp(argv[1], "limit")) check_limit();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;

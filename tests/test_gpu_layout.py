@@ -66,3 +66,35 @@ def test_constants_alone_in_padded_kernels(co, opts):
         return
     for k in ("status", "loss_init", "loss_final", "iters", "c_final"):
         assert np.array_equal(g[k], o[k], equal_nan=True), k
+
+
+def test_long_tape_beside_staged_expressions(co):
+    """Reverse AD near the LDS limit: a chain whose tape nearly fills it beside an
+    expression whose staged rows and scalars pass its plain program's. Each fits by
+    itself, and so does their launch (areas by their largest each: 164,416 bytes of
+    the 163,840; the plain programs: 161,040)."""
+    rng = np.random.default_rng(3)
+    N = 1000
+    xs = rng.uniform(-1, 1, (N, 1)).astype(np.float32)
+    chain = ([UN] * 260 + [BIN, CONST, VAR],
+             [float(SIN if i % 2 else 15) for i in range(260)] + [float(MUL), 0.0, 0.0],
+             [-1] * 261 + [0, -1], rng.standard_normal(1).astype(np.float32))
+    # 17 constants: sin(c c) x, then c f(x) and c with f in sin, cos, square
+    nt, nv, ci, K = [BIN] * 17 + [BIN, UN, BIN, CONST, CONST, VAR], [float(ADD)] * 17, [], 2
+    nv += [float(MUL), float(SIN), float(MUL), 0.0, 0.0, 0.0]
+    ci = [-1] * 20 + [0, 1, -1]
+    for i in range(15):
+        nt += [BIN, CONST, UN, VAR]
+        nv += [float(MUL), 0.0, float((SIN, 15, 34)[i % 3]), 0.0]
+        ci += [-1, K, -1, -1]
+        K += 1
+    nt += [UN, UN, VAR, VAR]
+    nv += [float(SIN), float(SIN), 0.0, 0.0]
+    ci += [-1, -1, -1, -1]
+    slots = [chain, (nt, nv, ci, (0.3 * rng.standard_normal(K)).astype(np.float32))]
+    pop = popio.build_pop(slots, xs, rng.standard_normal((2, N)).astype(np.float32))
+    print("long tape beside staged rows", flush=True)
+    g = co.optimize_ex(pop, 5, ad_mode=1, partitions=1)
+    o = lm_oracle.fit(pop, max_iter=5, ad_mode=1, partitions=1)
+    for k in ("status", "loss_init", "loss_final", "iters", "c_final"):
+        assert np.array_equal(g[k], o[k], equal_nan=True), k
