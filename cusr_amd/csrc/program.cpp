@@ -436,12 +436,12 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
         recount();
     }
     int mv = 0, nvars = 0, nvr = 0, vslots = 0, cslots = 0, n_c = 0, n_v = 0, tail = 0;
+    int *vroot = s.depth_stack.data();   // roots of the V subtrees
     for (;;) {
         for (int v = 0; v < D; v++) rows[v] = -1;
         mv = nvr = vslots = cslots = n_c = n_v = 0;
         // the variables M reads itself, and the maximal subtrees of operators
         // over constants or variables alone
-        int last_v = -1;
         for (int i = 0; i < n;) {
             if (nt[i] == NODE_VAR) {
                 int &r = rows[(int)nv[i++]];
@@ -458,8 +458,7 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
                 } else {
                     n_v += sn[i].ops;
                     vslots = std::max(vslots, need[i]);
-                    last_v = i;
-                    ++nvr;
+                    vroot[nvr++] = i;
                 }
                 i += size[i];
             }
@@ -478,12 +477,19 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
             recount();
             continue;
         }
-        if (nvr > 0 && tail + std::max(nvars - mv + vslots, cls[0] == 3 ? needm[0] : 0) > budget) {
-            into_m(last_v, last_v + size[last_v]);
-            recount();
-            continue;
+        if (nvr == 0 || tail + std::max(nvars - mv + vslots, cls[0] == 3 ? needm[0] : 0) <= budget)
+            break;
+        // the last V subtrees go to M, one more each time round, but at once as many
+        // as the rows of the values, the variables and V's slots alone refuse: M's
+        // slots then ask for at most need[0] more rounds (one by one, the decode of a
+        // sum of 64,000 sines took 57 s, now 22 ms)
+        int keep = 0;
+        for (int slots = 0; keep < nvr - 1; ++keep) {
+            slots = std::max(slots, need[vroot[keep]]);
+            if (keep + 1 + nvars + slots > budget) break;
         }
-        break;
+        for (int k = keep; k < nvr; ++k) into_m(vroot[k], vroot[k] + size[vroot[k]]);
+        recount();
     }
     // rows: M's variables, V's values, then V's other variables and slots over
     // M's slots

@@ -6,7 +6,8 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <random>
+#include <algorithm>
+#include <chrono>
 #include <vector>
 
 #include "../cusr_amd/csrc/launch_plan.h"
@@ -297,12 +298,46 @@ static void check_limit() {
     CHECK(at_limit > 50);
 }
 
+// Staging is linear in the nodes: a sum of n sines of variables, far more values than
+// the rows hold, and the same over 40 of 100 variables, which M reads itself too.
+static void check_long() {
+    auto seconds = [](Pop &p, int D) {
+        const auto t0 = std::chrono::steady_clock::now();
+        CHECK(p.decode(1024, D, 1) == CO_OK);
+        return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    };
+    for (int D : {1, 100}) {
+        const int used = D == 1 ? 1 : 40;
+        double s[2];
+        for (int big = 0; big < 2; big++) {
+            Pop p;
+            p.tree();
+            const int n = big ? 64000 : 2000;
+            for (int i = 0; i < n; i++) {
+                p.op(OP_ADD, true);
+                p.op(OP_SIN, false);
+                p.var(i % used);
+                if (i % 50 == 49) {
+                    p.op(OP_ADD, true);
+                    p.var(i / 50 % used);
+                }
+            }
+            p.con();
+            s[big] = std::min(seconds(p, D), std::min(seconds(p, D), seconds(p, D)));
+            CHECK(p.desc[0].vrows > 0 && p.desc[0].rows <= std::max(D + 1, 8));
+        }
+        printf("D %d: %.1f ms for 32 times %.2f ms\n", D, 1e3 * s[1], 1e3 * s[0]);
+        CHECK(s[1] < 32 * 5 * s[0] + 0.02);   // quadratic: 1,024 times
+    }
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
     else if (!strcmp(argv[1], "solve")) check_solve();
     else if (!strcmp(argv[1], "scalars")) check_scalars();
     else if (!strcmp(argv[1], "limit")) check_limit();
+    else if (!strcmp(argv[1], "long")) check_long();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;
