@@ -18,6 +18,7 @@
 #include <new>
 #include <vector>
 
+#include "device_buf.h"
 #include "launch_plan.h"
 #include "lm_device.h"
 #define CUSR_SPLIT_STEP_KERNELS
@@ -69,11 +70,6 @@ double now_ms() {
 
 double g_setup_ms = -1.0, g_loop_ms = -1.0;
 
-struct DevBuf {
-    void *p = nullptr;
-    size_t cap = 0;
-};
-
 // Page-locked host staging for the decoded programs (hipHostMalloc), grown
 // with 25 % headroom and never shrunk. Copies to the device from it run at
 // DMA speed; from pageable memory the runtime stages them through buffers of
@@ -86,8 +82,6 @@ struct HostBuf {
     T &operator[](size_t i) { return p[i]; }
     const T &operator[](size_t i) const { return p[i]; }
 };
-
-constexpr int kMaxRanges = 2;   // launch ranges of one fit (the upload pipeline's two)
 
 // launchers per (precision, AD mode) come from fit_kernels.hip, each variant
 // in its own translation unit so the four compile in parallel
@@ -133,11 +127,7 @@ struct Ctx {
     DevBuf prog, desc, X, Y, C0, C, status, li, lf, iters, stage;
     DevBuf data_X, data_Y;   // co_data_upload: X [D][N] column-major, y [N]
     DevBuf state;            // scratch of tail and split fits (run_fit)
-    // workspace of the V values (program.h) per launch range, and its columns
-    // in use: null where the range has none or they would not fit
-    DevBuf vwork[kMaxRanges];
-    void *v_ptr[kMaxRanges] = {};
-    size_t v_max = 0;        // bytes such a workspace may take: an eighth of the device's memory
+    VWork vwork;             // of the V values, per launch range
     void *static_scratch = nullptr;   // this device's address of `scratch`
     HostBuf<uint64_t> h_prog;
     HostBuf<ExprDesc> h_desc;
@@ -157,77 +147,17 @@ struct Ctx {
         }                                                                               \
     } while (0)
 
-int grow(DevBuf &b, size_t bytes) {
-    if (bytes == 0) bytes = 256;
-    if (bytes <= b.cap) return CO_OK;
-    if (b.p) (void)hipFree(b.p);
-    b.p = nullptr;
-    b.cap = 0;
-    hipError_t e = hipMalloc(&b.p, bytes);
-    if (e != hipSuccess) {
-        fprintf(stderr, "[cusr_co] hipMalloc(%zu) failed: %s\n", bytes, hipGetErrorString(e));
-        b.p = nullptr;
-        return (e == hipErrorOutOfMemory) ? CO_ERR_OOM : CO_ERR_CUDA;
-    }
-    b.cap = bytes;
-    return CO_OK;
-}
-
 #define CO_GROW(buf, bytes)                   \
     do {                                      \
         int r_ = grow((buf), (bytes));        \
         if (r_ != CO_OK) return r_;           \
     } while (0)
 
-// The V workspaces given back (a fit then runs V in every pass); true if there
-// were any. hipFree waits for the device.
-bool drop_vwork(Ctx *ctx) {
-    bool any = false;
-    for (int r = 0; r < kMaxRanges; ++r) {
-        if (ctx->vwork[r].p) {
-            (void)hipFree(ctx->vwork[r].p);
-            any = true;
-        }
-        ctx->vwork[r] = DevBuf();
-        ctx->v_ptr[r] = nullptr;
-    }
-    return any;
-}
-
-// grow for what a fit needs: out of memory, it takes the place of the V
-// workspaces, which a fit can do without.
-int grow_needed(Ctx *ctx, DevBuf &b, size_t bytes) {
-    int rc = grow(b, bytes);
-    if (rc == CO_ERR_OOM && drop_vwork(ctx)) rc = grow(b, bytes);
-    return rc;
-}
-
-#define CO_GROW_NEEDED(ctx, buf, bytes)                \
-    do {                                               \
-        int r_ = grow_needed((ctx), (buf), (bytes));   \
-        if (r_ != CO_OK) return r_;                    \
+#define CO_GROW_NEEDED(ctx, buf, bytes)                     \
+    do {                                                    \
+        int r_ = grow_needed((ctx)->vwork, (buf), (bytes)); \
+        if (r_ != CO_OK) return r_;                         \
     } while (0)
-
-// The workspace of range r for `cols` columns of N values of 8 bytes, grown with a quarter of headroom and kept. ctx->v_ptr[r] stays
-// null, and no error is returned, where it would pass v_max or does not fit.
-void set_vwork(Ctx *ctx, int r, int64_t cols, int N) {
-    DevBuf &b = ctx->vwork[r];
-    const size_t bytes = sizeof(double) * (size_t)cols * (size_t)N;
-    ctx->v_ptr[r] = nullptr;
-    if (bytes == 0 || bytes > ctx->v_max) return;
-    if (bytes > b.cap) {
-        if (b.p) (void)hipFree(b.p);
-        b = DevBuf();
-        const size_t want = bytes + bytes / 4;
-        if (hipMalloc(&b.p, want) != hipSuccess) {
-            (void)hipGetLastError();
-            b = DevBuf();
-            return;
-        }
-        b.cap = want;
-    }
-    ctx->v_ptr[r] = b.p;
-}
 
 template <typename T>
 int grow_host(HostBuf<T> &b, size_t n) {
@@ -380,7 +310,7 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
     const size_t words = (size_t)ctx->plan.words;
     rc = grow_buffers(ctx, h, words, in32, on_data, shared_y);
     if (rc != CO_OK) return rc;
-    set_vwork(ctx, 0, ctx->plan.vcols, h->N);
+    ctx->vwork.set(0, ctx->plan.vcols, h->N);
     hipStream_t s = ctx->stream;
     if (words)
         CO_HIP(hipMemcpyAsync(ctx->prog.p, ctx->h_prog.data(), sizeof(uint64_t) * words,
@@ -629,7 +559,7 @@ struct FitRun {
                 fk.rows = b.rows;
                 fk.tape = b.tape;
                 fk.uni_bytes = uni_bytes(b);
-                fk.V = ctx->v_ptr[range];
+                fk.V = ctx->vwork.ptr[range];
                 fk.parts = parts;
                 fk.pwaves = 1;
                 fk.wave_bytes = (int)b.wave_bytes;
@@ -648,7 +578,7 @@ struct FitRun {
                     fk.rows = b.rows;
                     fk.tape = b.tape;
                     fk.uni_bytes = uni_bytes(b);
-                    fk.V = ctx->v_ptr[range];
+                    fk.V = ctx->vwork.ptr[range];
                     fk.parts = seg[g].parts;
                     fk.pwaves = b.pwaves[g];
                     fk.wave_bytes = (int)b.wave_bytes;
@@ -865,7 +795,7 @@ int fit_pipelined(Ctx *ctx, const CoOptions &opt, const PopHeader *h, const int3
 #endif
         rc = decode_range(h, nt, nv, ci, metas, m0, m1, wb, ctx->h_prog.data(),
                           ctx->h_desc.data(), &rp);
-        if (rc == CO_OK) set_vwork(ctx, j, rp.vcols, h->N);
+        if (rc == CO_OK) ctx->vwork.set(j, rp.vcols, h->N);
 #ifdef CUSR_EXP_TIMING
         const double q1 = now_ms();
 #endif
@@ -1000,7 +930,7 @@ extern "C" int co_init(int device_id, void **handle_out) {
         ctx->lds_per_block = lds_per_block > 0 ? (size_t)lds_per_block : 0;
     size_t mem_free = 0, mem_total = 0;
     if (e == hipSuccess) e = hipMemGetInfo(&mem_free, &mem_total);
-    ctx->v_max = mem_total / 8;
+    ctx->vwork.max = mem_total / 8;
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
     for (int i = 0; i < kExtraStreams && e == hipSuccess; ++i)
         e = hipStreamCreateWithFlags(&ctx->lanes[i], hipStreamNonBlocking);
@@ -1393,7 +1323,7 @@ extern "C" void co_teardown(void *handle) {
                       &ctx->data_X, &ctx->data_Y, &ctx->state};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
-    drop_vwork(ctx);
+    ctx->vwork.drop();
     if (ctx->h_prog.p) (void)hipHostFree(ctx->h_prog.p);
     if (ctx->h_desc.p) (void)hipHostFree(ctx->h_desc.p);
     if (ctx->h_stage.p) (void)hipHostFree(ctx->h_stage.p);
