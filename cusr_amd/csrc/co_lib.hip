@@ -170,6 +170,7 @@ int grow_host(HostBuf<T> &b, size_t n) {
     void *q = nullptr;
     hipError_t e = hipHostMalloc(&q, want * sizeof(T), hipHostMallocDefault);
     if (e != hipSuccess) {
+        (void)hipGetLastError();
         fprintf(stderr, "[cusr_co] hipHostMalloc(%zu) failed: %s\n", want * sizeof(T),
                 hipGetErrorString(e));
         return (e == hipErrorOutOfMemory) ? CO_ERR_OOM : CO_ERR_CUDA;

@@ -26,6 +26,7 @@ static inline int grow(DevBuf &b, size_t bytes) {
     b.cap = 0;
     hipError_t e = hipMalloc(&b.p, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // it would stay for the next launch's check
         fprintf(stderr, "[cusr_co] hipMalloc(%zu) failed: %s\n", bytes, hipGetErrorString(e));
         b.p = nullptr;
         return (e == hipErrorOutOfMemory) ? CO_ERR_OOM : CO_ERR_CUDA;
