@@ -147,13 +147,7 @@ struct Ctx {
         }                                                                               \
     } while (0)
 
-#define CO_GROW(buf, bytes)                   \
-    do {                                      \
-        int r_ = grow((buf), (bytes));        \
-        if (r_ != CO_OK) return r_;           \
-    } while (0)
-
-#define CO_GROW_NEEDED(ctx, buf, bytes)                     \
+#define CO_GROW(ctx, buf, bytes)                            \
     do {                                                    \
         int r_ = grow_needed((ctx)->vwork, (buf), (bytes)); \
         if (r_ != CO_OK) return r_;                         \
@@ -203,21 +197,21 @@ int grow_buffers(Ctx *ctx, const PopHeader *h, size_t words, bool in32, bool on_
     // round's) does not free and allocate again (about 1 ms of a C5 round
     // when it did)
     if (sizeof(uint64_t) * words > ctx->prog.cap)
-        CO_GROW_NEEDED(ctx, ctx->prog, sizeof(uint64_t) * (words + words / 4));
-    CO_GROW_NEEDED(ctx, ctx->desc, sizeof(ExprDesc) * M);
-    CO_GROW_NEEDED(ctx, ctx->X, sizeof(double) * nX);
-    CO_GROW_NEEDED(ctx, ctx->Y, sizeof(double) * nY);
+        CO_GROW(ctx, ctx->prog, sizeof(uint64_t) * (words + words / 4));
+    CO_GROW(ctx, ctx->desc, sizeof(ExprDesc) * M);
+    CO_GROW(ctx, ctx->X, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->Y, sizeof(double) * nY);
     const size_t Ch = (size_t)C + (size_t)C / 4;
-    if (sizeof(double) * C > ctx->C0.cap) CO_GROW_NEEDED(ctx, ctx->C0, sizeof(double) * Ch);
-    if (sizeof(double) * C > ctx->C.cap) CO_GROW_NEEDED(ctx, ctx->C, sizeof(double) * Ch);
-    CO_GROW_NEEDED(ctx, ctx->status, sizeof(int32_t) * M);
-    CO_GROW_NEEDED(ctx, ctx->li, sizeof(double) * M);
-    CO_GROW_NEEDED(ctx, ctx->lf, sizeof(double) * M);
-    CO_GROW_NEEDED(ctx, ctx->iters, sizeof(int32_t) * M);
+    if (sizeof(double) * C > ctx->C0.cap) CO_GROW(ctx, ctx->C0, sizeof(double) * Ch);
+    if (sizeof(double) * C > ctx->C.cap) CO_GROW(ctx, ctx->C, sizeof(double) * Ch);
+    CO_GROW(ctx, ctx->status, sizeof(int32_t) * M);
+    CO_GROW(ctx, ctx->li, sizeof(double) * M);
+    CO_GROW(ctx, ctx->lf, sizeof(double) * M);
+    CO_GROW(ctx, ctx->iters, sizeof(int32_t) * M);
     size_t stage = esz * nX;
     if (in32 && esz * nY > stage) stage = esz * nY;
     if (in32 && esz * C > stage) stage = esz * C;
-    if (stage > ctx->stage.cap) CO_GROW_NEEDED(ctx, ctx->stage, stage + stage / 4);
+    if (stage > ctx->stage.cap) CO_GROW(ctx, ctx->stage, stage + stage / 4);
     return CO_OK;
 }
 
@@ -489,7 +483,7 @@ struct FitRun {
         Scratch own;
         if (!sc) {
             if (state_bytes + psum_bytes)
-                CO_GROW_NEEDED(ctx, ctx->state, state_bytes + psum_bytes);
+                CO_GROW(ctx, ctx->state, state_bytes + psum_bytes);
             own.p = ctx->state.p;
             own.cap = ctx->state.cap;
             sc = &own;
@@ -1052,9 +1046,9 @@ extern "C" int co_data_upload(void *handle, int N, int n_vars, const double *xs,
     ctx->data_N = -1;   // no data set until this upload completes
     if (ctx->on_data) ctx->resident = false;
     const size_t nX = (size_t)N * n_vars;
-    CO_GROW(ctx->data_X, sizeof(double) * nX);
-    CO_GROW(ctx->data_Y, sizeof(double) * N);
-    CO_GROW(ctx->stage, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->data_X, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->data_Y, sizeof(double) * N);
+    CO_GROW(ctx, ctx->stage, sizeof(double) * nX);
     hipStream_t s = ctx->stream;
     if (nX) {
         CO_HIP(hipMemcpyAsync(ctx->stage.p, xs, 8 * nX, hipMemcpyHostToDevice, s));
@@ -1106,8 +1100,8 @@ extern "C" int co_data_upload_device(void *handle, int N, int n_vars, const doub
     ctx->data_N = -1;   // no data set until this upload completes
     if (ctx->on_data) ctx->resident = false;
     const size_t nX = (size_t)N * n_vars;
-    CO_GROW(ctx->data_X, sizeof(double) * nX);
-    CO_GROW(ctx->data_Y, sizeof(double) * N);
+    CO_GROW(ctx, ctx->data_X, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->data_Y, sizeof(double) * N);
     hipStream_t s = ctx->stream;
     if (nX) {
         // row-major [N][D] straight from the caller's memory to column-major
@@ -1195,12 +1189,12 @@ extern "C" int co_eval_ex(void *handle, const PopHeader *h, const int32_t *nt, c
     const int uni = (eval_uni_doubles(plan) * (int)sizeof(double) + 15) & ~15;
     const size_t lds = uni + (size_t)plan.max_rows * kLanes * (precision == CO_PREC_FP64 ? 8 : 4);
     if (lds + sizeof(double) * CO_MAX_K > ctx->lds_per_block) return CO_ERR_BOUNDS;
-    CO_GROW(ctx->prog, sizeof(uint64_t) * words);
-    CO_GROW(ctx->desc, sizeof(ExprDesc) * M);
-    CO_GROW(ctx->X, sizeof(double) * nX);
-    CO_GROW(ctx->Y, sizeof(double) * nY);
-    CO_GROW(ctx->C0, sizeof(double) * C);
-    CO_GROW(ctx->stage, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->prog, sizeof(uint64_t) * words);
+    CO_GROW(ctx, ctx->desc, sizeof(ExprDesc) * M);
+    CO_GROW(ctx, ctx->X, sizeof(double) * nX);
+    CO_GROW(ctx, ctx->Y, sizeof(double) * nY);
+    CO_GROW(ctx, ctx->C0, sizeof(double) * C);
+    CO_GROW(ctx, ctx->stage, sizeof(double) * nX);
     hipStream_t s = ctx->stream;
     if (words)
         CO_HIP(hipMemcpyAsync(ctx->prog.p, ctx->h_prog.data(), sizeof(uint64_t) * words,

@@ -1,5 +1,5 @@
 """The library's device buffers when memory runs out (tests/device_buf_check.hip,
-compiled for the host with an allocator of its own)."""
+compiled for the host with a runtime of its own)."""
 import shutil
 import subprocess
 from pathlib import Path
@@ -18,12 +18,14 @@ def exe(tmp_path_factory):
     subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-Wall",
                     "-Wno-unused-function", "-Xclang", "-target-feature", "-Xclang",
                     "-packed-fp32-ops", f"-I{REPO / 'include'}",
-                    str(REPO / "tests" / "device_buf_check.hip"), "-o", str(out)],
+                    str(REPO / "tests" / "device_buf_check.hip"),
+                    str(REPO / "cusr_amd" / "csrc" / "program.cpp"), "-pthread",
+                    "-Wl,--unresolved-symbols=ignore-all", "-o", str(out)],
                    check=True, capture_output=True, timeout=300)
     return out
 
 
-@pytest.mark.parametrize("what", ["error"])
+@pytest.mark.parametrize("what", ["error", "room"])
 def test_device_buffers(exe, what):
     r = subprocess.run([str(exe), what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "device buffers ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
