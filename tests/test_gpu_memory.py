@@ -1,4 +1,5 @@
-"""A handle when device memory runs out: an allocation is refused, nothing else."""
+"""A handle when device memory runs out (an allocation is refused, nothing else), and
+fits whose V workspace passes the limit."""
 import ctypes
 
 import numpy as np
@@ -11,13 +12,28 @@ from tests.helpers import f64
 
 pytestmark = pytest.mark.gpu
 
+KEYS = ("c_final", "status", "loss_init", "loss_final", "iters")
 VAR, CONST, UN, BIN = popio.NODE_VAR, popio.NODE_CONST, popio.NODE_UFUNC, popio.NODE_BFUNC
 ADD, MUL, SIN = 1, 3, 14
-N = 100_000
+N = 1_000_000
 
 
 def _say(msg):
     print(f"[memory] {msg}", flush=True)
+
+
+def _hip():
+    """The HIP runtime that the library runs on."""
+    with open("/proc/self/maps") as f:
+        paths = {line.split()[-1] for line in f if "libamdhip64" in line}
+    assert len(paths) == 1, paths
+    return ctypes.CDLL(paths.pop())
+
+
+def _memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value, total.value
 
 
 def _pop(copies):
@@ -57,3 +73,23 @@ def test_call_after_a_refused_allocation(own):
     assert rc == ci.CO_ERR_OOM
     c0, x64, _ = f64(one)
     assert np.array_equal(own.evaluate(one, c0, x64), lm_oracle.eval_pop(one, c=c0, xs=x64))
+
+
+@pytest.mark.parametrize("opts", [dict(), dict(partitions=2), dict(ad_mode=1),
+                                  dict(precision=1), dict(precision=1, partitions=4),
+                                  dict(ad_mode=1, precision=1)])
+def test_fits_without_workspaces(own, opts):
+    """V run in every pass gives the bits that its kept values give: four expressions
+    whose columns take 96 MB, and 500 copies whose columns would take 48 GB."""
+    _, few = _pop(1)
+    _, many = _pop(500)
+    own.upload_data(*f64(many)[1:])
+    kept = own.optimize_data(few, 4, **opts)
+    free, total = _memory()
+    assert 8 * 3 * N * many["M"] > total // 8
+    _say(f"fit without workspaces {opts}")
+    run = own.optimize_data(many, 4, **opts)
+    assert free - _memory()[0] < 4 << 30
+    for k in KEYS:
+        assert np.array_equal(run[k].reshape(500, -1), np.tile(kept[k], (500, 1)),
+                              equal_nan=True), k
