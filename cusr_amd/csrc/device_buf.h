@@ -40,7 +40,7 @@ static inline int grow(DevBuf &b, size_t bytes) {
 struct VWork {
     DevBuf buf[kMaxRanges];
     void *ptr[kMaxRanges] = {};
-    size_t max = 0;   // bytes such a workspace may take: an eighth of the device's memory
+    size_t max = 0;   // bytes that each may take: an eighth of the device's memory
 
     // The workspaces given back (a fit then runs V in every pass); true if there
     // were any. hipFree waits for the device.
@@ -58,8 +58,8 @@ struct VWork {
     }
 
     // The workspace of range r for `cols` columns of N values of 8 bytes, grown with
-    // a quarter of headroom and kept. ptr[r] stays null, and no error is returned,
-    // where it would pass max or does not fit.
+    // a quarter of headroom (to max) and kept. ptr[r] stays null, and no error is
+    // returned, where it would pass max or does not fit.
     void set(int r, int64_t cols, int N) {
         DevBuf &b = buf[r];
         const size_t bytes = sizeof(double) * (size_t)cols * (size_t)N;
@@ -68,7 +68,7 @@ struct VWork {
         if (bytes > b.cap) {
             if (b.p) (void)hipFree(b.p);
             b = DevBuf();
-            const size_t want = bytes + bytes / 4;
+            const size_t want = bytes + bytes / 4 < max ? bytes + bytes / 4 : max;
             if (hipMalloc(&b.p, want) != hipSuccess) {
                 (void)hipGetLastError();
                 b = DevBuf();

@@ -215,10 +215,27 @@ static void check_error() {
     CHECK(g_live.empty());
 }
 
+// A workspace and its headroom stay within the limit.
+static void check_bound() {
+    g_size = 100000;
+    VWork v;
+    v.max = 4000;
+    for (int cols : {10, 100, 350, 400, 420, 500, 501, 3}) {
+        for (int r = 0; r < kMaxRanges; r++) {
+            v.set(r, cols, 1);
+            CHECK((v.ptr[r] != nullptr) == (8 * cols <= 4000));
+            if (v.ptr[r]) CHECK(v.buf[r].cap >= 8u * cols);
+        }
+        CHECK(g_used <= kMaxRanges * v.max);
+    }
+    CHECK(v.drop() && g_live.empty() && !v.drop());
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "error")) check_error();
     else if (!strcmp(argv[1], "room")) check_room();
+    else if (!strcmp(argv[1], "bound")) check_bound();
     else CHECK(!"check's name");
     puts("device buffers ok");
     return 0;

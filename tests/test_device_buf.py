@@ -25,7 +25,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("what", ["error", "room"])
+@pytest.mark.parametrize("what", ["error", "room", "bound"])
 def test_device_buffers(exe, what):
     r = subprocess.run([str(exe), what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "device buffers ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
