@@ -147,6 +147,55 @@ struct StagedNode {
     uint8_t prog, live;
 };
 
+// Sets of an expression's nodes, a bit each, in words of 64: the staging goes
+// through them instead of through the nodes, whose types and classes a branch
+// predictor cannot follow (its share of the decode of 60,000 expressions of 27
+// nodes, one thread: 32 -> 15 of 107 ms).
+struct NodeSets {
+    std::vector<uint64_t> bits;
+    int words = 0;
+    uint64_t *var, *op, *m;           // variable leaves, operators, M's operators
+    uint64_t *mvar, *vroot, *croot;   // variables M reads, the maximal V and C subtrees
+    void reserve(int n) { bits.resize(6 * (size_t)((n + 63) / 64)); }
+    void clear(int n) {
+        words = (n + 63) / 64;
+        uint64_t **const sets[6] = {&var, &op, &m, &mvar, &vroot, &croot};
+        for (int k = 0; k < 6; k++) *sets[k] = bits.data() + (size_t)k * words;
+        memset(bits.data(), 0, sizeof(uint64_t) * 6 * words);
+    }
+    static void mark(uint64_t *set, int i, bool on) { set[i >> 6] |= (uint64_t)on << (i & 63); }
+    // fn(i) for the members, ascending, until it returns false
+    template <typename Fn>
+    static void each(const uint64_t *set, int words, const uint64_t *but, const Fn &fn) {
+        for (int w = 0; w < words; w++)
+            for (uint64_t b = but ? set[w] & ~but[w] : set[w]; b; b &= b - 1)
+                if (!fn(w * 64 + __builtin_ctzll(b))) return;
+    }
+    // the operators of [i, end) go to M, and their variables
+    void to_m(int i, int end) {
+        for (int w = i >> 6; w < words && w * 64 < end; w++) {
+            uint64_t r = ~(uint64_t)0;
+            if (w * 64 < i) r &= ~(uint64_t)0 << (i & 63);
+            if (end - w * 64 < 64) r &= ~(~(uint64_t)0 << (end - w * 64));
+            m[w] |= op[w] & r;
+            mvar[w] |= var[w] & r;
+            vroot[w] &= ~r;
+            croot[w] &= ~r;
+        }
+    }
+};
+
+// The largest rows, constants beside a C program and scalar slots of the
+// expressions emitted (Plan).
+struct Most {
+    int rows = 0, ck = 0, cslots = 0;
+    void add(const Most &o) {
+        rows = std::max(rows, o.rows);
+        ck = std::max(ck, o.ck);
+        cslots = std::max(cslots, o.cslots);
+    }
+};
+
 // Per-thread working arrays, grown to the largest expression seen and not
 // cleared between expressions (every entry read is written first).
 struct TreeScratch {
@@ -155,6 +204,8 @@ struct TreeScratch {
     // M; and what the emission hands down
     std::vector<int> cls, needm;
     std::vector<StagedNode> st;
+    NodeSets set;
+    Most most;
     int rows[CO_MAX_VARS + 1];
     std::vector<Operand> res;
     std::vector<Visit> work;
@@ -163,6 +214,7 @@ struct TreeScratch {
         cls.resize(n + 1);
         needm.resize(n + 1);
         st.resize(n + 1);
+        set.reserve(n);
         size.resize(n + 1);
         left.resize(n + 1);
         cc.resize(n + 1);
@@ -179,7 +231,7 @@ static inline bool is_leaf(int t) { return t == NODE_VAR || t == NODE_CONST; }
 // operator ids, variable indices, prefix-order constant ranks and stack moves.
 // Returns CO_OK, CO_ERR_BOUNDS (value stack beyond CO_MAX_STACK) or
 // CO_ERR_PROGRAM, and its value-stack depth. Fills s.size / s.left / s.cc / s.cls,
-// s.needm, the counts of s.st and s.need (the spill slots of each subtree in the
+// s.needm, s.set, the counts of s.st and s.need (the spill slots of each subtree in the
 // emission's order) for the emission. stage_c: operators over constants alone
 // are class 2, to go to C; else class 3, to stay in M.
 static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int n, int K,
@@ -189,6 +241,8 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
     int *size = s.size.data(), *left = s.left.data(), *cc = s.cc.data(), *need = s.need.data();
     int *st = s.depth_stack.data(), *cls = s.cls.data(), *needm = s.needm.data();
     StagedNode *sn = s.st.data();
+    NodeSets &set = s.set;
+    set.clear(n);
     // prefix pass: constant ranks must be 0..K-1 in prefix order
     cc[0] = 0;
     for (int i = 0; i < n; i++) {
@@ -205,6 +259,7 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
         if (t == NODE_VAR || t == NODE_CONST) {
             if (t == NODE_VAR && node_int(nv[i], D) < 0) return CO_ERR_PROGRAM;
             cls[i] = t == NODE_VAR ? 1 : 2;
+            NodeSets::mark(set.var, i, t == NODE_VAR);
             size[i] = 1;
             need[i] = needm[i] = 0;
             sn[i].ops = sn[i].mops = 0;
@@ -219,6 +274,8 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
             needm[i] = cls[c] == 3 ? needm[c] : 0;
             sn[i].ops = sn[c].ops + 1;
             sn[i].mops = cls[c] == 3 ? sn[c].mops + 1 : 1;
+            NodeSets::mark(set.op, i, true);
+            NodeSets::mark(set.m, i, cls[i] == 3);
             st[sp - 1] = i;
         } else if (t == NODE_BFUNC) {
             if (!binary_op(node_int(nv[i], 64))) return CO_ERR_PROGRAM;
@@ -240,6 +297,15 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
             needm[i] = (ml && mr && a == b) ? a + 1 : (a > b ? a : b);
             sn[i].ops = sn[l].ops + sn[r].ops + 1;
             sn[i].mops = (ml ? sn[l].mops : 0) + (mr ? sn[r].mops : 0) + 1;
+            NodeSets::mark(set.op, i, true);
+            const bool m = cls[i] == 3;
+            NodeSets::mark(set.m, i, m);
+            for (int c : {l, r}) {
+                const bool leaf = sn[c].ops == 0;
+                NodeSets::mark(set.mvar, c, m & leaf & (cls[c] == 1));
+                NodeSets::mark(set.vroot, c, m & !leaf & (cls[c] == 1));
+                NodeSets::mark(set.croot, c, m & !leaf & (cls[c] == 2));
+            }
             st[sp - 1] = i;
         } else {
             return CO_ERR_PROGRAM;
@@ -247,6 +313,9 @@ static int check_tree(const int32_t *nt, const float *nv, const int32_t *ci, int
         if (sp > depth) depth = sp;
     }
     if (sp != 1) return CO_ERR_PROGRAM;
+    NodeSets::mark(set.mvar, 0, is_leaf(nt[0]) && cls[0] == 1);
+    NodeSets::mark(set.vroot, 0, !is_leaf(nt[0]) && cls[0] == 1);
+    NodeSets::mark(set.croot, 0, !is_leaf(nt[0]) && cls[0] == 2);
     *stack_depth = depth;
     if (depth > CO_MAX_STACK) return CO_ERR_BOUNDS;
     return CO_OK;
@@ -410,6 +479,7 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
               *need = s.need.data();
     int *cls = s.cls.data(), *needm = s.needm.data(), *rows = s.rows;
     StagedNode *sn = s.st.data();
+    NodeSets &set = s.set;
     int vars[CO_MAX_VARS + 1];         // variable rows: M's, then V's others
     const int plain_rows = D + need[0];
     const int budget = std::min(wide ? 4096 : kFastRows,
@@ -417,64 +487,61 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
     bool stage = staged && K > 0;
     // class 3 to every operator of [i, end), so that it stays in M
     auto into_m = [&](int i, int end) {
-        for (; i < end; ++i)
-            if (!is_leaf(nt[i])) cls[i] = 3;
+        set.to_m(i, end);
+        for (; i < end; ++i) cls[i] = sn[i].ops > 0 ? 3 : cls[i];
     };
-    // slots and operators of M after such a change, last node first
-    auto recount = [&] {
-        for (int i = n - 1; i >= 0; i--) {
-            if (is_leaf(nt[i]) || cls[i] != 3) continue;
-            const int l = i + 1, r = nt[i] == NODE_BFUNC ? l + left[i] : -1;
-            const bool ml = cls[l] == 3, mr = r >= 0 && cls[r] == 3;
-            const int a = ml ? needm[l] : 0, b = mr ? needm[r] : 0;
-            needm[i] = ml && mr && a == b ? a + 1 : std::max(a, b);
-            sn[i].mops = (ml ? sn[l].mops : 0) + (mr ? sn[r].mops : 0) + 1;
-        }
+    // slots and operators of M after such changes below end, last node first
+    auto recount = [&](int end) {
+        for (int w = (end - 1) >> 6; w >= 0; w--)
+            for (uint64_t b = set.m[w]; b;) {
+                const int k = 63 - __builtin_clzll(b), i = w * 64 + k;
+                b ^= (uint64_t)1 << k;
+                const bool bin = nt[i] == NODE_BFUNC;
+                const int l = i + 1, r = bin ? l + left[i] : l;
+                const bool ml = cls[l] == 3, mr = bin && cls[r] == 3;
+                const int x = ml ? needm[l] : 0, y = mr ? needm[r] : 0;
+                needm[i] = ml && mr && x == y ? x + 1 : std::max(x, y);
+                sn[i].mops = (ml ? sn[l].mops : 0) + (mr ? sn[r].mops : 0) + 1;
+            }
     };
     if (!stage) {
         into_m(0, n);
-        recount();
+        recount(n);
     }
     int mv = 0, nvars = 0, nvr = 0, vslots = 0, cslots = 0, n_c = 0, n_v = 0, tail = 0;
     int *vroot = s.depth_stack.data();   // roots of the V subtrees
+    const auto row = [&](int i) {
+        int &r = rows[(int)nv[i]];
+        if (r < 0) {
+            vars[nvars] = (int)nv[i];
+            r = nvars++;
+        }
+        return nvars < D;   // until every variable has its row
+    };
     for (;;) {
         for (int v = 0; v < D; v++) rows[v] = -1;
-        mv = nvr = vslots = cslots = n_c = n_v = 0;
+        nvars = nvr = vslots = cslots = n_c = n_v = 0;
         // the variables M reads itself, and the maximal subtrees of operators
         // over constants or variables alone
-        for (int i = 0; i < n;) {
-            if (nt[i] == NODE_VAR) {
-                int &r = rows[(int)nv[i++]];
-                if (r < 0) {
-                    vars[mv] = (int)nv[i - 1];
-                    r = mv++;
-                }
-            } else if (cls[i] == 3 || nt[i] == NODE_CONST) {
-                ++i;
-            } else {
-                if (cls[i] == 2) {
-                    n_c += sn[i].ops;
-                    cslots = std::max(cslots, need[i]);
-                } else {
-                    n_v += sn[i].ops;
-                    vslots = std::max(vslots, need[i]);
-                    vroot[nvr++] = i;
-                }
-                i += size[i];
-            }
-        }
-        nvars = mv;
-        if (nvr > 0 && mv < D)
-            for (int i = 0; i < n; i++)
-                if (nt[i] == NODE_VAR && rows[(int)nv[i]] < 0) {
-                    vars[nvars] = (int)nv[i];
-                    rows[(int)nv[i]] = nvars++;
-                }
+        NodeSets::each(set.mvar, set.words, nullptr, row);
+        mv = nvars;
+        NodeSets::each(set.croot, set.words, nullptr, [&](int i) {
+            n_c += sn[i].ops;
+            cslots = std::max(cslots, need[i]);
+            return true;
+        });
+        NodeSets::each(set.vroot, set.words, nullptr, [&](int i) {
+            n_v += sn[i].ops;
+            vslots = std::max(vslots, need[i]);
+            vroot[nvr++] = i;
+            return true;
+        });
+        if (nvr > 0 && mv < D) NodeSets::each(set.var, set.words, set.mvar, row);
         tail = mv + nvr;
         if (stage && (n_c > kWideCidxMax || (wide && nvars > kStageVarsMax))) {
             stage = false;
             into_m(0, n);
-            recount();
+            recount(n);
             continue;
         }
         if (nvr == 0 || tail + std::max(nvars - mv + vslots, cls[0] == 3 ? needm[0] : 0) <= budget)
@@ -489,7 +556,7 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
             if (keep + 1 + nvars + slots > budget) break;
         }
         for (int k = keep; k < nvr; ++k) into_m(vroot[k], vroot[k] + size[vroot[k]]);
-        recount();
+        recount(vroot[nvr - 1] + size[vroot[nvr - 1]]);
     }
     // rows: M's variables, V's values, then V's other variables and slots over
     // M's slots
@@ -555,8 +622,7 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
         sn[0].live = 0;
         sn[0].dest = -1;
     }
-    for (int i = 0; i < n; i++) {
-        if (is_leaf(nt[i])) continue;
+    NodeSets::each(set.op, set.words, nullptr, [&](int i) {
         const StagedNode t = sn[i];
         const bool bin = nt[i] == NODE_BFUNC;
         const int l = i + 1, r = bin ? l + left[i] : l;
@@ -609,7 +675,8 @@ static int emit_staged(const int32_t *nt, const float *nv, const int32_t *ci, in
         w.root = c_root || a.cidx >= 0 || b.cidx >= 0;
         w.cidx = c_root ? t.ops : a.cidx >= 0 ? a.cidx : b.cidx >= 0 ? b.cidx : 0;
         put(t.prog, k, w, t.dest);
-    }
+        return true;
+    });
     if (!wide && tape[M] > 255) return CO_ERR_BOUNDS;   // never: n <= 255 keeps it below
     d.map = 0;
     if (wide) {
@@ -738,12 +805,12 @@ class DecodePool {
     const pid_t pid_;
 };
 
-// Runs fn(m0, m1) over nthreads contiguous chunks of [0, M) on the decode
-// pool and this thread; without the pool, redo(0, M) runs on this thread.
+// Runs fn(m0, m1) over so many contiguous pieces of [0, M) on the decode pool and
+// this thread; without the pool, redo(0, M) runs on this thread.
 template <typename Fn, typename Redo>
-static void chunked(int M, int nthreads, const Fn &fn, const Redo &redo) {
-    if (nthreads > 1 && M > 0) {
-        const int chunk = (M + nthreads - 1) / nthreads;
+static void chunked(int M, int pieces, const Fn &fn, const Redo &redo) {
+    if (pieces > 1 && M > 0) {
+        const int chunk = (M + pieces - 1) / pieces;
         const int n = (M + chunk - 1) / chunk;
         const std::function<void(int)> job = [&](int i) {
             fn(i * chunk, std::min(M, (i + 1) * chunk));
@@ -783,16 +850,18 @@ static int64_t program_words(int n_nodes, bool wide, bool staged) {
 struct Layout {
     std::vector<int32_t> depth, gen, poff, rcs;
     int64_t words = 0;
-    int n_gen = 0, nthreads = 1;
+    int n_gen = 0, pieces = 1;   // pieces that the pool's threads take
+    std::mutex mu;   // over most, which the ranges of emit_all add to
+    Most most;
 };
 
 static int lay_out(const PopHeader *h, const int32_t *nt, const TreeMeta *metas, int M,
                    bool staged, Layout &lo) {
     const int D = h->n_vars;
     long nsum = 0;
-    for (int m = 0; m < M; m++) nsum += metas[m].n_nodes;
     for (int m = 0; m < M; m++) {
         const TreeMeta &t = metas[m];
+        nsum += t.n_nodes;
         if (t.K < 0 || t.n_nodes < 0 || t.node_offset < 0 || t.c_offset < 0 ||
             (long)t.node_offset + t.n_nodes > (long)h->total_nodes ||
             (long)t.c_offset + t.K > (long)h->total_c)
@@ -801,15 +870,25 @@ static int lay_out(const PopHeader *h, const int32_t *nt, const TreeMeta *metas,
     }
     lo.words = 0;
     lo.n_gen = 0;
+    lo.most = Most();
     lo.depth.resize(M);
     lo.gen.resize(M);
     lo.poff.resize(M);
     lo.rcs.assign(M, CO_OK);
     const unsigned hw = std::max(1u, std::thread::hardware_concurrency());
-    lo.nthreads = (int)std::min<int64_t>(std::min(16u, hw), nsum / kDecodeNodes + 1);
+    // four pieces a thread, so that none waits for the slowest (with the shallow trees
+    // not counted and the launch order by key, calls of one iteration on 60,000
+    // expressions x 300 of 12, 20 and 27 nodes: 4.4 -> 3.8, 6.3 -> 5.6, 8.1 -> 6.7 ms)
+    lo.pieces = (int)std::min<int64_t>(4 * std::min(16u, hw), nsum / kDecodeNodes + 1);
+    // a valid tree of n nodes stacks at most (n + 1) / 2 values: below twice the fast
+    // kernels' depth the count decides nothing
+    const auto shallow = [&](const TreeMeta &t) {
+        return staged && t.n_nodes < 2 * CO_FAST_MAX_STACK;
+    };
     auto depth_range = [&](int m0, int m1) {
         for (int m = m0; m < m1; m++) {
             const TreeMeta &t = metas[m];
+            if (shallow(t)) continue;
             const int32_t *tnt = nt + t.node_offset;
             int sp = 0, dmax = 0;
             for (int i = t.n_nodes - 1; i >= 0; i--) {
@@ -821,7 +900,15 @@ static int lay_out(const PopHeader *h, const int32_t *nt, const TreeMeta *metas,
             lo.gen[m] = co_fast_path(t.K, dmax, t.n_nodes, D) ? 0 : 1;
         }
     };
-    chunked(M, lo.nthreads, depth_range, depth_range);
+    int count = 0;
+    for (int m = 0; m < M; m++)
+        if (shallow(metas[m])) {
+            lo.depth[m] = -1;
+            lo.gen[m] = co_fast_path(metas[m].K, 0, metas[m].n_nodes, D) ? 0 : 1;
+        } else {
+            ++count;
+        }
+    if (count) chunked(M, lo.pieces, depth_range, depth_range);
     for (int m = 0; m < M; m++) {
         lo.poff[m] = (int32_t)lo.words;
         lo.words += program_words(metas[m].n_nodes, lo.gen[m] != 0, staged);
@@ -846,17 +933,19 @@ static int emit_all(const int32_t *nt, const float *nv, const int32_t *ci, const
             int dd = 0;
             int rc = check_tree(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset,
                                 t.n_nodes, t.K, D, stage_c, &dd, s);
-            if (rc == CO_OK && dd != lo.depth[m]) rc = CO_ERR_PROGRAM;   // never, for a valid tree
+            if (rc == CO_OK && lo.depth[m] >= 0 && dd != lo.depth[m]) rc = CO_ERR_PROGRAM;   // never, for a valid tree
             if (rc == CO_OK) rc = emit(m, out, s);
             lo.rcs[m] = rc;
             if (rc != CO_OK) return;
         }
+        std::lock_guard<std::mutex> g(lo.mu);
+        lo.most.add(s.most);
     };
     auto redo = [&](int m0, int m1) {
         std::fill(lo.rcs.begin(), lo.rcs.end(), CO_OK);
         range(m0, m1);
     };
-    chunked(M, lo.nthreads, range, redo);
+    chunked(M, lo.pieces, range, redo);
     for (int m = 0; m < M; m++)
         if (lo.rcs[m] != CO_OK) return lo.rcs[m];
     return CO_OK;
@@ -905,13 +994,28 @@ int decode_population(const PopHeader *h, const int32_t *nt, const float *nv,
     return CO_OK;
 }
 
-// The arrays of decode_range.
+// The arrays of decode_range: descriptors by expression, and what their order and
+// columns follow from, apart from them (a descriptor is 80 bytes, in another core's
+// cache).
 struct RangeScratch {
     Layout lo;
     std::vector<ExprDesc> desc;
-    std::vector<int64_t> cost;
-    std::vector<int32_t> start, ord, a, launch;
+    std::vector<uint32_t> key;
+    std::vector<int32_t> vrows, v_col, launch;
+    std::vector<uint64_t> a;
 };
+
+// Launch order by a key that sorts ascending: the general kernel's bin first, then
+// the fast K bins, largest K first; within a bin by K descending (the general bin)
+// and the costliest programs first (clamped to kCostBuckets).
+constexpr int kCostBits = 15, kCostBuckets = 1 << kCostBits;
+constexpr int kKeyBits = 1 + 6 + kCostBits, kHalfBits = kKeyBits / 2;
+static_assert(CO_MAX_K < 64 && kKeyBits == 2 * kHalfBits, "two digits of the launch key");
+static uint32_t launch_key(bool gen, int K, int64_t cost) {
+    const uint32_t c = (uint32_t)std::min<int64_t>(cost, kCostBuckets - 1);
+    return (uint32_t)!gen << (6 + kCostBits) | (uint32_t)(CO_MAX_K - K) << kCostBits |
+           (kCostBuckets - 1 - c);
+}
 
 int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const int32_t *ci,
                  const TreeMeta *all_metas, int m0, int m1, int64_t word_base, uint64_t *all_prog,
@@ -926,10 +1030,19 @@ int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const i
     Layout &lo = rs.lo;
     int rc = lay_out(h, nt, metas, M, true, lo);
     if (rc != CO_OK) return rc;
-    if ((int)rs.desc.size() < M) rs.desc.resize(M);
-    if ((int)rs.cost.size() < M) rs.cost.resize(M);
+    if ((int)rs.desc.size() < M) {
+        rs.desc.resize(M);
+        rs.key.resize(M);
+        rs.vrows.resize(M);
+        rs.v_col.resize(M);
+        rs.launch.resize(M);
+        rs.a.resize(M);
+    }
+    // by pointer: on another thread `rs` names that thread's own
     ExprDesc *desc = rs.desc.data();
-    int64_t *cost = rs.cost.data();
+    uint32_t *key = rs.key.data();
+    int32_t *vrows = rs.vrows.data(), *v_col = rs.v_col.data(), *launch = rs.launch.data();
+    uint64_t *a = rs.a.data();
     rc = emit_all(nt, nv, ci, metas, M, D, true, stage_constants(h->N), prog, lo,
                   [&](int m, uint64_t *out, TreeScratch &s) {
         const TreeMeta &t = metas[m];
@@ -938,63 +1051,48 @@ int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const i
         d.c_off = t.c_offset;
         d.y_row = m0 + m;
         d.gen = lo.gen[m];
-        return emit_staged(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset, t.n_nodes,
-                           t.K, D, h->N, lo.gen[m] != 0, true, out, d, &cost[m], s);
+        int64_t cost = 0;
+        const int e = emit_staged(nt + t.node_offset, nv + t.node_offset, ci + t.node_offset,
+                                  t.n_nodes, t.K, D, h->N, lo.gen[m] != 0, true, out, d, &cost, s);
+        key[m] = launch_key(d.gen, t.K, cost);
+        vrows[m] = d.vrows;
+        s.most.add({d.rows, d.n_c > 0 ? d.K : 0, d.cslots});
+        return e;
     });
     if (rc != CO_OK) return rc;
-    int max_rows = 0, max_ck = 0, max_cslots = 0;
+    // Columns by expression, and the launch order: two stable counting sorts from
+    // the last expression on, by the lower and the upper half of the key.
     int64_t vcols = 0;
+    int32_t next[2][(1 << kHalfBits) + 1] = {};
+    constexpr uint32_t kHalf = (1u << kHalfBits) - 1;
     for (int m = 0; m < M; m++) {
-        ExprDesc &d = desc[m];
-        if (d.rows > max_rows) max_rows = d.rows;
-        if (d.n_c > 0 && d.K > max_ck) max_ck = d.K;
-        if (d.cslots > max_cslots) max_cslots = d.cslots;
-        d.v_col = (int32_t)vcols;
-        vcols += d.vrows;
+        v_col[m] = (int32_t)vcols;
+        vcols += vrows[m];
+        next[0][(key[m] & kHalf) + 1]++;
+        next[1][(key[m] >> kHalfBits) + 1]++;
     }
-    std::vector<int32_t> &start = rs.start, &ord = rs.ord;
-    k_bins(metas, M, start, ord);
-    {
-        // launch positions: the general kernel's bin first, then the fast K
-        // bins, largest K first; within a bin by K descending (the general
-        // bin) and the costliest programs first (fixed per-pass cost plus
-        // op_cost of each instruction), so the longest-running workgroups
-        // start earliest and a bin ends on cheap ones. Three stable counting
-        // sorts over reversed ord: by cost descending (clamped to
-        // kCostBuckets), by K descending, by kernel (general first); ties keep
-        // the order of ord reversed
-        constexpr int kCostBuckets = 1 << 15;
-        std::vector<int32_t> &a = rs.a, &launch = rs.launch;
-        a.resize(M);
-        launch.resize(M);
-        for (int p = 0; p < M; p++) a[p] = ord[M - 1 - p];
-        std::vector<int32_t> next(kCostBuckets + 1, 0);
-        auto bucket = [&](int32_t m) {
-            const int64_t c = cost[m] < kCostBuckets - 1 ? cost[m] : kCostBuckets - 1;
-            return (int)(kCostBuckets - 1 - c);
-        };
-        for (int p = 0; p < M; p++) next[bucket(a[p]) + 1]++;
-        for (int i = 0; i < kCostBuckets; i++) next[i + 1] += next[i];
-        for (int p = 0; p < M; p++) launch[next[bucket(a[p])]++] = a[p];
-        std::vector<int32_t> knext(CO_MAX_K + 2, 0);
-        for (int p = 0; p < M; p++) knext[CO_MAX_K - metas[launch[p]].K + 1]++;
-        for (int i = 0; i <= CO_MAX_K; i++) knext[i + 1] += knext[i];
-        for (int p = 0; p < M; p++) a[knext[CO_MAX_K - metas[launch[p]].K]++] = launch[p];
-        int gpos = 0, fpos = lo.n_gen;
-        for (int p = 0; p < M; p++) launch[lo.gen[a[p]] ? gpos++ : fpos++] = a[p];
-        const auto put = [&](int p0, int p1) {
-            for (int p = p0; p < p1; p++) descs[p] = desc[launch[p]];
-        };
-        chunked(M, M >= 4096 ? lo.nthreads : 1, put, put);
-    }
+    for (uint32_t i = 0; i < kHalf; i++)
+        for (int d = 0; d < 2; d++) next[d][i + 1] += next[d][i];
+    for (int m = M - 1; m >= 0; m--)
+        a[next[0][key[m] & kHalf]++] = (uint64_t)key[m] << 32 | (uint32_t)m;
+    for (int p = 0; p < M; p++)
+        launch[next[1][a[p] >> (32 + kHalfBits)]++] = (int32_t)a[p];
+    const auto put = [&](int p0, int p1) {
+        for (int p = p0; p < p1; p++) {
+            const int m = launch[p];
+            descs[p] = desc[m];
+            descs[p].v_col = v_col[m];
+        }
+    };
+    chunked(M, M >= 4096 ? lo.pieces : 1, put, put);
     plan->M = M;
     plan->N = h->N;
     plan->D = D;
     plan->total_nodes = h->total_nodes;
     plan->total_c = h->total_c;
-    plan->max_rows = max_rows;
-    plan->max_ck = max_ck;
-    plan->max_cslots = max_cslots;
+    plan->max_rows = lo.most.rows;
+    plan->max_ck = lo.most.ck;
+    plan->max_cslots = lo.most.cslots;
     plan->words = lo.words;
     plan->vcols = vcols;
     plan->n_gen = lo.n_gen;

@@ -331,6 +331,49 @@ static void check_long() {
     }
 }
 
+// Kernel, launch order and columns of a population around the fast kernels' bounds:
+// chains right and left of a stack depth of 16 (31 and 33 nodes), K 0 to 20.
+static void check_order() {
+    Pop p;
+    srand(7);
+    for (int m = 0; m < 6000; m++) {
+        p.tree();
+        const int depth = 14 + rand() % 5, K = rand() % 21;
+        for (int i = 1; i < depth; i++) p.op(OP_ADD, true);   // depth leaves stack up
+        for (int i = 0; i < depth; i++) {
+            const bool sine = rand() % 4 == 0;
+            if (sine) p.op(OP_SIN, false);
+            if (i < K) p.con();
+            else p.var(0);
+        }
+    }
+    CHECK(p.decode(1000, 1, 32) == CO_OK);
+    std::vector<int32_t> route(p.metas.size()), v_col(p.metas.size()), vrows(p.metas.size());
+    CHECK(decode_population(&p.h, p.nt.data(), p.nv.data(), p.ci.data(), p.metas.data(), nullptr,
+                            nullptr, nullptr, nullptr, nullptr, route.data()) == CO_OK);
+    int gen = 0;
+    for (int32_t r : route) gen += r;
+    CHECK(gen == p.plan.n_gen && gen > 500 && gen < 5500);
+    int rows = 0, ck = 0;
+    for (size_t q = 0; q < p.desc.size(); q++) {
+        const ExprDesc &d = p.desc[q];
+        CHECK(d.gen == route[d.y_row] && d.gen == (q < (size_t)gen));
+        if (q > 0 && d.gen == p.desc[q - 1].gen) CHECK(d.K <= p.desc[q - 1].K);
+        CHECK(d.K == p.metas[d.y_row].K && d.c_off == p.metas[d.y_row].c_offset);
+        v_col[d.y_row] = d.v_col;
+        vrows[d.y_row] = d.vrows;
+        rows = std::max(rows, d.rows);
+        if (d.n_c > 0) ck = std::max(ck, d.K);
+    }
+    CHECK(rows == p.plan.max_rows && ck == p.plan.max_ck);
+    int64_t cols = 0;
+    for (size_t m = 0; m < v_col.size(); m++) {
+        CHECK(v_col[m] == cols);
+        cols += vrows[m];
+    }
+    CHECK(cols == p.plan.vcols && cols > 0);
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
@@ -338,6 +381,7 @@ int main(int argc, char **argv) {
     else if (!strcmp(argv[1], "scalars")) check_scalars();
     else if (!strcmp(argv[1], "limit")) check_limit();
     else if (!strcmp(argv[1], "long")) check_long();
+    else if (!strcmp(argv[1], "order")) check_order();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;
