@@ -443,14 +443,14 @@ static int64_t program_words(int n_nodes, bool wide, bool staged);
 // Rows of a wavefront's LDS that an expression may use (variables, V values,
 // slots): what its plain program takes, n_vars and its slots, or this many.
 // V subtrees beyond stay in M, the last ones first. A row of the fp64 forward
-// kernels to K = 8 is 2 KB (four points per lane), and their registers let four
-// wavefronts on a SIMD at K = 1, three at 2 and 3, two beyond: as many as these
-// rows leave room for in a CU's 160 KB. Elsewhere a row is 512 bytes or 1 KB
-// (from N = 16,384 on two points per lane); more than eight rows cost reverse
-// AD wavefronts (twelve: C3 67.9 -> 70.4 ms).
-static int row_budget(int K, int N) {
-    return K > 3 || N >= 16384 ? 8 : K <= 1 ? 4 : 6;
-}
+// kernels to K = 8 is 2 KB (four points per lane), and their registers let three
+// wavefronts on a SIMD at K = 1 to 3, two beyond: as many as these rows leave room
+// for in a CU's 160 KB. Measured at K = 1, 4 rows -> 6 -> 8: 16,384 x 1,024 2.09 ->
+// 1.68 -> 2.12 ms, 60,000 x 300 3.37 -> 2.73 -> 3.11, reverse AD 5.90 -> 4.11 -> 3.46;
+// 6 -> 8 at K = 2 and 3: 16,384 x 1,024 2.48 -> 3.34 and 2.99 -> 4.06 ms. Elsewhere a
+// row is 512 bytes or 1 KB (from N = 16,384 on two points per lane); more than eight
+// rows cost reverse AD wavefronts (twelve: C3 67.9 -> 70.4 ms).
+static int row_budget(int K, int N) { return K > 3 || N >= 16384 ? 8 : 6; }
 // A wide expression with more variable rows than this is not staged: its plain
 // rows may fill the LDS, which then has no room for C's scalars.
 constexpr int kStageVarsMax = 128;
