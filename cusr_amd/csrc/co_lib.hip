@@ -83,9 +83,6 @@ struct HostBuf {
     const T &operator[](size_t i) const { return p[i]; }
 };
 
-// launchers per (precision, AD mode) come from fit_kernels.hip, each variant
-// in its own translation unit so the four compile in parallel
-
 // Device memory of a fit beyond its inputs and outputs: the loop state of
 // paused (tail) or split fits, then the split path's partition sums. Either
 // the handle's buffer, grown as needed, or a fixed region that is never grown
@@ -321,13 +318,13 @@ int upload_population(Ctx *ctx, const PopHeader *h, const int32_t *nt, const flo
 }
 
 // The launches of one fit, planned and issued range by range. The
-// descriptors of a range are in launch order (decode_population /
-// decode_range): a population decoded in several ranges has its bins planned
-// range by range.
+// descriptors of a range are in launch order (decode_range): a population
+// decoded in several ranges has its bins planned range by range.
 
 // The split path's step launch for a bin: the fast bins (K = 1..CO_FAST_MAX_K,
-// every expression of that K) take the instance whose solve is unrolled for
-// their K, the general bin and K = 0 the runtime-K one.
+// every expression of that K) take the instance whose solve knows their K, a group
+// of bins the padded one of its largest K, the general bin and K = 0 the runtime-K
+// one.
 template <int KS>
 static void launch_step_k(unsigned n, hipStream_t s, const FitArgs &fa, int mixed) {
     lm_step_kernel<KS><<<n, kLanes, 0, s>>>(fa, mixed);

@@ -7,9 +7,9 @@
 // scalar loads and every branch on it is a scalar branch, so the 64 lanes stay
 // converged and the fetch/decode cost is shared by 64*P points. Per point a
 // lane computes the value and the gradient row and folds r^2, J^T r and the
-// upper triangle of J^T J into registers; a butterfly over the 64 lanes then
-// gives every lane the same sums, and every lane solves the same damped
-// K x K system, so accept/reject and the lambda update stay on the device.
+// upper triangle of J^T J into registers (the matrix unit, at large K); the lanes'
+// sums are combined and stored in LDS, lane i factors row i of the damped K x K
+// system (damped_solve), and accept/reject and the lambda update stay on the device.
 //
 // Arithmetic follows one fixed order, which the CPU oracle reproduces:
 //   * lane l sums its points in ascending order from 0.0, fma(a, b, acc);
@@ -23,9 +23,12 @@
 // accepted point is reused. The reference recomputes both (batch_lm_ad.cu:363,
 // :400); the numbers are identical because the Jacobian depends only on c.
 //
-// LDS per wavefront: the batch's inputs x[v][p][lane], the spill slots
-// [s][p][lane], the constants and the pass sums; reverse AD adds its tape
-// [t][p][lane]. All indices are uniform, so accesses are bank-conflict free.
+// LDS per wavefront: the scalar area of the constant program C (program.h), the rows
+// [row][p][lane] of the batch (M's variables, V's values, then V's other variables
+// and slots over M's slots), in reverse AD the tape [t][p][lane], and the rows of the
+// matrix sums where a kernel has them. Per workgroup: the constants, the pass sums
+// and the partitions' sums. All indices are uniform, so accesses are bank-conflict
+// free.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -1014,7 +1017,8 @@ struct PassArgs {
     int Kr;             // constants
     uint64_t map;
     int vmode;          // V_*
-    void *V;            // [vrows][N] workspace columns, of the fit's type (null: none)
+    void *V;            // [vrows] workspace columns of N values, of the pass's type (the
+                        // fp64 audits of a mixed fit write theirs over its own; null: none)
     UniLds u;           // C's scalars (n_c > 0)
     const double *X;    // [D][N] column-major
     const double *y;    // this expression's targets [N]
@@ -1671,8 +1675,8 @@ struct FitArgs {
     double lambda0, xtol;
     int rows, tape;         // per-wave LDS rows of this launch ([row][P][64] each; the
                             // general kernel takes its expression's own)
-    void *V;                // [columns][N] workspace of the V values (null: run V in
-                            // every pass), of the fit's type
+    void *V;                // workspace of the V values, 8 N bytes a column (null: run V
+                            // in every pass)
     int uni_bytes;          // per-wave scalar area of this launch, its first bytes (likewise)
     int parts;              // point partitions per expression (1, 2 or 4)
     int pwaves;             // wavefronts of the workgroup (divides parts)
@@ -1906,10 +1910,9 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
     }
     double lf = loss, li = loss_init;
     if constexpr (sizeof(R) == 4) {
-        // fp64 losses at the delivered point and at the start; the fp64
-        // value pass reuses the same LDS bytes per row and lane (half the
-        // points of the fp32 passes). A lane sums its points in the same
-        // ascending order at any number of points per pass.
+        // fp64 losses at the delivered point and at the start, by value passes of
+        // audit_points per lane in the fit passes' LDS. A lane sums its points in
+        // the same ascending order at any number of points per pass.
         constexpr int AP = fit_audit_points<GEN, R, K, AD, LN>();
         constexpr int KA = GEN ? 0 : K;
         WaveLds<double, AP> w64;
@@ -1952,9 +1955,10 @@ __device__ __forceinline__ void fit_one(const FitArgs &fa, const ExprDesc &e, do
 #ifndef CUSR_W64_TABLE
 #define CUSR_W64_TABLE 1, 1, 1, 2, 2, 2, 2, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1
 #endif
-// fp64 reverse AD, the fit kernels (N below the split path's): no cap except
-// K = 9 (256 VGPRs with 23 spilled beats 300 at one wave per SIMD; from K = 10
-// the spills grow to 76 and more)
+// fp64 reverse AD, the fit kernels (N below the split path's): no cap except K = 9.
+// None of them spills, and K = 9 takes 212 VGPRs with the cap and without, only
+// scheduled otherwise (8,192 x 1,000 at K = 9: 18.75 ms with it, 19.15 without);
+// K = 11 is the one that a cap would bind (256 VGPRs and 2 AGPRs).
 #ifndef CUSR_WREV64_TABLE
 #define CUSR_WREV64_TABLE 1, 1, 1, 1, 1, 1, 1, 1, 1, 2, 1, 1, 1, 1, 1, 1, 1
 #endif
@@ -1973,10 +1977,12 @@ constexpr int waves_per_eu() {
                           : CUSR_WAVES_OTHER;
 }
 // fp64 reverse AD on the split path (the pass kernels: one wavefront per
-// workgroup, one point per lane): two waves per SIMD from K = 9 to 14, where
-// one wavefront per SIMD issued its SALU and VALU back to back (C3 127.4 ->
-// 116.7 ms); K = 15, 16 keep their 358 and 390 VGPRs (at 256 they spill
-// heavily: C3 126.6 ms with two waves for K = 9..16).
+// workgroup, one point per lane): two waves per SIMD from K = 9 to 14. Before the
+// matrix sums (K >= 12) and the lane-wise solve this kept them to 256 VGPRs (C3
+// 127.4 -> 116.7 ms); now they take 178-224 (K = 9 to 11) and 88-118 (12 to 16)
+// either way, and the caps only keep K = 12 to 14 off the accumulator registers.
+// With no cap: 8,192 x 2,048 at K = 9 32.57 -> 32.65 ms, K = 13 40.06 -> 39.91, K = 14
+// 40.78 -> 40.34, K 4-16 31.05 -> 30.82 (runs of one side differ by 0.1).
 #ifndef CUSR_WREV64_SPLIT_TABLE
 #define CUSR_WREV64_SPLIT_TABLE 1, 1, 1, 1, 1, 1, 1, 1, 1, 2, 2, 2, 2, 2, 2, 1, 1
 #endif
