@@ -1003,6 +1003,16 @@ struct RangeScratch {
     std::vector<uint32_t> key;
     std::vector<int32_t> vrows, v_col, launch;
     std::vector<uint64_t> a;
+    // those of at most kKept expressions (31 MB) stay with the thread
+    static constexpr size_t kKept = 1 << 18;
+    void trim() {
+        if (desc.size() <= kKept && lo.depth.size() <= kKept) return;
+        std::vector<ExprDesc>().swap(desc);
+        std::vector<uint32_t>().swap(key);
+        std::vector<uint64_t>().swap(a);
+        for (std::vector<int32_t> *v : {&vrows, &v_col, &launch, &lo.depth, &lo.gen, &lo.poff, &lo.rcs})
+            std::vector<int32_t>().swap(*v);
+    }
 };
 
 // Launch order by a key that sorts ascending: the general kernel's bin first, then
@@ -1027,6 +1037,10 @@ int decode_range(const PopHeader *h, const int32_t *nt, const float *nv, const i
     // working arrays kept per calling thread: for large populations fresh pages
     // cost a tenth of the decode
     static thread_local RangeScratch rs;
+    struct Trim {
+        RangeScratch &of;
+        ~Trim() { of.trim(); }
+    } trim{rs};
     Layout &lo = rs.lo;
     int rc = lay_out(h, nt, metas, M, true, lo);
     if (rc != CO_OK) return rc;

@@ -2,12 +2,14 @@
 // launches by against what the device reads and writes by them
 // (cusr_amd/csrc/program.h, launch_plan.h). Built and run by tests/test_layout.py with the
 // check's name; prints "layout ok".
+#include <malloc.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
 #include <chrono>
+#include <thread>
 #include <vector>
 
 #include "../cusr_amd/csrc/launch_plan.h"
@@ -374,6 +376,33 @@ static void check_order() {
     CHECK(cols == p.plan.vcols && cols > 0);
 }
 
+// What a thread keeps of its decodes is bounded: the working arrays of 400,000
+// expressions (48 MB) are given back.
+static void check_kept() {
+    Pop p;
+    for (int m = 0; m < 400000; m++) {
+        p.tree();
+        p.op(OP_ADD, true);
+        p.con();
+        p.var(0);
+    }
+    CHECK(p.decode(100, 1, 1) == CO_OK);   // the pool's threads, the outputs' arrays
+    const auto used = [] {
+        const struct mallinfo2 i = mallinfo2();
+        return (double)(i.uordblks + i.hblkhd);
+    };
+    double kept = 0.0;
+    std::thread([&] {
+        const double before = used();
+        Plan plan = {};
+        CHECK(decode_range(&p.h, p.nt.data(), p.nv.data(), p.ci.data(), p.metas.data(), 0,
+                           p.h.M_prob, 0, p.prog.data(), p.desc.data(), &plan) == CO_OK);
+        kept = used() - before;
+    }).join();
+    printf("kept %.1f MB\n", kept / 1e6);
+    CHECK(kept < 4e6);
+}
+
 int main(int argc, char **argv) {
     CHECK(argc == 2);
     if (!strcmp(argv[1], "eval")) check_eval();
@@ -382,6 +411,7 @@ int main(int argc, char **argv) {
     else if (!strcmp(argv[1], "limit")) check_limit();
     else if (!strcmp(argv[1], "long")) check_long();
     else if (!strcmp(argv[1], "order")) check_order();
+    else if (!strcmp(argv[1], "kept")) check_kept();
     else CHECK(!"check's name");
     puts("layout ok");
     return 0;

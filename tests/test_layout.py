@@ -24,7 +24,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("what", ["eval", "solve", "scalars", "limit", "long", "order"])
+@pytest.mark.parametrize("what", ["eval", "solve", "scalars", "limit", "long", "order", "kept"])
 def test_layout(exe, what):
     r = subprocess.run([str(exe), what], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and "layout ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
